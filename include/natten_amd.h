@@ -135,7 +135,9 @@ int na_mfma_selftest(int32_t dtype, float *out, void *stream);
  * parameters.  Launches nothing and reads no device memory.
  */
 enum na_kernel_path_t {
-  NA_PATH_GENERIC = 0, /* vector-ALU kernels: every dtype / head_dim / stride */
+  NA_PATH_GENERIC = 0, /* 32-bit arithmetic: vector-ALU kernels for every
+                          dtype / head_dim / stride, and their matrix-core
+                          form for most float32 or strided problems */
   NA_PATH_MFMA = 1,    /* 32-query matrix-core kernels */
   NA_PATH_LEAN = 2,    /* workgroup-staged 16x16x32 matrix-core kernels */
   NA_PATH_DENSE = 3    /* dense (FMHA) kernels: key or query tiles streamed

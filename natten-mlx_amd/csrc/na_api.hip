@@ -141,6 +141,15 @@ bool use_msplit(const na_params *p, const na::Prob &P) {
   return (p->flags & NA_FLAG_GENERIC) == 0 && na::msplit_eligible(P, p->dtype);
 }
 
+// The generic family's problems that run on matrix cores in 32-bit arithmetic.
+bool use_wave_fwd(const na_params *p, const na::Prob &P) {
+  return (p->flags & NA_FLAG_GENERIC) == 0 && na::wave_fwd_eligible(P, p->dtype);
+}
+
+bool use_wave_bwd(const na_params *p, const na::Prob &P) {
+  return (p->flags & NA_FLAG_GENERIC) == 0 && na::wave_eligible(P, p->dtype);
+}
+
 size_t align256(size_t n) { return (n + 255) & ~size_t(255); }
 
 size_t delta_bytes(const na::Prob &P) {
@@ -448,6 +457,8 @@ int na_fwd(const na_params *p, const void *q, const void *k, const void *v,
   else if (use_mfma(p, P))
     na::mfma_fwd(P, p->dtype, q, k, v, extra_k, extra_v, out, lse,
                  as_stream(stream));
+  else if (use_wave_fwd(p, P))
+    na::wave_fwd(P, p->dtype, q, k, v, out, lse, as_stream(stream));
   else
     na::valu_fwd(P, p->dtype, q, k, v, extra_k, extra_v, out, lse,
                  as_stream(stream));
@@ -502,6 +513,8 @@ int na_bwd(const na_params *p, const void *q, const void *k, const void *v,
       na::valu_delta(P, p->dtype, out, dout, dlse, delta, st);
     na::mfma_bwd(P, p->dtype, q, k, v, extra_k, extra_v, out, lse, dout, dlse,
                  delta, dq, dk, dv, st);
+  } else if (use_wave_bwd(p, P)) {
+    na::wave_bwd(P, p->dtype, q, k, v, out, lse, dout, dlse, dq, dk, dv, st);
   } else {
     na::valu_bwd(P, p->dtype, q, k, v, extra_k, extra_v, out, lse, dout, dlse,
                  dq, dk, dv, delta, st);

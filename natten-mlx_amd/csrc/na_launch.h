@@ -165,6 +165,19 @@ void merge_bwd(int dtype, int n, int64_t rows, int D, const void *const *outs,
                const float *const *lses, const void *dout, const float *dlse,
                void *const *d_outs, float *const *d_lses, hipStream_t st);
 
+// Fused forward / backward on matrix cores in 32-bit arithmetic
+// (na_wave.hip): float32, and strided bf16 / fp16 problems, without
+// per-sample extents, additional tokens or dense mode.  The backward is one
+// launch and reads no workspace.
+bool wave_eligible(const Prob &P, int dtype);      // backward
+bool wave_fwd_eligible(const Prob &P, int dtype);  // forward: a subset
+void wave_fwd(const Prob &P, int dtype, const void *q, const void *k,
+              const void *v, void *out, float *lse, hipStream_t st);
+void wave_bwd(const Prob &P, int dtype, const void *q, const void *k,
+              const void *v, const void *out, const float *lse,
+              const void *dout, const float *dlse, void *dq, void *dk,
+              void *dv, hipStream_t st);
+
 // Generic pieces reused around the MFMA backward.
 void valu_delta(const Prob &P, int dtype, const void *out, const void *dout,
                 const float *dlse, float *delta, hipStream_t st);

@@ -1,0 +1,975 @@
+// na_wave.hip — fused neighborhood attention on matrix cores in 32-bit
+// arithmetic: float32 tensors, and bf16 / fp16 tensors with strided queries.
+//
+// Problem class (wave_eligible): float32 with head_dim 16/32/64/128, or
+// bf16/fp16 with head_dim 32/64/128 where some axis is strided; on every axis
+// stride 1 or dilation 1, and a causal axis or an odd K with d*K <= L; no
+// per-sample extents, additional tokens or dense mode.  Everything else of
+// those types stays with the vector-ALU kernels (na_valu.hip), whose results
+// these match to rounding: probabilities, score gradients and sums stay
+// float32 for every storage type.
+//
+// One wave owns 16 queries of one dilation phase (a T0 x T1 x T2 box) and
+// needs no other wave: no barrier, 16 rows of its own in LDS.  The keys its
+// queries' windows cover form a box [lo, lo + E) per axis; its points are
+// numbered row-major and taken 16 at a time, so a chunk is always full
+// (K = 7, tile 4 x 4: 100 points = 7 chunks; one chunk per box row would be
+// 10).  Lane l = 16 gq + n loads row n of the chunk (16 bytes of every 64):
+// the A operand of S^T = K Q^T as it lies in memory.  V goes through the
+// wave's LDS rows, as float32, to be read transposed for O^T += V^T P^T on
+// v_mfma_f32_16x16x4_f32: the lane's scores of step r are that step's B
+// operand as they come out of the score MFMA.  The rows' box coordinates,
+// packed into one word with a guard bit per axis, go through LDS too; one
+// subtraction each way tests a key against all axes of a query's window.
+// The next chunk's loads are issued once its operands are free, so they fly
+// during the softmax and the second product.
+//
+// What bounds it: the f32 matrix cores run 64 FLOP per cycle and SIMD (157
+// TFLOP/s on the chip), and a 16-query tile multiplies the whole box, about
+// twice its windows' keys; then the chain load -> scores -> softmax -> product
+// of the few waves a small problem has.  Against the vector-ALU kernels, which
+// read every key row once per query from L2: float32 [2, 61, 45, 8, 32] K = 7
+// forward 52 -> 17 us, backward 279 -> 41 us; bf16 [4, 57, 75, 4, 64] K = 7
+// stride 2 forward 40 -> 18 us, backward 188 -> 34 us; float32 [4, 128, 128,
+// 8, 64] K = 3, the least work per key, 249 -> 137 and 985 -> 425 us.
+//
+// A value that is not finite must reach only the queries whose windows hold
+// it, but 0 * inf in a product over the box is NaN.  So a wave whose result
+// holds a NaN computes its rows again key by key (the `again` blocks).
+#include <algorithm>
+#include <cmath>
+
+#include "na_common.h"
+#include "na_launch.h"
+
+namespace na {
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// A lane's 16-byte fragment of each 64-byte piece of a row, the 16x16 score
+// product over one piece, and the fragment as float32 (EPF elements from
+// element EPF * gq of the piece).
+template <typename T>
+struct Wv;
+template <>
+struct Wv<float> {
+  typedef f32x4 frag;
+  static constexpr int EPF = 4;
+  static __device__ __forceinline__ f32x4 mma(frag a, frag b, f32x4 c) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
+    return c;
+  }
+};
+template <>
+struct Wv<bf16_t> {
+  typedef __bf16 frag __attribute__((ext_vector_type(8)));
+  static constexpr int EPF = 8;
+  static __device__ __forceinline__ f32x4 mma(frag a, frag b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
+};
+template <>
+struct Wv<f16_t> {
+  typedef _Float16 frag __attribute__((ext_vector_type(8)));
+  static constexpr int EPF = 8;
+  static __device__ __forceinline__ f32x4 mma(frag a, frag b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
+};
+
+// Tiling of the query grid (forward, dQ) or the key grid (dK / dV).
+struct WvGrid {
+  int32_t T[3], lgT[3], nt[3];  // tile extents (powers of two), tiles per phase
+  FastDiv fG[3], fnt[3];        // d * nt, nt
+  FastDiv fGrid;                // tiles per (sample, head)
+  int32_t n_tiles, n_wg;        // waves, workgroups launched (a multiple of 8)
+};
+
+struct WvAx {
+  int32_t K, nh, d, s, causal, O;
+  int32_t Lq, Lrem;    // phase r of the keys holds Lq + (r < Lrem) points
+  int32_t tok, otok;   // token strides of one position: input and output grid
+};
+
+struct WvProb {
+  WvAx ax[3];
+  int32_t B, H, Hkv, rep;
+  int64_t Ltot, Otot;  // tokens per sample: input and output grid
+  FastDiv fH, fHkv, fRep;
+  float scale, sl2;    // sl2 = scale * log2(e)
+  WvGrid gq, gk;       // query tiles, key tiles
+};
+
+// Box coordinates packed into one word, a guard bit above each field.
+template <int R>
+struct Pk {
+  static constexpr int W = R == 1 ? 32 : R == 2 ? 16 : 10;  // field width
+  static constexpr uint32_t kMax = (1u << (W - 1)) - 1;     // largest coordinate
+  static constexpr uint32_t kGuard =
+      R == 1 ? 0x80000000u : R == 2 ? 0x80008000u : (1u << 9) | (1u << 19) | (1u << 29);
+  static constexpr uint32_t kAll =
+      R == 1 ? kMax : R == 2 ? kMax * 0x10001u : kMax * 0x100401u;
+  static __device__ __forceinline__ constexpr int shift(int a) { return (2 - a) * (R == 1 ? 0 : W); }
+};
+
+struct WvTile {
+  int b, h;
+  int r[3], i0[3], nv[3], Lr[3], Qr[3];
+};
+
+__device__ __forceinline__ int wv_start(const WvAx &x, int ip, int Lr) {
+  return x.causal ? max(ip - x.K + 1, 0) : min(max(ip - x.nh, 0), Lr - x.K);
+}
+__device__ __forceinline__ int wv_end(const WvAx &x, int ip, int Lr) {
+  return x.causal ? ip + 1 : min(max(ip - x.nh, 0), Lr - x.K) + x.K;
+}
+// Query indices [first, last) whose windows hold key j: the positions are
+// [j <= K-1 ? 0 : j - K/2, j >= Lr-K ? Lr : j + K/2 + 1) (causal [j, j + K)),
+// of which every s-th carries a query.
+__device__ __forceinline__ int wv_istart(const WvAx &x, int j) {
+  const int p = x.causal ? j : (j <= x.K - 1 ? 0 : j - x.nh);
+  return x.s == 1 ? p : (p + x.s - 1) / x.s;
+}
+__device__ __forceinline__ int wv_iend(const WvAx &x, int j, int Lr, int Qr) {
+  const int p = x.causal ? min(j + x.K, Lr) : (j >= Lr - x.K ? Lr : j + x.nh + 1);
+  return x.s == 1 ? p : min((p + x.s - 1) / x.s, Qr);
+}
+
+template <int R>
+__device__ __forceinline__ bool wv_decode(const WvProb &P, const WvGrid &G, const FastDiv &fHn,
+                                          uint32_t tile, bool keys, WvTile &t) {
+  const uint32_t rest = fdiv(tile, G.fGrid);
+  uint32_t sp = tile - rest * G.fGrid.d;
+  const uint32_t bq = fdiv(rest, fHn);
+  t.h = (int)(rest - bq * fHn.d);
+  t.b = (int)bq;
+  bool any = t.b < P.B;
+#pragma unroll
+  for (int a = 2; a >= 3 - R; --a) {
+    const WvAx &x = P.ax[a];
+    uint32_t g = sp;
+    if (a > 3 - R) {
+      const uint32_t qd = fdiv(sp, G.fG[a]);
+      g = sp - qd * G.fG[a].d;
+      sp = qd;
+    }
+    const int rr = (int)fdiv(g, G.fnt[a]);
+    t.r[a] = rr;
+    t.i0[a] = ((int)g - rr * G.nt[a]) << G.lgT[a];
+    t.Lr[a] = x.Lq + (rr < x.Lrem ? 1 : 0);
+    t.Qr[a] = x.s == 1 ? t.Lr[a] : x.O;
+    t.nv[a] = min((keys ? t.Lr[a] : t.Qr[a]) - t.i0[a], G.T[a]);
+    any = any && t.nv[a] > 0;
+  }
+  return any;
+}
+
+// Index of the lane's row (position n of the tile, the last one past its end)
+// on axis a.
+__device__ __forceinline__ int wv_row(const WvGrid &G, const WvTile &t, int a, int n, bool &valid) {
+  int sh = 0;
+  for (int c = 2; c > a; --c) sh += G.lgT[c];
+  const int u = (n >> sh) & (G.T[a] - 1);
+  valid = valid && u < t.nv[a];
+  return t.i0[a] + min(u, t.nv[a] - 1);
+}
+
+// A box of rows numbered row-major: extents, byte strides of its points in
+// one tensor (and a second one), and the decoding of a point's number.
+template <int R, bool TWO>
+struct WvBox {
+  int lo[3], E[3], npts;
+  uint32_t SK[3], SO[3];
+  float r2, r1;
+  __device__ __forceinline__ void finish() {
+    npts = 1;
+#pragma unroll
+    for (int a = 3 - R; a < 3; ++a) npts *= max(E[a], 0);
+    r2 = __builtin_amdgcn_rcpf((float)E[2]);
+    r1 = R == 3 ? __builtin_amdgcn_rcpf((float)E[1]) : 0.f;
+  }
+  // Packed coordinates and byte offsets of point x.  The quotients come
+  // from a product with the reciprocal: (x + 1/2) / E is at least 1/(2 E)
+  // from an integer and the product is off by less than x 2^-22 / E, so they
+  // are exact for x < 2^20.
+  __device__ __forceinline__ uint32_t point(int x, uint32_t &off, uint32_t &off2) const {
+    const int xc = min(x, npts - 1);
+    int e0 = 0, e1 = 0, e2 = xc;
+    if (R >= 2) {
+      e1 = (int)(((float)xc + 0.5f) * r2);
+      e2 = xc - e1 * E[2];
+    }
+    if (R == 3) {
+      e0 = (int)(((float)e1 + 0.5f) * r1);
+      e1 -= e0 * E[1];
+    }
+    off = (uint32_t)e2 * SK[2];
+    if (R >= 2) off += (uint32_t)e1 * SK[1];
+    if (R == 3) off += (uint32_t)e0 * SK[0];
+    off2 = off;
+    if (TWO) {
+      off2 = (uint32_t)e2 * SO[2];
+      if (R >= 2) off2 += (uint32_t)e1 * SO[1];
+      if (R == 3) off2 += (uint32_t)e0 * SO[0];
+    }
+    uint32_t c = (uint32_t)e2;
+    if (R >= 2) c |= (uint32_t)e1 << Pk<R>::shift(1);
+    if (R == 3) c |= (uint32_t)e0 << Pk<R>::shift(0);
+    return x < npts ? c : Pk<R>::kAll;  // past the box: in no window
+  }
+};
+
+// A lane's window in box coordinates, packed: wl its first point, wh its last.
+template <int R>
+struct WvWin {
+  uint32_t wl = 0, wh = 0;
+  bool none = false;
+  __device__ __forceinline__ void axis(int a, int first, int last) {
+    none = none || last < first;
+    wl |= (uint32_t)first << Pk<R>::shift(a);
+    wh |= (uint32_t)last << Pk<R>::shift(a);
+  }
+  __device__ __forceinline__ void finish() {
+    if (none) {
+      wl = Pk<R>::kAll;
+      wh = 0;
+    }
+  }
+  // every field of (c - wl) and (wh - c) is non-negative
+  __device__ __forceinline__ bool holds(uint32_t c) const {
+    constexpr uint32_t g = Pk<R>::kGuard;
+    return (((c | g) - wl) & ((wh | g) - c) & g) == g;
+  }
+};
+
+template <typename T, int NF>
+__device__ __forceinline__ void ld_row(const char *base, uint32_t off, typename Wv<T>::frag (&f)[NF]) {
+#pragma unroll
+  for (int i = 0; i < NF; ++i)
+    f[i] = *reinterpret_cast<const typename Wv<T>::frag *>(base + (size_t)(off + 64u * i));
+}
+
+// Four consecutive elements as float32, and their store.
+template <typename T>
+__device__ __forceinline__ f32x4 ld4(const char *p) {
+  f32x4 v;
+  if constexpr (sizeof(T) == 4) {
+    v = *reinterpret_cast<const f32x4 *>(p);
+  } else {
+    float x[4];
+    VecIO<T, 4>::load(reinterpret_cast<const T *>(p), x);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = x[r];
+  }
+  return v;
+}
+template <typename T>
+__device__ __forceinline__ void st4(char *p, f32x4 v) {
+  const float x[4] = {v[0], v[1], v[2], v[3]};
+  VecIO<T, 4>::store(reinterpret_cast<T *>(p), x);
+}
+
+template <typename T>
+__device__ __forceinline__ float wv_dot(typename Wv<T>::frag a, typename Wv<T>::frag b, float c) {
+#pragma unroll
+  for (int e = 0; e < Wv<T>::EPF; ++e) c = fmaf((float)a[e], (float)b[e], c);
+  return c;
+}
+
+// The lane's fragments of its row n into LDS row `row` as float32.
+template <typename T, int NF>
+__device__ __forceinline__ void wv_lds(float *row, int gq, const typename Wv<T>::frag (&f)[NF]) {
+  constexpr int N = Wv<T>::EPF;
+#pragma unroll
+  for (int i = 0; i < NF; ++i)
+#pragma unroll
+    for (int e = 0; e < N; e += 4) {
+      const f32x4 v = {(float)f[i][e], (float)f[i][e + 1], (float)f[i][e + 2], (float)f[i][e + 3]};
+      *reinterpret_cast<f32x4 *>(row + 4 * N * i + N * gq + e) = v;
+    }
+}
+
+// The 16x16 products of rows a[0..NF) with rows b: up to four sums of their
+// own, added pairwise (a single chain over head_dim lost 1.2e-7 of a forward's
+// output where the lane-group sums of na_valu.hip lose 1.0e-7), which also
+// keeps several products in flight.
+template <typename T, int NF>
+__device__ __forceinline__ f32x4 wv_scores(const typename Wv<T>::frag (&a)[NF],
+                                           const typename Wv<T>::frag (&b)[NF]) {
+  constexpr int N = NF < 4 ? NF : 4;
+  f32x4 s[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < NF; ++i) s[i % N] = Wv<T>::mma(a[i], b[i], s[i % N]);
+  if constexpr (N == 4) return (s[0] + s[1]) + (s[2] + s[3]);
+  if constexpr (N == 2) return s[0] + s[1];
+  return s[0];
+}
+
+// acc^T += X^T W: X the 16 LDS rows, the lane's w[r] the weight of row
+// 4 gq + r in its column.
+template <int NDB, int RS>
+__device__ __forceinline__ void wv_acc(const float *xt, const float (&w)[4], f32x4 (&acc)[NDB]) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+      acc[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(xt[r * RS + 16 * db], w[r], acc[db], 0, 0, 0);
+}
+
+__device__ __forceinline__ float wv_quad_max(float x) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float wv_quad_sum(float x) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+// This wave's LDS operations so far are complete.
+__device__ __forceinline__ void wv_lds_sync() {
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+  __builtin_amdgcn_wave_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <int NDB>
+__device__ __forceinline__ bool wv_nan(const f32x4 (&a)[NDB], float t) {
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) t += a[db][r];
+  return __builtin_amdgcn_ballot_w64(!(t == t)) != 0;  // inf - inf too: no harm
+}
+
+// Workgroups reach the 8 XCDs in turn; each XCD gets a contiguous run of them.
+__device__ __forceinline__ int wv_wg(int bid, int n_wg) { return (bid & 7) * (n_wg >> 3) + (bid >> 3); }
+
+// Waves per workgroup (they are independent; at head_dim 128 the backward's
+// LDS rows of four would pass 64 KB).
+template <int D>
+constexpr int wv_waves() {
+  return D == 128 ? 2 : 4;
+}
+// LDS row stride in floats: 4 mod 64 banks apart (36, 68, ...; 20 for 16), so
+// the 16 rows' 16-byte writes and the transposed reads of 4 row groups x 16
+// columns are free of conflicts.
+template <int D>
+constexpr int wv_rs() {
+  return D + 4;
+}
+
+template <typename T, int D, int R>
+__global__ void __launch_bounds__(64 * wv_waves<D>())
+    k_wvfwd(WvProb P, const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v,
+            T *__restrict__ out, float *__restrict__ lse) {
+  typedef typename Wv<T>::frag frag;
+  constexpr int ES = sizeof(T), NF = D * ES / 64, NDB = D / 16, RS = wv_rs<D>(), NW = wv_waves<D>();
+  __shared__ __align__(16) float smem[NW * (16 * RS + 16)];
+
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, n = lane & 15, gq = lane >> 4;
+  const uint32_t tile = (uint32_t)(wv_wg(blockIdx.x, P.gq.n_wg) * NW + w);
+  WvTile t;
+  if (!wv_decode<R>(P, P.gq, P.fH, tile, false, t)) return;
+  const int hk = (int)fdiv((uint32_t)t.h, P.fRep);
+
+  // the tile's key box, the lane's query and its window
+  WvBox<R, false> box;
+  WvWin<R> win;
+  bool qv = true;
+  int64_t ktok = 0;
+  int qtok = 0, otok = 0;
+#pragma unroll
+  for (int a = 3 - R; a < 3; ++a) {
+    const WvAx &x = P.ax[a];
+    box.lo[a] = wv_start(x, t.i0[a] * x.s, t.Lr[a]);
+    box.E[a] = wv_end(x, (t.i0[a] + t.nv[a] - 1) * x.s, t.Lr[a]) - box.lo[a];
+    box.SK[a] = (uint32_t)(x.d * x.tok) * (uint32_t)(P.Hkv * D * ES);
+    ktok += (int64_t)(t.r[a] + x.d * box.lo[a]) * x.tok;
+    const int i = wv_row(P.gq, t, a, n, qv);
+    qtok += (t.r[a] + x.d * x.s * i) * x.tok;
+    otok += (t.r[a] + x.d * i) * x.otok;
+    win.axis(a, wv_start(x, i * x.s, t.Lr[a]) - box.lo[a],
+             wv_end(x, i * x.s, t.Lr[a]) - 1 - box.lo[a]);
+  }
+  box.finish();
+  win.finish();
+  const int64_t kofs = ((t.b * P.Ltot + ktok) * P.Hkv + hk) * (D * ES);
+  const char *kb = reinterpret_cast<const char *>(k) + kofs;
+  const char *vb = reinterpret_cast<const char *>(v) + kofs;
+  const char *qb = reinterpret_cast<const char *>(q) + (t.b * P.Ltot * P.H + t.h) * (D * ES);
+
+  frag qf[NF], kf[NF], vf[NF];
+  ld_row<T>(qb, (uint32_t)qtok * (uint32_t)(P.H * D * ES) + 16u * gq, qf);
+  uint32_t cd, ko, unused;
+  auto load = [&](int c) {
+    cd = box.point(16 * c + n, ko, unused);
+    ld_row<T>(kb, ko + 16u * gq, kf);
+    ld_row<T>(vb, ko + 16u * gq, vf);
+  };
+  load(0);
+
+  float *vrow = smem + w * (16 * RS + 16);
+  uint32_t *crow = reinterpret_cast<uint32_t *>(vrow + 16 * RS);
+  const float *vt = vrow + 4 * gq * RS + n;
+  f32x4 o[NDB];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  const int nch = (box.npts + 15) >> 4;
+  for (int c = 0; c < nch; ++c) {
+    f32x4 s = wv_scores<T>(kf, qf);
+    wv_lds<T>(vrow + n * RS, gq, vf);
+    if (gq == 0) crow[n] = cd;
+    load(c + 1);  // past the last chunk: its last point again
+    wv_lds_sync();
+    const uint4 cc = *reinterpret_cast<const uint4 *>(crow + 4 * gq);
+    const uint32_t c4[4] = {cc.x, cc.y, cc.z, cc.w};
+    float mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      s[r] = win.holds(c4[r]) ? s[r] : -INFINITY;
+      mx = fmaxf(mx, s[r]);
+    }
+    mx = wv_quad_max(mx) * P.sl2;
+    // the reference point may trail the running maximum by up to 8 (a
+    // factor 2^8 in P, exact after the division by l)
+    if (__builtin_amdgcn_ballot_w64(mx > m + 8.f) != 0) {
+      const float mn = fmaxf(m, mx);
+      const float alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+      l *= alpha;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) o[db] *= alpha;
+      m = mn;
+    }
+    const float mu = m == -INFINITY ? 0.f : m;
+    float p[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      p[r] = __builtin_amdgcn_exp2f(fmaf(s[r], P.sl2, -mu));
+      l += p[r];
+    }
+    wv_acc<NDB, RS>(vt, p, o);
+  }
+  l = wv_quad_sum(l);
+  if (wv_nan(o, l)) {  // again, key by key
+    m = -INFINITY;
+    l = 0.f;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int x = 0; x < box.npts; ++x) {
+      cd = box.point(x, ko, unused);
+      ld_row<T>(kb, ko + 16u * gq, kf);
+      float s = 0.f;
+#pragma unroll
+      for (int i = 0; i < NF; ++i) s = wv_dot<T>(qf[i], kf[i], s);
+      s = wv_quad_sum(s) * P.sl2;
+      if (win.holds(cd)) {
+        const float mn = fmaxf(m, s);
+        const float mu = mn == -INFINITY ? 0.f : mn;
+        const float alpha = exp2f(m - mu), pr = exp2f(s - mu);
+        l = fmaf(l, alpha, pr);
+        m = mn;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+          o[db] = o[db] * alpha + pr * ld4<T>(vb + ko + (16 * db + 4 * gq) * ES);
+      }
+    }
+  }
+  if (!qv) return;
+  const float inv = 1.f / l;
+  const int64_t orow = (t.b * P.Otot + otok) * P.H + t.h;
+  char *ob = reinterpret_cast<char *>(out) + orow * (D * ES);
+#pragma unroll
+  for (int db = 0; db < NDB; ++db) st4<T>(ob + (16 * db + 4 * gq) * ES, o[db] * inv);
+  if (lse != nullptr && gq == 0) lse[orow] = (m + __log2f(l)) * kLn2;
+}
+
+// Backward.  Workgroups [0, gk.n_wg) own key tiles (dK, dV; the longer role,
+// dispatched first), the rest query tiles (dQ); delta = rowsum(dO * O) - dlse
+// is formed from the rows each role reads anyway plus O.
+template <typename T, int D, int R, bool STR>
+__global__ void __launch_bounds__(64 * wv_waves<D>())
+    k_wvbwd(WvProb P, const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v,
+            const T *__restrict__ out, const float *__restrict__ lse, const T *__restrict__ dout,
+            const float *__restrict__ dlse, T *__restrict__ dq, T *__restrict__ dk,
+            T *__restrict__ dv) {
+  typedef typename Wv<T>::frag frag;
+  constexpr int ES = sizeof(T), NF = D * ES / 64, NDB = D / 16, RS = wv_rs<D>(), NW = wv_waves<D>();
+  constexpr int LW = 2 * 16 * RS + 48;  // floats per wave
+  __shared__ __align__(16) float smem[NW * LW];
+
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, n = lane & 15, gq = lane >> 4;
+  float *xrow = smem + w * LW;
+  uint32_t *crow = reinterpret_cast<uint32_t *>(xrow + 2 * 16 * RS);
+  const float *xt = xrow + 4 * gq * RS + n;
+  const char *qc = reinterpret_cast<const char *>(q), *kc = reinterpret_cast<const char *>(k);
+  const char *vc = reinterpret_cast<const char *>(v), *oc = reinterpret_cast<const char *>(out);
+  const char *gc = reinterpret_cast<const char *>(dout);
+  const uint32_t HB = (uint32_t)(P.H * D * ES);  // bytes per token of q, out, dout
+  WvTile t;
+  WvWin<R> win;
+
+  if ((int)blockIdx.x >= P.gk.n_wg) {
+    // =============================== dQ ===============================
+    const uint32_t tile =
+        (uint32_t)(wv_wg((int)blockIdx.x - P.gk.n_wg, P.gq.n_wg) * NW + w);
+    if (!wv_decode<R>(P, P.gq, P.fH, tile, false, t)) return;
+    const int hk = (int)fdiv((uint32_t)t.h, P.fRep);
+    WvBox<R, false> box;
+    bool qv = true;
+    int64_t ktok = 0;
+    int qtok = 0, otok = 0;
+#pragma unroll
+    for (int a = 3 - R; a < 3; ++a) {
+      const WvAx &x = P.ax[a];
+      box.lo[a] = wv_start(x, t.i0[a] * x.s, t.Lr[a]);
+      box.E[a] = wv_end(x, (t.i0[a] + t.nv[a] - 1) * x.s, t.Lr[a]) - box.lo[a];
+      box.SK[a] = (uint32_t)(x.d * x.tok) * (uint32_t)(P.Hkv * D * ES);
+      ktok += (int64_t)(t.r[a] + x.d * box.lo[a]) * x.tok;
+      const int i = wv_row(P.gq, t, a, n, qv);
+      qtok += (t.r[a] + x.d * x.s * i) * x.tok;
+      otok += (t.r[a] + x.d * i) * x.otok;
+      win.axis(a, wv_start(x, i * x.s, t.Lr[a]) - box.lo[a],
+               wv_end(x, i * x.s, t.Lr[a]) - 1 - box.lo[a]);
+    }
+    box.finish();
+    win.finish();
+    const int64_t kofs = ((t.b * P.Ltot + ktok) * P.Hkv + hk) * (D * ES);
+    const char *kb = kc + kofs, *vb = vc + kofs;
+    const int64_t qofs = (t.b * P.Ltot * P.H + t.h) * (D * ES);
+    const int64_t orow0 = t.b * P.Otot * P.H + t.h;
+    const uint32_t qo = (uint32_t)qtok * HB, oo = (uint32_t)otok * HB;
+
+    frag qf[NF], df[NF], kf[NF], vf[NF];
+    ld_row<T>(qc + qofs, qo + 16u * gq, qf);
+    ld_row<T>(gc + orow0 * (D * ES), oo + 16u * gq, df);
+    float delta = 0.f;
+    {
+      frag of[NF];
+      ld_row<T>(oc + orow0 * (D * ES), oo + 16u * gq, of);
+#pragma unroll
+      for (int i = 0; i < NF; ++i) delta = wv_dot<T>(df[i], of[i], delta);
+    }
+    uint32_t cd, ko, unused;
+    auto load = [&](int c) {
+      cd = box.point(16 * c + n, ko, unused);
+      ld_row<T>(kb, ko + 16u * gq, kf);
+      ld_row<T>(vb, ko + 16u * gq, vf);
+    };
+    load(0);
+    const int64_t orow = orow0 + (int64_t)otok * P.H;
+    const float lse2 = lse[orow] * kLog2e;
+    delta = wv_quad_sum(delta) - (dlse != nullptr ? dlse[orow] : 0.f);
+    f32x4 acc[NDB];
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) acc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int nch = (box.npts + 15) >> 4;
+    for (int c = 0; c < nch; ++c) {
+      const f32x4 s = wv_scores<T>(kf, qf), dp = wv_scores<T>(vf, df);
+      wv_lds<T>(xrow + n * RS, gq, kf);
+      if (gq == 0) crow[n] = cd;
+      load(c + 1);
+      wv_lds_sync();
+      const uint4 cc = *reinterpret_cast<const uint4 *>(crow + 4 * gq);
+      const uint32_t c4[4] = {cc.x, cc.y, cc.z, cc.w};
+      float ds[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float p = __builtin_amdgcn_exp2f(fmaf(s[r], P.sl2, -lse2));
+        ds[r] = win.holds(c4[r]) ? p * (dp[r] - delta) : 0.f;
+      }
+      wv_acc<NDB, RS>(xt, ds, acc);
+    }
+    if (wv_nan(acc, 0.f)) {  // again, key by key
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) acc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int x = 0; x < box.npts; ++x) {
+        cd = box.point(x, ko, unused);
+        ld_row<T>(kb, ko + 16u * gq, kf);
+        ld_row<T>(vb, ko + 16u * gq, vf);
+        float s = 0.f, dp = 0.f;
+#pragma unroll
+        for (int i = 0; i < NF; ++i) {
+          s = wv_dot<T>(qf[i], kf[i], s);
+          dp = wv_dot<T>(df[i], vf[i], dp);
+        }
+        s = wv_quad_sum(s);
+        dp = wv_quad_sum(dp);
+        if (win.holds(cd)) {
+          const float ds = exp2f(fmaf(s, P.sl2, -lse2)) * (dp - delta);
+#pragma unroll
+          for (int db = 0; db < NDB; ++db)
+            acc[db] += ds * ld4<T>(kb + ko + (16 * db + 4 * gq) * ES);
+        }
+      }
+    }
+    if (!qv) return;
+    char *db_ = reinterpret_cast<char *>(dq) + qofs + qo;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) st4<T>(db_ + (16 * db + 4 * gq) * ES, acc[db] * P.scale);
+    return;
+  }
+
+  // ============================== dK / dV ==============================
+  const uint32_t tile = (uint32_t)(wv_wg(blockIdx.x, P.gk.n_wg) * NW + w);
+  if (!wv_decode<R>(P, P.gk, P.fHkv, tile, true, t)) return;
+  // the box of queries whose windows hold the tile's keys
+  WvBox<R, STR> box;
+  bool kv = true, on = true;  // on: the key's position carries a query
+  int64_t qtok = 0, otok = 0;
+  int ktok = 0;
+#pragma unroll
+  for (int a = 3 - R; a < 3; ++a) {
+    const WvAx &x = P.ax[a];
+    box.lo[a] = wv_istart(x, t.i0[a]);
+    box.E[a] = wv_iend(x, t.i0[a] + t.nv[a] - 1, t.Lr[a], t.Qr[a]) - box.lo[a];
+    box.SK[a] = (uint32_t)(x.d * x.s * x.tok) * HB;
+    box.SO[a] = (uint32_t)(x.d * x.otok) * HB;
+    qtok += (int64_t)(t.r[a] + x.d * x.s * box.lo[a]) * x.tok;
+    otok += (int64_t)(t.r[a] + x.d * box.lo[a]) * x.otok;
+    const int j = wv_row(P.gk, t, a, n, kv);
+    ktok += (t.r[a] + x.d * j) * x.tok;
+    on = on && (!STR || j % x.s == 0);
+    win.axis(a, wv_istart(x, j) - box.lo[a], wv_iend(x, j, t.Lr[a], t.Qr[a]) - 1 - box.lo[a]);
+  }
+  box.finish();
+  win.finish();
+  const int64_t kofs = (t.b * P.Ltot * P.Hkv + t.h) * (D * ES);
+  const uint32_t ko = (uint32_t)ktok * (uint32_t)(P.Hkv * D * ES);
+  frag kf[NF], vf[NF];
+  ld_row<T>(kc + kofs, ko + 16u * gq, kf);
+  ld_row<T>(vc + kofs, ko + 16u * gq, vf);
+  f32x4 adk[NDB], adv[NDB];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db) {
+    adk[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    adv[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  float *const grow = xrow + 16 * RS;                              // dO rows
+  float *const lrow = reinterpret_cast<float *>(crow) + 16;        // lse * log2(e)
+  float *const drow = lrow + 16;                                   // delta
+  const float *const gt = xt + 16 * RS;
+  const int nch = (box.npts + 15) >> 4;
+  // (row of the output grid, head h) at byte offset oo of that head's rows
+  const uint32_t rowsh = (uint32_t)(D * ES);
+  for (int hr = 0; hr < P.rep && nch > 0; ++hr) {
+    const int h = t.h * P.rep + hr;
+    const char *qb = qc + ((t.b * P.Ltot + qtok) * P.H + h) * (D * ES);
+    const int64_t orow0 = (t.b * P.Otot + otok) * P.H + h;
+    const char *gb = gc + orow0 * (D * ES), *ob = oc + orow0 * (D * ES);
+    const float *lb = lse + orow0, *dlb = dlse != nullptr ? dlse + orow0 : nullptr;
+    frag qf[NF], gf[NF], of[NF];
+    uint32_t cd, qo, oo;
+    float ls, dl;
+    auto load = [&](int c) {
+      cd = box.point(16 * c + n, qo, oo);
+      ld_row<T>(qb, qo + 16u * gq, qf);
+      ld_row<T>(gb, oo + 16u * gq, gf);
+      ld_row<T>(ob, oo + 16u * gq, of);
+      ls = lb[oo / rowsh];
+      dl = dlb != nullptr ? dlb[oo / rowsh] : 0.f;
+    };
+    load(0);
+    for (int c = 0; c < nch; ++c) {
+      const f32x4 s = wv_scores<T>(qf, kf), dp = wv_scores<T>(gf, vf);
+      float delta = 0.f;
+#pragma unroll
+      for (int i = 0; i < NF; ++i) delta = wv_dot<T>(gf[i], of[i], delta);
+      delta = wv_quad_sum(delta) - dl;
+      wv_lds<T>(xrow + n * RS, gq, qf);
+      wv_lds<T>(grow + n * RS, gq, gf);
+      if (gq == 0) {
+        crow[n] = cd;
+        lrow[n] = ls * kLog2e;
+        drow[n] = delta;
+      }
+      load(c + 1);
+      wv_lds_sync();
+      const uint4 cc = *reinterpret_cast<const uint4 *>(crow + 4 * gq);
+      const uint32_t c4[4] = {cc.x, cc.y, cc.z, cc.w};
+      const f32x4 l4 = *reinterpret_cast<const f32x4 *>(lrow + 4 * gq);
+      const f32x4 d4 = *reinterpret_cast<const f32x4 *>(drow + 4 * gq);
+      float p[4], ds[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float e = __builtin_amdgcn_exp2f(fmaf(s[r], P.sl2, -l4[r]));
+        p[r] = win.holds(c4[r]) ? e : 0.f;
+        ds[r] = win.holds(c4[r]) ? e * (dp[r] - d4[r]) : 0.f;
+      }
+      wv_acc<NDB, RS>(gt, p, adv);
+      wv_acc<NDB, RS>(xt, ds, adk);
+    }
+  }
+  if (wv_nan(adk, 0.f) || wv_nan(adv, 0.f)) {  // again, query by query
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) {
+      adk[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+      adv[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    for (int hr = 0; hr < P.rep; ++hr) {
+      const int h = t.h * P.rep + hr;
+      const char *qb = qc + ((t.b * P.Ltot + qtok) * P.H + h) * (D * ES);
+      const int64_t orow0 = (t.b * P.Otot + otok) * P.H + h;
+      for (int x = 0; x < box.npts; ++x) {
+        frag qf[NF], gf[NF], of[NF];
+        uint32_t qo, oo;
+        const uint32_t cd = box.point(x, qo, oo);
+        const char *gb = gc + orow0 * (D * ES), *ob = oc + orow0 * (D * ES);
+        ld_row<T>(qb, qo + 16u * gq, qf);
+        ld_row<T>(gb, oo + 16u * gq, gf);
+        ld_row<T>(ob, oo + 16u * gq, of);
+        float s = 0.f, dp = 0.f, delta = 0.f;
+#pragma unroll
+        for (int i = 0; i < NF; ++i) {
+          s = wv_dot<T>(kf[i], qf[i], s);
+          dp = wv_dot<T>(vf[i], gf[i], dp);
+          delta = wv_dot<T>(gf[i], of[i], delta);
+        }
+        s = wv_quad_sum(s);
+        dp = wv_quad_sum(dp);
+        delta = wv_quad_sum(delta);
+        const int64_t orow = orow0 + oo / rowsh;
+        if (dlse != nullptr) delta -= dlse[orow];
+        if (win.holds(cd)) {
+          const float pr = exp2f(fmaf(s, P.sl2, -lse[orow] * kLog2e));
+          const float ds = pr * (dp - delta);
+#pragma unroll
+          for (int db = 0; db < NDB; ++db) {
+            adv[db] += pr * ld4<T>(gb + oo + (16 * db + 4 * gq) * ES);
+            adk[db] += ds * ld4<T>(qb + qo + (16 * db + 4 * gq) * ES);
+          }
+        }
+      }
+    }
+  }
+  if (!kv) return;
+  char *dkb = reinterpret_cast<char *>(dk) + kofs + ko;
+  char *dvb = reinterpret_cast<char *>(dv) + kofs + ko;
+#pragma unroll
+  for (int db = 0; db < NDB; ++db) {
+    st4<T>(dkb + (16 * db + 4 * gq) * ES, adk[db] * P.scale);
+    st4<T>(dvb + (16 * db + 4 * gq) * ES, adv[db]);
+  }
+  if (STR && !on) {  // no query here: its rows of dq are zero
+    for (int hr = 0; hr < P.rep; ++hr) {
+      char *zb = reinterpret_cast<char *>(dq) +
+                 ((t.b * P.Ltot + ktok) * P.H + t.h * P.rep + hr) * (D * ES);
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+        st4<T>(zb + (16 * db + 4 * gq) * ES, f32x4{0.f, 0.f, 0.f, 0.f});
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Host side.
+
+int phase_max(const Axis &x) { return (x.L + x.d - 1) / x.d; }
+
+// Tile extents (product 16) with the fewest chunks over the grid.
+void wv_tile(const Prob &P, bool keys, int T[3]) {
+  const int lead = 3 - P.rank;
+  double best = 1e300;
+  for (int l0 = 0; l0 <= 4; ++l0)
+    for (int l1 = 0; l0 + l1 <= 4; ++l1) {
+      const int Tt[3] = {1 << l0, 1 << l1, 1 << (4 - l0 - l1)};
+      bool ok = true;
+      for (int a = 0; a < lead; ++a) ok = ok && Tt[a] == 1;
+      if (!ok) continue;
+      double tiles = 1.0, pts = 1.0;
+      for (int a = lead; a < 3; ++a) {
+        const Axis &x = P.ax[a];
+        const int Lr = phase_max(x), Qr = x.s == 1 ? Lr : x.O;
+        const int len = keys ? Lr : Qr;
+        tiles *= (double)x.d * ((len + Tt[a] - 1) / Tt[a]);
+        pts *= keys ? std::min(Qr, (Tt[a] + x.K - 2) / x.s + 1)
+                    : std::min(Lr, (Tt[a] - 1) * x.s + x.K);
+      }
+      const double cost = tiles * std::ceil(pts / 16.0);
+      if (cost < best) {
+        best = cost;
+        for (int a = 0; a < 3; ++a) T[a] = Tt[a];
+      }
+    }
+}
+
+WvGrid wv_grid(const Prob &P, bool keys, int waves) {
+  WvGrid G{};
+  int T[3] = {1, 1, 16};
+  wv_tile(P, keys, T);
+  int64_t grid = 1;
+  for (int a = 0; a < 3; ++a) {
+    const Axis &x = P.ax[a];
+    const int Lr = phase_max(x), len = keys || x.s == 1 ? Lr : x.O;
+    G.T[a] = T[a];
+    while ((1 << G.lgT[a]) < T[a]) ++G.lgT[a];
+    G.nt[a] = (len + T[a] - 1) / T[a];
+    G.fG[a] = make_fastdiv((uint32_t)(x.d * G.nt[a]));
+    G.fnt[a] = make_fastdiv((uint32_t)G.nt[a]);
+    grid *= (int64_t)x.d * G.nt[a];
+  }
+  G.fGrid = make_fastdiv((uint32_t)grid);
+  G.n_tiles = (int32_t)(P.B * (keys ? P.Hkv : P.H) * grid);
+  G.n_wg = ((G.n_tiles + waves - 1) / waves + 7) & ~7;
+  return G;
+}
+
+WvProb make_wvprob(const Prob &P, bool backward) {
+  WvProb W{};
+  W.B = P.B;
+  W.H = P.H;
+  W.Hkv = P.Hkv;
+  W.rep = P.rep;
+  int32_t tok = 1, otok = 1;
+  for (int a = 2; a >= 0; --a) {
+    const Axis &x = P.ax[a];
+    WvAx &y = W.ax[a];
+    y.K = x.K;
+    y.nh = x.K / 2;
+    y.d = x.d;
+    y.s = x.s;
+    y.causal = x.causal;
+    y.O = x.O;
+    y.Lq = x.L / x.d;
+    y.Lrem = x.L % x.d;
+    y.tok = tok;
+    y.otok = otok;
+    tok *= x.L;
+    otok *= x.O;
+  }
+  W.Ltot = tok;
+  W.Otot = otok;
+  W.fH = make_fastdiv((uint32_t)P.H);
+  W.fHkv = make_fastdiv((uint32_t)P.Hkv);
+  W.fRep = make_fastdiv((uint32_t)P.rep);
+  W.scale = P.scale;
+  W.sl2 = P.scale * kLog2e;
+  const int waves = P.D == 128 ? wv_waves<128>() : wv_waves<64>();
+  W.gq = wv_grid(P, false, waves);
+  if (backward) W.gk = wv_grid(P, true, waves);
+  return W;
+}
+
+bool strided(const Prob &P) { return P.ax[0].s != 1 || P.ax[1].s != 1 || P.ax[2].s != 1; }
+
+}  // namespace
+
+bool wave_eligible(const Prob &P, int dtype) {
+  if (P.dense || P.sample_extent != nullptr || P.n_extra > 0) return false;
+  if (dtype == NA_F32 ? (P.D != 16 && P.D != 32 && P.D != 64 && P.D != 128)
+                      : ((P.D != 32 && P.D != 64 && P.D != 128) || !strided(P)))
+    return false;
+  // the running maximum is taken over unscaled scores
+  if (!(P.scale > 0.f) || !std::isfinite(P.scale)) return false;
+  // box extents within the packed coordinate fields, box points within the
+  // range of the reciprocal division (an inverse box spans at most
+  // T + 2 (K - 1) points, a forward one (T - 1) s + K, s <= K: T <= 16)
+  const int64_t field = P.rank == 1 ? (int64_t)1 << 18 : P.rank == 2 ? 32767 : 511;
+  int64_t pts = 1;
+  for (int a = 3 - P.rank; a < 3; ++a) {
+    const Axis &x = P.ax[a];
+    if (x.s != 1 && (x.d != 1 || x.s > x.K)) return false;
+    if (!x.causal && ((x.K % 2) == 0 || (int64_t)x.d * x.K > x.L)) return false;
+    const int64_t e = std::min<int64_t>(phase_max(x), 16 + std::max<int64_t>(2 * x.K, 16 * x.s + x.K));
+    if (e > field) return false;
+    pts *= e;
+  }
+  if (pts > ((int64_t)1 << 18)) return false;
+  // 32-bit byte offsets inside a sample, 32-bit tile numbers
+  const int64_t es = dtype == NA_F32 ? 4 : 2;
+  const int64_t tokens = (int64_t)P.ax[0].L * P.ax[1].L * P.ax[2].L;
+  if (tokens * std::max(P.H, P.Hkv) * P.D * es >= ((int64_t)1 << 31)) return false;
+  return (int64_t)P.B * P.H * tokens < ((int64_t)1 << 30);
+}
+
+// The forward at head_dim 128 with strided queries: where a tile's box holds
+// many times a window's keys, the product over the box costs more than the
+// window alone on the vector ALU (K = 3 stride 3 on 4096 positions, 16 times:
+// bf16 7.5 us there, 9.8 here; float32 3 x 3 stride 2, 9 times: 16.6 and 20.4;
+// bf16 3 x 3 stride 2: 17.5 and 17.0).  Narrower heads gain at every ratio
+// (bf16 K = 3 stride 3: 5.9 -> 5.2 at head_dim 64), and so does the backward.
+bool wave_fwd_eligible(const Prob &P, int dtype) {
+  if (!wave_eligible(P, dtype)) return false;
+  if (P.D != 128 || !strided(P)) return true;
+  int T[3] = {1, 1, 16};
+  wv_tile(P, false, T);
+  int64_t pts = 1;
+  for (int a = 3 - P.rank; a < 3; ++a) {
+    const Axis &x = P.ax[a];
+    pts *= std::min(phase_max(x), (T[a] - 1) * x.s + x.K);
+  }
+  return pts <= (int64_t)P.kprod * (dtype == NA_F32 ? 8 : 12);
+}
+
+#define WV_R(KERNEL, TT, DD)                       \
+  do {                                             \
+    if (P.rank == 1) KERNEL(TT, DD, 1);            \
+    else if (P.rank == 2) KERNEL(TT, DD, 2);       \
+    else KERNEL(TT, DD, 3);                        \
+  } while (0)
+#define WV_D(KERNEL, TT)                           \
+  do {                                             \
+    if (P.D == 32) WV_R(KERNEL, TT, 32);           \
+    else if (P.D == 64) WV_R(KERNEL, TT, 64);      \
+    else WV_R(KERNEL, TT, 128);                    \
+  } while (0)
+#define WV_ALL(KERNEL)                                    \
+  do {                                                    \
+    if (dtype == NA_F32) {                                \
+      if (P.D == 16) WV_R(KERNEL, float, 16);             \
+      else WV_D(KERNEL, float);                           \
+    } else if (dtype == NA_BF16) {                        \
+      WV_D(KERNEL, bf16_t);                               \
+    } else {                                              \
+      WV_D(KERNEL, f16_t);                                \
+    }                                                     \
+  } while (0)
+
+void wave_fwd(const Prob &P, int dtype, const void *q, const void *k, const void *v, void *out,
+              float *lse, hipStream_t st) {
+  const WvProb W = make_wvprob(P, false);
+  if (W.gq.n_tiles == 0) return;
+#define WV_F(TT, DD, RR)                                                                        \
+  hipLaunchKernelGGL((k_wvfwd<TT, DD, RR>), dim3(W.gq.n_wg), dim3(64 * wv_waves<DD>()), 0, st, W, \
+                     (const TT *)q, (const TT *)k, (const TT *)v, (TT *)out, lse)
+  WV_ALL(WV_F);
+#undef WV_F
+}
+
+void wave_bwd(const Prob &P, int dtype, const void *q, const void *k, const void *v,
+              const void *out, const float *lse, const void *dout, const float *dlse, void *dq,
+              void *dk, void *dv, hipStream_t st) {
+  const WvProb W = make_wvprob(P, true);
+  if (W.gq.n_tiles == 0) return;
+  const bool str = strided(P);
+#define WV_BL(TT, DD, RR, SS)                                                               \
+  hipLaunchKernelGGL((k_wvbwd<TT, DD, RR, SS>), dim3(W.gk.n_wg + W.gq.n_wg),                \
+                     dim3(64 * wv_waves<DD>()), 0, st, W, (const TT *)q, (const TT *)k,     \
+                     (const TT *)v, (const TT *)out, lse, (const TT *)dout, dlse, (TT *)dq, \
+                     (TT *)dk, (TT *)dv)
+  // 16-bit problems come here only with a stride
+#define WV_B(TT, DD, RR)                                                       \
+  do {                                                                         \
+    if (sizeof(TT) == 2 || str) WV_BL(TT, DD, RR, true);                       \
+    else WV_BL(TT, DD, RR, (sizeof(TT) == 2));                                 \
+  } while (0)
+  WV_ALL(WV_B);
+#undef WV_B
+#undef WV_BL
+}
+
+#undef WV_ALL
+#undef WV_D
+#undef WV_R
+
+}  // namespace na

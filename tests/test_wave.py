@@ -1,0 +1,111 @@
+"""The 32-bit matrix-core kernels (na_wave.hip: float32, and strided
+bf16 / fp16): their window rules against the oracle's windows on the CPU, and
+on an MI355X forward + LSE + backward against the float64 oracle at the edges
+of their tiles, and non-finite values against the vector-ALU kernels."""
+
+import pytest
+import torch
+
+from _helpers import DEV, assert_close, randn
+from oracle import na as O
+from oracle import window as W
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("K,s", [(1, 1), (3, 1), (3, 2), (3, 3), (5, 2), (5, 4), (7, 3), (7, 7)])
+def test_strided_inverse_windows(K, s, causal):
+    """A key's queries: of the positions [j <= K-1 ? 0 : j - K/2, j >= L-K ?
+    L : j + K/2 + 1) (causal [j, j + K)) every s-th; both ends are
+    non-decreasing in j, so a tile of keys has a box of queries no longer
+    than (T - 1 + K - 1) / s + 1, or the K - 1 more of a clamped edge."""
+    for L in list(range(max(K, 1), 3 * K + 6)) + [40]:
+        n_out = -(-L // s)
+        idx, valid = W.axis_indices(range(0, L, s), L, K, 1, causal)
+        held = [set() for _ in range(L)]
+        for o in range(n_out):
+            for j, ok in zip(idx[o].tolist(), valid[o].tolist()):
+                if ok:
+                    held[j].add(o)
+        last = (0, 0)
+        for j in range(L):
+            lo = j if causal else (0 if j <= K - 1 else j - K // 2)
+            hi = min(j + K, L) if causal else (L if j >= L - K else j + K // 2 + 1)
+            lo, hi = -(-lo // s), min(-(-hi // s), n_out)
+            assert set(range(lo, hi)) == held[j], (L, K, s, j)
+            assert lo >= last[0] and hi >= last[1]
+            last = (lo, hi)
+
+
+def _ids(cases):
+    return [f"{c[0]}-{'x'.join(map(str, c[2]))}-d{c[5]}-k{'x'.join(map(str, c[6]))}"
+            f"-s{'x'.join(map(str, c[8]))}" for c in cases]
+
+
+F32, BF16, F16 = torch.float32, torch.bfloat16, torch.float16
+# (dtype, B, spatial, H, Hkv, D, kernel, dilation, stride, causal)
+CASES = [
+    (F32, 1, (1,), 1, 1, 16, (1,), (1,), (1,), (True,)),            # one row
+    (F32, 2, (16,), 2, 1, 32, (3,), (1,), (1,), (False,)),          # one whole tile
+    (F32, 1, (17,), 3, 3, 64, (15,), (1,), (1,), (False,)),         # one row over
+    (F32, 1, (150,), 4, 2, 128, (63,), (2,), (1,), (False,)),       # wide box, phases
+    (F32, 2, (13, 11), 2, 2, 32, (7, 7), (1, 1), (1, 1), (False, False)),
+    (F32, 1, (9, 33), 2, 1, 16, (3, 5), (3, 2), (1, 1), (False, True)),
+    (F32, 1, (14, 17), 6, 2, 64, (5, 7), (1, 1), (2, 3), (False, True)),
+    (F32, 1, (6, 9, 10), 2, 1, 32, (3, 5, 3), (1, 1, 3), (1, 2, 1), (True, False, False)),
+    (BF16, 2, (31,), 2, 2, 64, (5,), (1,), (4,), (False,)),
+    (BF16, 1, (19, 23), 4, 2, 32, (7, 3), (1, 2), (5, 1), (False, False)),
+    (F16, 1, (15, 12), 2, 1, 128, (3, 5), (1, 1), (3, 2), (False, False)),
+    (F16, 1, (7, 8, 9), 2, 2, 32, (3, 3, 5), (1, 1, 1), (3, 1, 2), (False, True, False)),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES, ids=_ids(CASES))
+def test_against_oracle(case):
+    import natten_amd
+
+    dtype, B, sp, H, Hkv, D, ks, dil, st, caus = case
+    print(f"[case] wave {case}", flush=True)
+    fn = {1: natten_amd.na1d, 2: natten_amd.na2d, 3: natten_amd.na3d}[len(sp)]
+    q, k, v = (randn((B, *sp, h, D), dtype, i) for i, h in enumerate((H, Hkv, Hkv)))
+    ts = [t.to(DEV).requires_grad_(True) for t in (q, k, v)]
+    out, lse = fn(*ts, ks, st, dil, caus, return_lse=True)
+
+    def f(a, b, c):
+        return O.na_functional(a, b, c, ks, st, dil, caus, return_lse=True)
+
+    ro, rl = f(q, k, v)
+    assert_close(out, ro, dtype, "out")
+    assert_close(lse, rl, dtype, "lse")
+    go, gl = randn(out.shape, dtype, 7), randn(lse.shape, dtype, 8)
+    torch.autograd.backward((out, lse), (go.to(DEV), gl.to(DEV)))
+    for t, r, n in zip(ts, O.grads(f, (q, k, v), (go, gl)), ("dq", "dk", "dv")):
+        assert_close(t.grad, r, dtype, n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("where", ["q", "k", "v", "grad"])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")], ids=str)
+def test_non_finite_values_stay_in_their_windows(where, bad):
+    """A tile's product runs over a box wider than its queries' windows; a
+    NaN or infinity may reach no more than the vector-ALU kernels let it reach
+    (they also give NaN where a window's first score is -inf)."""
+    import natten_amd
+    from natten_amd._core import hip
+
+    for dtype, st in ((F32, 1), (BF16, 2)):
+        ts = [randn((1, 21, 19, 2, 32), dtype, i).to(DEV) for i in range(3)]
+        go = randn((1, -(-21 // st), -(-19 // st), 2, 32), dtype, 3).to(DEV)
+        bad_t = dict(zip(("q", "k", "v", "grad"), (*ts, go)))[where]
+        bad_t[0, 6, 4, 1, 3] = bad
+        ts = [t.requires_grad_(True) for t in ts]
+        res = []
+        for generic in (False, True):
+            with hip.generic_kernels(generic):
+                out = natten_amd.na2d(*ts, (7, 5), st)
+                res.append([out, *torch.autograd.grad(out, ts, go)])
+        for a, b in zip(*res):
+            fin = torch.isfinite(b)
+            assert bool(fin.any()) and bool(torch.isfinite(a[fin]).all())
+            assert_close(a[fin], b[fin].double(), dtype, where)
+        assert where == "grad" or not bool(torch.isfinite(res[0][0]).all())
