@@ -63,6 +63,8 @@ EXTRA_FLAGS = {
     "na_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "na_lean.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "na_dense.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "na_wave.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "na_wsplit.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 

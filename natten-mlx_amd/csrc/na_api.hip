@@ -150,6 +150,10 @@ bool use_wave_bwd(const na_params *p, const na::Prob &P) {
   return (p->flags & NA_FLAG_GENERIC) == 0 && na::wave_eligible(P, p->dtype);
 }
 
+bool use_wsplit(const na_params *p, const na::Prob &P, na::WsplitPass pass) {
+  return (p->flags & NA_FLAG_GENERIC) == 0 && na::wsplit_eligible(P, p->dtype, pass);
+}
+
 size_t align256(size_t n) { return (n + 255) & ~size_t(255); }
 
 size_t delta_bytes(const na::Prob &P) {
@@ -569,6 +573,8 @@ int na_qk_fwd(const na_params *p, const void *q, const void *k, void *logits,
   else if (use_msplit(p, P))
     na::msplit_qk(P, p->dtype, q, k, logits, P.scale, -INFINITY,
                   as_stream(stream));
+  else if (use_wsplit(p, P, na::kWsQk))
+    na::wsplit_qk(P, q, k, logits, as_stream(stream));
   else
     na::valu_qk(P, p->dtype, q, k, logits, as_stream(stream));
   return launch_status("na_qk_fwd");
@@ -587,6 +593,8 @@ int na_av_fwd(const na_params *p, const void *attn, const void *v, void *out,
     na::lsplit_av(P, p->dtype, attn, v, out, 1.f, as_stream(stream));
   else if (use_msplit(p, P))
     na::msplit_av(P, p->dtype, attn, v, out, 1.f, as_stream(stream));
+  else if (use_wsplit(p, P, na::kWsAv))
+    na::wsplit_av(P, attn, v, out, as_stream(stream));
   else
     na::valu_av(P, p->dtype, attn, v, out, as_stream(stream));
   return launch_status("na_av_fwd");
@@ -607,6 +615,8 @@ int na_qk_bwd(const na_params *p, const void *q, const void *k,
   } else if (use_msplit(p, P)) {
     na::msplit_av(P, p->dtype, dlogits, k, dq, P.scale, as_stream(stream));
     na::msplit_inv(P, p->dtype, dlogits, q, dk, P.scale, as_stream(stream));
+  } else if (use_wsplit(p, P, na::kWsBwd)) {
+    na::wsplit_qk_bwd(P, q, k, dlogits, dq, dk, as_stream(stream));
   } else {
     na::valu_qk_bwd(P, p->dtype, q, k, dlogits, dq, dk, as_stream(stream));
   }
@@ -628,6 +638,8 @@ int na_av_bwd(const na_params *p, const void *attn, const void *v,
   } else if (use_msplit(p, P)) {
     na::msplit_qk(P, p->dtype, dout, v, dattn, 1.f, 0.f, as_stream(stream));
     na::msplit_inv(P, p->dtype, attn, dout, dv, 1.f, as_stream(stream));
+  } else if (use_wsplit(p, P, na::kWsBwd)) {
+    na::wsplit_av_bwd(P, attn, v, dout, dattn, dv, as_stream(stream));
   } else {
     na::valu_av_bwd(P, p->dtype, attn, v, dout, dattn, dv, as_stream(stream));
   }

@@ -178,6 +178,29 @@ void wave_bwd(const Prob &P, int dtype, const void *q, const void *k,
               const void *dout, const float *dlse, void *dq, void *dk,
               void *dv, hipStream_t st);
 
+// Float32 split ops, and the allin1 ops on float32 rows of rank 2 (or head_dim
+// above 16), on float32 matrix cores (na_wsplit.hip): stride 1, odd K with
+// d*K <= L or causal axes, at most 512 slots.
+enum WsplitPass { kWsQk, kWsAv, kWsBwd };
+bool wsplit_eligible(const Prob &P, int dtype, WsplitPass pass);
+void wsplit_qk(const Prob &P, const void *q, const void *k, void *logits, hipStream_t st);
+void wsplit_av(const Prob &P, const void *attn, const void *v, void *out, hipStream_t st);
+void wsplit_qk_bwd(const Prob &P, const void *q, const void *k, const void *dl, void *dq,
+                   void *dk, hipStream_t st);
+void wsplit_av_bwd(const Prob &P, const void *attn, const void *v, const void *dout,
+                   void *dattn, void *dv, hipStream_t st);
+bool wsplit_rpb_eligible(const RpbProb &A, WsplitPass pass);
+void wsplit_rpb_dot(const RpbProb &A, const float *x, const float *y, const float *rpb,
+                    float *out, int scale_x, float fill, hipStream_t st);
+void wsplit_rpb_gather(const RpbProb &A, const float *w, const float *y, float *out,
+                       float post, hipStream_t st);
+void wsplit_rpb_inverse(const RpbProb &A, const float *w, const float *x, float *out,
+                        float post, hipStream_t st);
+void wsplit_rpb_qk_bwd(const RpbProb &A, const float *dl, const float *q, const float *key,
+                       float *dq, float *dk, hipStream_t st);
+void wsplit_rpb_av_bwd(const RpbProb &A, const float *attn, const float *v,
+                       const float *dout, float *dattn, float *dv, hipStream_t st);
+
 // Generic pieces reused around the MFMA backward.
 void valu_delta(const Prob &P, int dtype, const void *out, const void *dout,
                 const float *dlse, float *delta, hipStream_t st);

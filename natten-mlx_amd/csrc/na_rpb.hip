@@ -2171,6 +2171,10 @@ void launch_dot(const RpbProb &A, const void *x, const void *y,
                 hipStream_t st) {
   if constexpr (sizeof(TX) == 4 && sizeof(TY) == 4) {
     if (r1_dot(A, (const float *)x, (const float *)y, rpb, out, scale_x, st)) return;
+    if (wsplit_rpb_eligible(A, kWsQk)) {
+      wsplit_rpb_dot(A, (const float *)x, (const float *)y, rpb, out, scale_x, fill, st);
+      return;
+    }
   }
   constexpr int V = vmax_of<TX, TY>();
   const RShape s = rshape(A.D, V);
@@ -2200,6 +2204,10 @@ void launch_gather(const RpbProb &A, const float *w, const void *y, void *out,
                    float post, hipStream_t st) {
   if constexpr (sizeof(TY) == 4 && sizeof(TO) == 4) {
     if (r1_gather(A, w, (const float *)y, (float *)out, post, st)) return;
+    if (wsplit_rpb_eligible(A, kWsAv)) {
+      wsplit_rpb_gather(A, w, (const float *)y, (float *)out, post, st);
+      return;
+    }
   }
   constexpr int V = vmax_of<TY, TO>();
   const RShape s = rshape(A.D, V);
@@ -2230,6 +2238,10 @@ void launch_inverse(const RpbProb &A, const float *w, const void *x, void *out,
       return;
     if (r1_inverse(A, w, (const float *)x, (float *)out, post, st)) return;
     if (r1p_inverse(A, w, (const float *)x, (float *)out, post, st)) return;
+    if (wsplit_rpb_eligible(A, kWsBwd)) {
+      wsplit_rpb_inverse(A, w, (const float *)x, (float *)out, post, st);
+      return;
+    }
   }
   constexpr int V = vmax_of<TX, TO>();
   const RShape s = rshape(A.D, V);
@@ -2315,6 +2327,11 @@ void rpb_qk_bwd(const RpbProb &A, int dtype, const void *q, const void *key,
       pair = true;
       if (pbias) n_fused = nph;
     }
+    if (!pair && wsplit_rpb_eligible(A, kWsBwd)) {
+      wsplit_rpb_qk_bwd(A, dlogits, (const float *)q, (const float *)key, (float *)dq,
+                        (float *)dk, st);
+      pair = true;
+    }
   }
   if (!pair && drpb != nullptr && dq != nullptr && dtype == NA_F32 && A.n_rows > 0) {
     // the staged gather's blocks, or the phase-major one's
@@ -2399,6 +2416,11 @@ void rpb_av_bwd(const RpbProb &A, int dtype, int out_dtype, const float *attn,
        r1p_av_bwd_pair(A, attn, (const float *)value, (const float *)dout, dattn,
                        (float *)dvalue, st)))
     return;
+  if (dtype == NA_F32 && dattn != nullptr && dvalue != nullptr && wsplit_rpb_eligible(A, kWsBwd)) {
+    wsplit_rpb_av_bwd(A, attn, (const float *)value, (const float *)dout, dattn,
+                      (float *)dvalue, st);
+    return;
+  }
   with_dtype(dtype, [&](auto tag) {
     using T = decltype(tag);
     if (out_dtype == NA_F32) {

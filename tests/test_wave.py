@@ -109,3 +109,70 @@ def test_non_finite_values_stay_in_their_windows(where, bad):
             assert bool(fin.any()) and bool(torch.isfinite(a[fin]).all())
             assert_close(a[fin], b[fin].double(), dtype, where)
         assert where == "grad" or not bool(torch.isfinite(res[0][0]).all())
+
+
+# (B, spatial, H, Hkv, D, kernel, dilation, causal): the float32 split ops
+SPLIT = [
+    (1, (15,), 1, 1, 16, (13,), (1,), (False,)),               # a tile less one row
+    (2, (49,), 2, 1, 64, (7,), (3,), (False,)),                # phases, one row over
+    (1, (33,), 1, 1, 128, (31,), (1,), (True,)),               # causal: slots before the sample
+    (1, (9, 17), 2, 2, 32, (5, 5), (1, 3), (False, False)),
+    (2, (8, 13), 4, 2, 16, (3, 7), (2, 1), (True, False)),
+    (1, (5, 6, 9), 3, 1, 32, (3, 3, 5), (1, 2, 1), (False, True, False)),
+    (1, (24, 24), 1, 1, 32, (21, 23), (1, 1), (False, False)),  # most slots: one wave per group
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", SPLIT, ids=[f"{'x'.join(map(str, c[1]))}-d{c[4]}" for c in SPLIT])
+def test_split_against_oracle(case):
+    import natten_amd
+    from natten_amd import functional as F
+
+    B, sp, H, Hkv, D, ks, dil, caus = case
+    print(f"[case] wave split {case}", flush=True)
+    r = len(sp)
+    qk, av = getattr(F, f"na{r}d_qk"), getattr(F, f"na{r}d_av")
+    q, k, v = (randn((B, *sp, h, D), F32, i) for i, h in enumerate((H, Hkv, Hkv)))
+    ts = [t.to(DEV).requires_grad_(True) for t in (q, k, v)]
+    logits = qk(ts[0], ts[1], ks, dil, is_causal=caus, scale=0.3)
+    ref_l = O.na_qk(q, k, ks, 1, dil, caus, 0.3)
+    assert_close(logits, ref_l, F32, "logits")
+    attn = torch.softmax(ref_l, -1).float()
+    ta = attn.to(DEV).requires_grad_(True)
+    out = av(ta, ts[2], ks, dil, is_causal=caus)
+    assert_close(out, O.na_av(attn, v, ks, 1, dil, caus), F32, "out")
+    gl = randn(logits.shape, F32, 7)
+    go = randn(out.shape, F32, 8)
+    got = (*torch.autograd.grad(logits, ts[:2], gl.to(DEV)),
+           *torch.autograd.grad(out, (ta, ts[2]), go.to(DEV)))
+    gl = torch.where(torch.isfinite(ref_l), gl.double(), 0.0)  # no gradient at -inf
+    ref = (*O.grads(lambda a, b: torch.where(torch.isfinite(ref_l),
+                                             O.na_qk(a, b, ks, 1, dil, caus, 0.3), 0.0),
+                    (q, k), (gl,)),
+           *O.grads(lambda a, b: O.na_av(a, b, ks, 1, dil, caus), (attn, v), (go,)))
+    for g, w, n in zip(got, ref, ("dq", "dk", "dattn", "dv")):
+        # sums of up to 483 products of unit normals in float32
+        assert_close(g, w, F32, n, scale_tol=4.0)
+
+
+@pytest.mark.gpu
+def test_split_non_finite_values_stay_in_their_windows():
+    """As above for AV and the inverse pass, whose products run over a box."""
+    from natten_amd import functional as F
+
+    q, v, k = (randn((1, 21, 19, 2, 32), F32, i).to(DEV) for i in range(3))
+    clean = [F.na2d_av(torch.softmax(F.na2d_qk(q, k, 7), -1), v, 7)]
+    v2 = v.clone()
+    v2[0, 6, 4, 1, 3] = float("nan")
+    out = F.na2d_av(torch.softmax(F.na2d_qk(q, k, 7), -1), v2, 7)
+    bad = torch.isnan(out)
+    holds = torch.zeros(21, 19, dtype=torch.bool)
+    for i in range(21):
+        for j in range(19):
+            a, b = min(max(i - 3, 0), 14), min(max(j - 3, 0), 12)
+            holds[i, j] = a <= 6 < a + 7 and b <= 4 < b + 7
+    want = torch.zeros_like(bad)
+    want[0, :, :, 1, 3] = holds.to(DEV)
+    assert torch.equal(bad, want)
+    assert torch.allclose(out[~bad], clean[0][~bad], atol=1e-6)
