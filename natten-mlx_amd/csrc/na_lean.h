@@ -82,7 +82,8 @@ struct LProb {
   int32_t ebox;       // staged rows: Em2 (rank 1) or Em0 * Em1 * 2^lgP2
   int32_t lgP2;       // rank >= 2: staged box rows are 2^lgP2 >= Em2 wide
   int32_t rep;        // query heads per key/value head
-  int32_t sl;         // rank 3: box layers (axis 0) staged at a time
+  int32_t sl;         // box layers (rank 3: axis 0) or rows (rank 2: axis 1)
+                      // staged at a time
   float scale;
   FastDiv fH, fRep;
   FastDiv fHkv;       // key/value heads
@@ -330,8 +331,8 @@ __device__ __forceinline__ float ldf(const float *base, int off) {
 
 // Element offset of staged-box unit (row kk of the LDS layout, 16-byte unit
 // o): box coordinates from the layout (shifts; rank 3 divides by Em1 and
-// adds the first staged layer s0), clamped onto the tile's true box, then
-// 24-bit products with the strides.
+// adds the first staged layer s0; rank 2 the first staged row), clamped onto
+// the tile's true box, then 24-bit products with the strides.
 template <int R>
 __device__ __forceinline__ int unit_offset(const LProb &P, const LTile &t,
                                            int kk, int o, int s0) {
@@ -340,7 +341,7 @@ __device__ __forceinline__ int unit_offset(const LProb &P, const LTile &t,
     const int row = kk >> P.lgP2;
     e2 = kk & ((1 << P.lgP2) - 1);
     if (R == 2) {
-      e1 = row;
+      e1 = row + s0;
     } else {
       e0 = (int)fdiv((uint32_t)row, P.fE1);
       e1 = row - e0 * P.ax[1].Em;
@@ -387,11 +388,12 @@ __device__ __forceinline__ void unit_walk(const LProb &P, const LTile &t,
     const int row0 = kk0 >> P.lgP2, drow = step >> P.lgP2;
     int base = t.kbase + 8 * o + __umul24((unsigned)min(e2, t.E[2] - 1), (unsigned)t.SK[2]);
     if (R == 3) base += __umul24((unsigned)min(s0, t.E[0] - 1), (unsigned)t.SK[0]);
-    const int Em1 = P.ax[1].Em;
+    const int rows = R == 2 ? P.sl : P.ax[1].Em;  // staged rows, from row r0
+    const int r0 = R == 2 ? s0 : 0;
 #pragma unroll
     for (int j = 0; j < NU; ++j) {
-      const int row = min(row0 + j * drow, Em1 - 1);
-      g[j] = base + __umul24((unsigned)min(row, t.E[1] - 1), (unsigned)t.SK[1]);
+      const int row = min(row0 + j * drow, rows - 1);
+      g[j] = base + __umul24((unsigned)min(row + r0, t.E[1] - 1), (unsigned)t.SK[1]);
       la[j] = __umul24((row << P.lgP2) + e2, RS) + 8 * o;
     }
     return;
@@ -521,22 +523,24 @@ __device__ __forceinline__ void stage_box(const LProb &P, const LTile &t,
 
 // A slab of the box of two tensors staged in two steps, so its loads can be
 // in flight while the previous slab is computed: load() issues every unit
-// of the lane (two rounds of four, the units of stage_box) into registers,
+// of the lane (NR rounds of four, the units of stage_box) into registers,
 // store() writes them to LDS.  Used where a box is staged in several slabs
-// and two rounds cover a slab (ebox * D / 8 <= 8 * nthr).
+// and NR rounds cover a slab (ebox * D / 8 <= 4 NR nthr): two at rank 3, one
+// at rank 2, whose slabs are a few rows.
 template <typename T, int D, int R>
 struct SlabPrefetch {
+  static constexpr int NR = R == 2 ? 1 : 2;
   typedef typename L16<T>::v8 v8;
   static constexpr int OCT = D / 8;
   static constexpr int RSE = lds_row(D);
-  v8 x[2][4], y[2][4];
-  int la[2][4];
+  v8 x[NR][4], y[NR][4];
+  int la[NR][4];
   __device__ __forceinline__ void load(const LProb &P, const LTile &t,
                                        const T *__restrict__ xg,
                                        const T *__restrict__ yg, int tid, int nthr,
                                        int s0) {
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
+    for (int r = 0; r < NR; ++r) {
       int g[4];
       // a round past the layout clamps to its last row (real rows,
       // rewritten with the same values)
@@ -551,7 +555,7 @@ struct SlabPrefetch {
   __device__ __forceinline__ void store(typename L16<T>::e *xs,
                                         typename L16<T>::e *ys) const {
 #pragma unroll
-    for (int r = 0; r < 2; ++r)
+    for (int r = 0; r < NR; ++r)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         *reinterpret_cast<v8 *>(xs + la[r][j]) = x[r][j];
@@ -570,6 +574,16 @@ int ilog2c(int x) {
 }
 
 constexpr size_t kLdsBudget = 80 * 1024;  // per workgroup: >= 2 per CU
+
+// Rank-2 forward boxes beyond this are staged in row slabs although they would
+// fit the budget: three workgroups to a CU instead of two ([2, 96, 96, 8, 64]
+// K = 9, 78 KB: 27.4 -> 22.7 us; [2, 112, 112, 4, 64] K = 5, 60 KB: 19.5 ->
+// 16.4; [2, 72, 100, 8, 128] K = 5: 41 -> 28).  Head_dim 32, with half the
+// loads per row, gains from four workgroups per CU on ([4, 112, 112, 4, 32]
+// K = 11: 34.2 -> 31.9; [4, 56, 56, 4, 32] K = 13: 13.1 -> 14.0).  The backward, whose slabs restage
+// the query box too, keeps what fits ([4, 56, 56, 4, 64] K = 7, 69 KB: 26.4 us
+// whole, 30.9 in slabs).
+constexpr size_t kRowSlabBox = 160 * 1024 / 3;
 
 // LDS budget per workgroup; NATTEN_AMD_LEAN_LDS_KB overrides it (tuning).
 size_t lds_budget() {
@@ -607,7 +621,8 @@ struct LChoice {
   int T[3];      // wave tile (product 16 over the active axes)
   int W, sa;     // waves per workgroup and the axis they are stacked along
   int Em[3];     // workgroup key box (largest over tiles)
-  int sl;        // rank 3: box layers staged at a time (Em[0]: all at once)
+  int sl;        // box layers (rank 3) or rows (rank 2) staged at a time
+                 // (Em of that axis: all at once)
   bool cpr1;     // every wave sub-box row is at most 16 keys wide
   bool ok;
 };
@@ -619,6 +634,9 @@ int lds_rows(int R, const int Em[3]) {
   while (p2 < Em[2]) p2 <<= 1;
   return Em[0] * Em[1] * p2;
 }
+
+// The axis a box is staged along in slabs: layers at rank 3, rows at rank 2.
+int slab_axis(int R) { return R == 2 ? 1 : 0; }
 
 // LDS rows of the additional tokens (forward): n_extra rounded up to 16.
 int lean_nxr(const Prob &P) { return (P.n_extra + 15) & ~15; }
@@ -745,15 +763,37 @@ LChoice lean_choice_compute(const Prob &P, LMode mode) {
       if (W > 1 && best.T[sa] * (W - 1) >= (x.L + x.d - 1) / x.d) continue;
       int Em[3];
       for (int a = 0; a < 3; ++a) Em[a] = ext(a, best.T[a] * (a == sa ? W : 1));
-      // rank 3 may stage the box a few layers (axis 0) at a time
-      int sl = Em[0];
-      while (sl > 1 && lean_lds_bytes(P, mode, lds_rows(R, Em) / Em[0] * sl, W) > lds_budget())
-        --sl;
-      const int ebox = lds_rows(R, Em) / Em[0] * sl;
+      // rank 3 may stage the box a few layers (axis 0) at a time; the fused
+      // rank-2 kernels a few rows, as many as one round of prefetched units
+      // covers, where a wave's part of a row is one chunk (the backward: two,
+      // which an inverse box has beside an edge of the image)
+      const int sx = slab_axis(R);
+      int sl = Em[sx];
+      const int lrows = lds_rows(R, Em) / Em[sx];  // LDS rows per layer or row
+      const bool rows2 = R == 2 && P.sample_extent == nullptr && P.n_extra == 0 &&
+                         ((best.cpr1 && (mode == kLFwd || mode == kLBwd)) ||
+                          (mode == kLBwd && ext(2, best.T[2]) <= 32));
+      bool early = rows2 && mode == kLFwd;  // slabs before the budget asks for them
+      if (early && P.D == 32) {
+        int64_t wgs = (int64_t)P.B * P.H;
+        for (int a = lead; a < 3; ++a) {
+          const int tw = best.T[a] * (a == sa ? W : 1), Lr = (P.ax[a].L + P.ax[a].d - 1) / P.ax[a].d;
+          wgs *= (int64_t)P.ax[a].d * ((Lr + tw - 1) / tw);
+        }
+        early = wgs >= 4 * kLeanCUs;
+      }
+      if (R == 2 &&
+          lean_lds_bytes(P, mode, lrows * sl, W) > (early ? kRowSlabBox : lds_budget())) {
+        if (!rows2) continue;
+        sl = std::min(sl, 4 * 64 * W / (P.D / 8) / lrows);
+        if (sl < 1) continue;
+      }
+      while (R == 3 && sl > 1 && lean_lds_bytes(P, mode, lrows * sl, W) > lds_budget()) --sl;
+      const int ebox = lrows * sl;
       if (lean_lds_bytes(P, mode, ebox, W) > lds_budget()) continue;
       // staged rows per wave over all slabs, each extra slab (a restaging
       // round trip and barrier) counted as a quarter more
-      const int nsl = (Em[0] + sl - 1) / sl;
+      const int nsl = (Em[sx] + sl - 1) / sl;
       const double per_wave = (double)lds_rows(R, Em) / W * (1.0 + 0.25 * (nsl - 1));
       if (per_wave < best_per_wave * 0.999 ||
           (per_wave < best_per_wave * 1.001 && sl > best.sl)) {
@@ -773,7 +813,7 @@ LChoice lean_choice_compute(const Prob &P, LMode mode) {
   // CU where 784 four-wave ones put 16 (13.9 vs 14.3 us; the forward,
   // lighter per wave, is not faster with them).  NATTEN_AMD_LEAN_WAVES
   // turns this off.
-  if (best.ok && mode == kLBwd && R == 2 && !lean_waves_forced()) {
+  if (best.ok && mode == kLBwd && R == 2 && best.sl == best.Em[1] && !lean_waves_forced()) {
     auto tiles_of = [&](int W, int sa) {
       int64_t n = (int64_t)P.B * P.Hkv;
       for (int a = lead; a < 3; ++a) {
@@ -803,7 +843,7 @@ LChoice lean_choice_compute(const Prob &P, LMode mode) {
           cur = b;
           best.W = W;
           best.sa = sa;
-          best.sl = Em[0];
+          best.sl = Em[1];
           for (int a = 0; a < 3; ++a) best.Em[a] = Em[a];
         }
       }
@@ -886,7 +926,7 @@ LProb make_lprob(const Prob &P, const LChoice &C) {
     y.fd = make_fastdiv((uint32_t)x.d);
     grid *= x.d * y.nt;
   }
-  L.ebox = lds_rows(P.rank, C.Em) / C.Em[0] * C.sl;
+  L.ebox = lds_rows(P.rank, C.Em) / C.Em[slab_axis(P.rank)] * C.sl;
   L.sl = C.sl;
   L.hl = 0;
   L.fHg = make_fastdiv(1u);
@@ -926,9 +966,10 @@ bool lean_shape_ok(const Prob &P, int dtype) {
   const int64_t elems = (int64_t)P.B * P.ax[0].L * P.ax[1].L * P.ax[2].L *
                         std::max(P.H, P.Hkv) * P.D;
   if (elems >= (int64_t(1) << 31)) return false;
-  // per-axis element strides fit the 24-bit multiplies of the staging code
+  // element strides of the problem's own axes fit the 24-bit multiplies of the
+  // staging code (a unit axis before them has no steps)
   int64_t tok = 1;
-  for (int a = 2; a >= 0; --a) {
+  for (int a = 2; a >= 3 - P.rank; --a) {
     if ((int64_t)P.ax[a].d * tok * std::max(P.H, P.Hkv) * P.D >= (int64_t(1) << 24))
       return false;
     tok *= P.ax[a].L;

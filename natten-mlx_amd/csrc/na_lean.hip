@@ -127,7 +127,13 @@ __device__ __forceinline__ void fwd_group(const typename L16<T>::e *ks,
 // rule alone (the causal fields are known zero at compile time, so the
 // setup's selects between the two rules fold away).
 // PFS: the box is staged in several slabs and each slab's loads are issued
-// while the previous slab is computed (SlabPrefetch).
+// while the previous slab is computed (SlabPrefetch).  At rank 2 slabs are box
+// rows and only this form has them: a box that does not fit LDS whole (head_dim
+// 64 from K = 9 to 13, head_dim 128 from K = 5) ran as one-wave workgroups or on
+// 32-query tiles straight from L2 (fp16 [1, 384, 384, 8, 64] K = 13 forward 494
+// -> 292 us, backward 1358 -> 1102; [1, 256, 256, 16, 128] K = 7 454 -> 267 and
+// 1247 -> 907; [2, 96, 96, 8, 64] K = 9 backward 245 -> 92).  Loading a slab after
+// the one before it is done instead: 318 and 1152 us for the first of these.
 template <typename T, int D, int R, bool CPR1, bool VX, bool CA, bool PFS>
 __global__ void __launch_bounds__(512)
     k_wfwd(LProb Pin, const T *__restrict__ q, const T *__restrict__ k,
@@ -144,6 +150,8 @@ __global__ void __launch_bounds__(512)
   constexpr int NB = 256 / D;   // chunks per softmax group
   constexpr int NDB = D / 16;   // 16-row blocks of O^T
   constexpr int RSE = lds_row(D);
+  constexpr bool SLAB2 = R == 2 && PFS;      // slabs of box rows
+  constexpr int SX = R == 2 ? 1 : 0;         // the slabs' axis
   extern __shared__ __align__(16) char smem[];
 
   // setup is straight-line arithmetic on kernel arguments (so their loads
@@ -267,8 +275,8 @@ __global__ void __launch_bounds__(512)
   // 8 gq) and the transposing read (row 4 gq + n / 4, column 4 (n % 4))
   const int ka_off = n * RSE + 8 * gq;
   const int tr_off = (4 * gq + (n >> 2)) * RSE + 4 * (n & 3);
-  const int nsl = R == 3 ? (t.E[0] + P.sl - 1) / P.sl : 1;
-  const int rows1 = R > 1 ? ws.we[1] - ws.ws[1] : 1;
+  const int nsl = R == 3 || SLAB2 ? (t.E[SX] + P.sl - 1) / P.sl : 1;
+  const int rows1 = R > 1 && !SLAB2 ? ws.we[1] - ws.ws[1] : 1;
   // additional-token chunks, run after the last slab's box chunks; their
   // rows sit before the box (LDS rows -nxr .. -1 from ks)
   const int nxc = VX ? nxr >> 4 : 0;
@@ -291,12 +299,14 @@ __global__ void __launch_bounds__(512)
     }
     if (!ws.any) continue;
     // the wave's box rows inside this slab
-    const int a0 = R == 3 ? max(ws.ws[0], s0) : 0;
-    const int b0 = R == 3 ? min(ws.we[0], s0 + P.sl) : 1;
+    const int a0 = R == 3 || SLAB2 ? max(ws.ws[SX], s0) : 0;
+    const int b0 = R == 3 || SLAB2 ? min(ws.we[SX], s0 + P.sl) : 1;
     const int nchb = b0 > a0 ? (b0 - a0) * rows1 * ws.cpr : 0;
     const int nch = nchb + (si == nsl - 1 ? nxc : 0);
     Cursor cc{a0, ws.ws[1], 0};
-    const int key0 = (((a0 - s0) * Em1 + ws.ws[1]) << P.lgP2) + ws.ws[2];
+    const int e1b = SLAB2 ? a0 : ws.ws[1];  // the first chunk's box row
+    const int key0 = SLAB2 ? ((a0 - s0) << P.lgP2) + ws.ws[2]
+                           : (((a0 - s0) * Em1 + ws.ws[1]) << P.lgP2) + ws.ws[2];
     // chunk rows and masks of a group of G chunks from chunk c0
     auto group = [&](int c0, auto g_) {
       constexpr int G = decltype(g_)::value;
@@ -311,7 +321,7 @@ __global__ void __launch_bounds__(512)
         // closed forms: one box row (rank 1) or one chunk per row (rank 2,
         // CPR1; rank 3, CPR1, whose slabs are one layer a0); otherwise the
         // cursor
-        const int e1 = R >= 2 && CPR1 ? ws.ws[1] + c : cc.e1;
+        const int e1 = R >= 2 && CPR1 ? e1b + c : cc.e1;
         const int cs = R == 1 ? c : CPR1 ? 0 : cc.cs;
         if (R > 1) ok = ok && (unsigned)(e1 - wl[1]) < (unsigned)ww[1];
         if (R == 3) ok = ok && (unsigned)((CPR1 ? a0 : cc.e0) - wl[0]) < (unsigned)ww[0];
@@ -494,14 +504,16 @@ __device__ __forceinline__ int lane_rows(const LProb &P, const LTile &t,
 // Closed forms where the walk is one box row (rank 1: chunk c is columns
 // 16 c..) or one chunk per row (rank 2, CPR1: chunk c is row ws1 + c; rank
 // 3, CPR1, a slab of one layer a0: the same on that layer, whose row test
-// l0ok is the caller's); otherwise the cursor walks rows and segments.
+// l0ok is the caller's; rank 2, a slab's rows from e1b: chunk c is row e1b +
+// c); otherwise the cursor walks rows and segments.
 template <int R, bool CPR1>
 __device__ __forceinline__ void pair_rows(const WSub &ws, Cursor &cc, int c0,
                                           int nch, int s0, int Em1, int lgP2,
                                           int key0,
                                           const int wl[3], const int ww[3],
                                           int kb[2], bool rok[2], int cs[2],
-                                          bool layer = false, bool l0ok = false) {
+                                          bool layer = false, bool l0ok = false,
+                                          int e1b = -1) {
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int c = c0 + h;
@@ -513,9 +525,11 @@ __device__ __forceinline__ void pair_rows(const WSub &ws, Cursor &cc, int c0,
     } else if ((R == 2 || layer) && CPR1) {
       kb[h] = key0 + (real ? c << lgP2 : 0);
       cs[h] = 0;
-      rok[h] = real && (unsigned)(ws.ws[1] + c - wl[1]) < (unsigned)ww[1] && (R == 2 || l0ok);
+      rok[h] = real && (unsigned)((e1b >= 0 ? e1b : ws.ws[1]) + c - wl[1]) < (unsigned)ww[1] &&
+               (R == 2 || l0ok);
     } else {
-      kb[h] = real ? (((cc.e0 - s0) * Em1 + cc.e1) << lgP2) + ws.ws[2] + 16 * cc.cs : key0;
+      const int row = R == 3 ? (cc.e0 - s0) * Em1 + cc.e1 : cc.e1 - (e1b >= 0 ? s0 : 0);
+      kb[h] = real ? (row << lgP2) + ws.ws[2] + 16 * cc.cs : key0;
       cs[h] = cc.cs;
       bool ok = real;
       if (R > 1) ok = ok && (unsigned)(cc.e1 - wl[1]) < (unsigned)ww[1];
@@ -553,6 +567,8 @@ __global__ void __launch_bounds__(512)
   constexpr int NT = D / 32;
   constexpr int NDB = D / 16;
   constexpr int RSE = lds_row(D);
+  constexpr bool SLAB2 = R == 2 && PFS;      // slabs of box rows
+  constexpr int SX = R == 2 ? 1 : 0;         // the slabs' axis
   extern __shared__ __align__(16) char smem[];
 
   const uint32_t tile = (uint32_t)xcd_tile(blockIdx.x, P.n_launch);
@@ -635,8 +651,8 @@ __global__ void __launch_bounds__(512)
     }
     // the K / V box in slabs of P.sl layers along axis 0 (rank 3); a single
     // slab is staged once for every query head of the group
-    const int nsl = R == 3 ? (t.E[0] + P.sl - 1) / P.sl : 1;
-    const int rows1 = R > 1 ? ws.we[1] - ws.ws[1] : 1;
+    const int nsl = R == 3 || SLAB2 ? (t.E[SX] + P.sl - 1) / P.sl : 1;
+    const int rows1 = R > 1 && !SLAB2 ? ws.we[1] - ws.ws[1] : 1;
     SlabPrefetch<T, D, R> pf;
     if constexpr (PFS) {
       pf.load(P, t, k, v, tid, nthr, 0);
@@ -691,21 +707,22 @@ __global__ void __launch_bounds__(512)
       }
       if (!ws.any) continue;
       if (si == 0) delta = quad_sum(dsum) - dl;
-      const int a0 = R == 3 ? max(ws.ws[0], s0) : 0;
-      const int b0 = R == 3 ? min(ws.we[0], s0 + P.sl) : 1;
+      const int a0 = R == 3 || SLAB2 ? max(ws.ws[SX], s0) : 0;
+      const int b0 = R == 3 || SLAB2 ? min(ws.we[SX], s0 + P.sl) : 1;
       const int nchb = b0 > a0 ? (b0 - a0) * rows1 * ws.cpr : 0;
       const int nch = nchb + (si == nsl - 1 ? nxc : 0);
-      const int key0 = (((a0 - s0) * Em1 + ws.ws[1]) << P.lgP2) + ws.ws[2];
+      const int key0 = SLAB2 ? ((a0 - s0) << P.lgP2) + ws.ws[2]
+                             : (((a0 - s0) * Em1 + ws.ws[1]) << P.lgP2) + ws.ws[2];
       // a slab of one layer (rank 3, CPR1: launched only with one-layer
       // slabs): its chunks are the rows of layer a0
       constexpr bool layer = R == 3 && CPR1;
       const bool l0ok = (unsigned)(a0 - wl[0]) < (unsigned)ww[0];
-      Cursor cc{a0, ws.ws[1], 0};
+      Cursor cc{a0, SLAB2 ? a0 : ws.ws[1], 0};
       for (int c0 = 0; c0 < nch; c0 += 2) {
         int kb[2], cs[2];
         bool rok[2];
         pair_rows<R, CPR1>(ws, cc, c0, nchb, s0, Em1, P.lgP2, key0, wl, ww, kb, rok, cs,
-                           layer, l0ok);
+                           layer, l0ok, SLAB2 ? a0 : -1);
         bool ext[2] = {false, false};
         if (VX) {
 #pragma unroll
@@ -738,7 +755,7 @@ __global__ void __launch_bounds__(512)
             kt[db] = __builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7);
           }
         };
-        constexpr bool EARLY_KT = D == 32 || R != 1;
+        constexpr bool EARLY_KT = D == 32 || (R != 1 && D < 128);
         if (EARLY_KT) read_kt();
         __builtin_amdgcn_sched_barrier(0);  // keep every read of the pair ahead
         // S^T masked through its initial value, dP^T - delta through its
@@ -840,15 +857,15 @@ __global__ void __launch_bounds__(512)
     adv[j] = zero4();
   }
   const int qbase0 = t.kbase;  // query box rows of head hk * rep
-  const int nsl = R == 3 ? (t.E[0] + P.sl - 1) / P.sl : 1;
-  const int rows1 = R > 1 ? ws.we[1] - ws.ws[1] : 1;
-  // rank 1 and 2 (without the slab prefetch): each query box's first round
+  const int nsl = R == 3 || SLAB2 ? (t.E[SX] + P.sl - 1) / P.sl : 1;
+  const int rows1 = R > 1 && !SLAB2 ? ws.we[1] - ws.ws[1] : 1;
+  // rank 1 and 2: each query box's (or slab's) first round
   // (three units per lane, two for the wider rank-1 heads) is loaded before
   // the barrier that ends the reads of the LDS it replaces (the dQ half's
   // K/V box, or the previous query head's box), so a wave that is done
   // with its chunks has those loads in flight while the others finish
   // (rank 3 keeps its registers for the slabs)
-  constexpr bool PRE = R <= 2 && !PFS;
+  constexpr bool PRE = R <= 2;
   typedef QboxRound<T, D, R, (R == 1 && D >= 64 ? 2 : 3)> QP;
   for (int hr = 0; hr < P.rep; ++hr) {
     t.kbase = qbase0 + hr * D;  // query head hk * rep + hr
@@ -867,18 +884,19 @@ __global__ void __launch_bounds__(512)
     }
     __syncthreads();
     if (!ws.any) continue;
-    const int a0 = R == 3 ? max(ws.ws[0], s0) : 0;
-    const int b0 = R == 3 ? min(ws.we[0], s0 + P.sl) : 1;
+    const int a0 = R == 3 || SLAB2 ? max(ws.ws[SX], s0) : 0;
+    const int b0 = R == 3 || SLAB2 ? min(ws.we[SX], s0 + P.sl) : 1;
     const int nch = b0 > a0 ? (b0 - a0) * rows1 * ws.cpr : 0;
-    const int key0 = (((a0 - s0) * Em1 + ws.ws[1]) << P.lgP2) + ws.ws[2];
+    const int key0 = SLAB2 ? ((a0 - s0) << P.lgP2) + ws.ws[2]
+                             : (((a0 - s0) * Em1 + ws.ws[1]) << P.lgP2) + ws.ws[2];
     constexpr bool layer = R == 3 && CPR1;
     const bool l0ok = (unsigned)(a0 - wl[0]) < (unsigned)ww[0];
-    Cursor cc{a0, ws.ws[1], 0};
+    Cursor cc{a0, SLAB2 ? a0 : ws.ws[1], 0};
     for (int c0 = 0; c0 < nch; c0 += 2) {
       int kb[2], cs[2];
       bool rok[2];
       pair_rows<R, CPR1>(ws, cc, c0, nch, s0, Em1, P.lgP2, key0, wl, ww, kb, rok, cs,
-                         layer, l0ok);
+                         layer, l0ok, SLAB2 ? a0 : -1);
       v8 qr[2][NT], orr[2][NT];
       float ls2[2][4];
 #pragma unroll
@@ -908,7 +926,7 @@ __global__ void __launch_bounds__(512)
           qt[db] = __builtin_shufflevector(q0, q1, 0, 1, 2, 3, 4, 5, 6, 7);
         }
       };
-      constexpr bool EARLY_T = D == 32 || R != 1;
+      constexpr bool EARLY_T = D == 32 || (R != 1 && D < 128);
       if (EARLY_T) read_t();
       __builtin_amdgcn_sched_barrier(0);  // keep every read of the pair ahead
       // S masked through its initial value, dP - delta through its
@@ -1047,7 +1065,8 @@ bool lean_plan(const Prob &P, int dtype, bool backward, LeanPlanInfo *o) {
     o->Em[a] = C.Em[a];
   }
   o->W = C.W;
-  o->slabs = (C.Em[0] + C.sl - 1) / C.sl;
+  const int sx = slab_axis(P.rank);
+  o->slabs = (C.Em[sx] + C.sl - 1) / C.sl;
   o->hl = L.hl;
   o->workgroups = L.n_tiles;
   o->lds = (int)lean_lds_bytes(P, mode, L.ebox, C.W);
@@ -1071,6 +1090,7 @@ void lean_fwd(const Prob &P, int dtype, const void *q, const void *k,
   const bool pfs = P.rank == 3 && !vx && (C.Em[0] + C.sl - 1) / C.sl > 1 && !L.hl &&
                    (int64_t)L.ebox * (P.D / 8) <= (int64_t)8 * 64 * C.W &&
                    3 * lds_f > (size_t)160 * 1024 && C.W <= 4 && !slab_prefetch_off();
+  const bool slab2 = P.rank == 2 && C.sl < C.Em[1];
   const size_t lds = lean_lds_bytes(P, kLFwd, L.ebox, C.W);
   const dim3 grid(L.n_launch), block(64 * C.W);
 #define LF_LAUNCH2(TT, DD, RR, CC, VV, AA, PP)                                  \
@@ -1082,6 +1102,9 @@ void lean_fwd(const Prob &P, int dtype, const void *q, const void *k,
     if (RR == 3 && !VV && pfs) {                                              \
       if (ca) LF_LAUNCH2(TT, DD, RR, CC, VV, true, (RR == 3 && !VV));         \
       else LF_LAUNCH2(TT, DD, RR, CC, VV, false, (RR == 3 && !VV));           \
+    } else if (RR == 2 && CC && !VV && slab2) {                               \
+      if (ca) LF_LAUNCH2(TT, DD, RR, CC, VV, true, (RR == 2 && CC && !VV));   \
+      else LF_LAUNCH2(TT, DD, RR, CC, VV, false, (RR == 2 && CC && !VV));     \
     } else {                                                                  \
       if (ca) LF_LAUNCH2(TT, DD, RR, CC, VV, true, false);                    \
       else LF_LAUNCH2(TT, DD, RR, CC, VV, false, false);                      \
@@ -1130,6 +1153,7 @@ void lean_bwd(const Prob &P, int dtype, const void *q, const void *k,
   const bool pfs = P.rank == 3 && !vx && (C.Em[0] + C.sl - 1) / C.sl > 1 &&
                    (int64_t)L.ebox * (P.D / 8) <= (int64_t)8 * 64 * C.W &&
                    3 * lds > (size_t)160 * 1024 && C.W <= 4 && !slab_prefetch_off();
+  const bool slab2 = P.rank == 2 && C.sl < C.Em[1];
 #define LB_LAUNCH2(TT, DD, RR, CC, VV, AA, PP)                                  \
   hipLaunchKernelGGL((k_wbwd<TT, DD, RR, CC, VV, AA, PP>), grid, block, lds, st, L, \
                      (const TT *)q, (const TT *)k, (const TT *)v,              \
@@ -1140,6 +1164,9 @@ void lean_bwd(const Prob &P, int dtype, const void *q, const void *k,
     if (RR == 3 && !VV && pfs) {                                              \
       if (ca) LB_LAUNCH2(TT, DD, RR, CC, VV, true, (RR == 3 && !VV));         \
       else LB_LAUNCH2(TT, DD, RR, CC, VV, false, (RR == 3 && !VV));           \
+    } else if (RR == 2 && !VV && slab2) {                                     \
+      if (ca) LB_LAUNCH2(TT, DD, RR, CC, VV, true, (RR == 2 && !VV));         \
+      else LB_LAUNCH2(TT, DD, RR, CC, VV, false, (RR == 2 && !VV));           \
     } else {                                                                  \
       if (ca) LB_LAUNCH2(TT, DD, RR, CC, VV, true, false);                    \
       else LB_LAUNCH2(TT, DD, RR, CC, VV, false, false);                      \

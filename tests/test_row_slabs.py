@@ -1,0 +1,73 @@
+"""Rank-2 lean kernels whose box is staged a few rows at a time: the plan (CPU),
+and forward + LSE + backward against the oracle at the edges of slabs, tiles and
+images (MI355X)."""
+
+import pytest
+import torch
+
+from _helpers import DEV, assert_close, randn
+from oracle import na as O
+
+F16, BF16 = torch.float16, torch.bfloat16
+
+
+def _plan(B, sp, H, Hkv, D, ks, dil, caus, dtype, backward):
+    from natten_amd._core import hip
+
+    q = torch.empty((B, *sp, H, D), dtype=dtype, device="meta")
+    k = torch.empty((B, *sp, Hkv, D), dtype=dtype, device="meta")
+    return hip.kernel_plan(q, k, ks, (1, 1), dil, caus, backward=backward)
+
+
+def test_large_images_and_sequences_run_lean():
+    """The 24-bit stride limit is on the axes a problem has, not on the unit
+    axes before them."""
+    for sp, H, D, ks in (((384, 384), 8, 64, (7, 7)), ((256, 256), 16, 64, (7, 7)),
+                         ((65536,), 16, 64, (63,))):
+        from natten_amd._core import hip
+
+        q = torch.empty((1, *sp, H, D), dtype=F16, device="meta")
+        one, no = (1,) * len(sp), (False,) * len(sp)
+        for backward in (False, True):
+            assert hip.kernel_path(q, q, ks, one, one, no, backward=backward) == "lean"
+
+
+# (dtype, B, spatial, H, Hkv, D, kernel, dilation, causal)
+CASES = [
+    (F16, 1, (20, 19), 2, 1, 64, (13, 13), (1, 1), (False, False)),   # two-chunk inverse rows
+    (F16, 1, (33, 17), 1, 1, 64, (13, 9), (1, 1), (True, False)),
+    (BF16, 1, (49, 56), 2, 2, 64, (11, 11), (2, 3), (False, False)),  # phases of unequal length
+    (BF16, 2, (14, 23), 2, 1, 128, (7, 7), (1, 1), (False, False)),
+    (F16, 1, (19, 16), 4, 1, 128, (5, 7), (1, 1), (False, True)),     # four heads per box
+    (F16, 1, (9, 13), 1, 1, 128, (9, 13), (1, 1), (False, True)),     # window = image
+    (BF16, 1, (18, 35), 1, 1, 128, (13, 13), (1, 1), (False, False)),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=[f"{c[2]}-d{c[5]}-k{c[6]}" for c in CASES])
+def test_planned_in_row_slabs(case):
+    p = _plan(*case[1:], case[0], True)
+    assert p["path"] == "lean" and p["slabs"] > 1, p
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES, ids=[f"{c[2]}-d{c[5]}-k{c[6]}" for c in CASES])
+def test_row_slabs_against_oracle(case):
+    import natten_amd
+
+    dtype, B, sp, H, Hkv, D, ks, dil, caus = case
+    print(f"[case] row slabs {case}", flush=True)
+    q, k, v = (randn((B, *sp, h, D), dtype, i) for i, h in enumerate((H, Hkv, Hkv)))
+    ts = [t.to(DEV).requires_grad_(True) for t in (q, k, v)]
+    out, lse = natten_amd.na2d(*ts, ks, 1, dil, caus, return_lse=True)
+
+    def f(a, b, c):
+        return O.na_functional(a, b, c, ks, 1, dil, caus, return_lse=True)
+
+    ro, rl = f(q, k, v)
+    assert_close(out, ro, dtype, "out")
+    assert_close(lse, rl, dtype, "lse")
+    go, gl = randn(out.shape, dtype, 7), randn(lse.shape, dtype, 8)
+    torch.autograd.backward((out, lse), (go.to(DEV), gl.to(DEV)))
+    for t, r, n in zip(ts, O.grads(f, (q, k, v), (go, gl)), ("dq", "dk", "dv")):
+        assert_close(t.grad, r, dtype, n)
