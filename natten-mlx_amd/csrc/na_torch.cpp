@@ -1,13 +1,18 @@
-// The fused op as a torch custom operator with its autograd node in C++
-// (natten_amd::na_fused), over the C ABI of libnatten_amd.so.
+// The differentiable ops as torch custom operators with their autograd nodes
+// in C++ over the C ABI of libnatten_amd.so: the fused op (natten_amd::na_fused),
+// the split ops (na_split_qk, na_split_av) and the DiNAT ops (na_rpb_qk,
+// na_rpb_av).
 //
 // The reference's autograd layer (autograd/na1d.py:34-53, na2d.py:34-64,
 // na3d.py) wraps the fused forward / backward in an mx.custom_function; the
-// Python twin here is autograd/fused.py's _FusedNA.  This node does the same
-// work without Python in the backward and without ctypes marshalling in
+// Python twins here are autograd/fused.py's _FusedNA, autograd/split.py's and
+// autograd/allin1.py's Functions.  These nodes do the same work without Python in the backward and without ctypes marshalling in
 // either direction: an eager training step is host-bound (the config-2
 // kernels take ~21 us per step, the host path several times that), so the
-// per-call host cost is what a caller who does not capture graphs sees.
+// per-call host cost is what a caller who does not capture graphs sees.  A split
+// or DiNAT step has two nodes each way: eager, against the Python Functions over
+// ctypes, split [4, 56, 56, 4, 32] K = 7 186 -> 107 us, DiNAT [8, 2048, 12, 12]
+// K = 7 188 -> 116 us (66 and 57 us of them on the GPU).
 //
 // Built with the host compiler against torch's headers only (no HIP
 // headers): the caller passes torch's current stream handle, and the
@@ -19,6 +24,7 @@
 #include <torch/library.h>
 
 #include <cstdint>
+#include <cstring>
 #include <vector>
 
 #include "natten_amd.h"
@@ -96,6 +102,25 @@ na_params make_params(const at::Tensor &q, const at::Tensor &k, at::IntArrayRef 
   return p;
 }
 
+// A node's parameters as one saved value: the parameter block's bytes in
+// 64-bit words, then `more`.  No device pointer is kept in it.
+template <typename P>
+std::vector<int64_t> pack(const P &p, std::initializer_list<int64_t> more) {
+  std::vector<int64_t> v((sizeof(P) + 7) / 8);
+  std::memcpy(v.data(), &p, sizeof(P));
+  v.insert(v.end(), more);
+  return v;
+}
+template <typename P>
+P unpack(const std::vector<int64_t> &v, const int64_t **more) {
+  P p;
+  std::memcpy(&p, v.data(), sizeof(P));
+  *more = v.data() + (sizeof(P) + 7) / 8;
+  return p;
+}
+
+void *as_stream(int64_t s) { return reinterpret_cast<void *>(s); }
+
 at::Tensor contig(const at::Tensor &t) { return t.defined() ? t.contiguous() : t; }
 
 struct FusedNA : public torch::autograd::Function<FusedNA> {
@@ -156,13 +181,9 @@ struct FusedNA : public torch::autograd::Function<FusedNA> {
                     reinterpret_cast<void *>(stream)),
              "na_fwd");
     ctx->save_for_backward({q, k, v, extra_k, extra_v, out, lse, sample_extent});
-    ctx->saved_data["kernel"] = kernel;
-    ctx->saved_data["stride"] = stride;
-    ctx->saved_data["dilation"] = dilation;
-    ctx->saved_data["causal"] = causal;
-    ctx->saved_data["scale"] = scale;
-    ctx->saved_data["flags"] = flags;
-    ctx->saved_data["stream"] = stream;
+    na_params saved = p;
+    saved.sample_extent = nullptr;  // read from the saved tensor again
+    ctx->saved_data["p"] = pack(saved, {stream});
     // lse is differentiable too: its gradient enters the backward as
     // delta - dlse
     ctx->set_materialize_grads(false);
@@ -181,16 +202,12 @@ struct FusedNA : public torch::autograd::Function<FusedNA> {
       glse = glse.contiguous();
       if (glse.scalar_type() != at::kFloat) glse = glse.to(at::kFloat);
     }
-    const auto kernel = ctx->saved_data["kernel"].toIntVector();
-    const auto stride = ctx->saved_data["stride"].toIntVector();
-    const auto dilation = ctx->saved_data["dilation"].toIntVector();
-    const auto causal = ctx->saved_data["causal"].toIntVector();
-    const double scale = ctx->saved_data["scale"].toDouble();
-    const int64_t flags = ctx->saved_data["flags"].toInt();
-    void *stream = reinterpret_cast<void *>(ctx->saved_data["stream"].toInt());
-    const int64_t n_extra = extra_k.defined() ? extra_k.size(1) : 0;
-    const na_params p = make_params(q, k, kernel, stride, dilation, causal, scale, n_extra, flags,
-                                    sample_extent);
+    const std::vector<int64_t> packed = ctx->saved_data["p"].toIntVector();
+    const int64_t *more;
+    na_params p = unpack<na_params>(packed, &more);
+    p.sample_extent = static_cast<const int32_t *>(cptr(sample_extent));
+    void *stream = as_stream(more[0]);
+    const int64_t n_extra = p.n_extra;
     const size_t ws_bytes = na_bwd_workspace_bytes(&p);
     at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
     at::Tensor dek = n_extra ? at::empty_like(extra_k) : at::Tensor();
@@ -224,6 +241,245 @@ std::tuple<at::Tensor, at::Tensor> na_fused(const at::Tensor &q, const at::Tenso
   return {r[0], r[1]};
 }
 
+// ---- split ops (autograd/split.py) ----------------------------------------
+// The caller has validated shapes (functional.py) and passes tensors of
+// supported dtypes on one device.
+
+std::vector<int64_t> split_sizes(const at::Tensor &x, at::IntArrayRef stride, int64_t last) {
+  std::vector<int64_t> sz(x.sizes().begin(), x.sizes().end());
+  for (size_t a = 0; a < stride.size(); ++a) sz[1 + a] = (sz[1 + a] + stride[a] - 1) / stride[a];
+  sz.back() = last;
+  return sz;
+}
+
+int64_t product(at::IntArrayRef v) {
+  int64_t n = 1;
+  for (const int64_t x : v) n *= x;
+  return n;
+}
+
+at::Tensor to_type(const at::Tensor &t, at::ScalarType s) {
+  return t.scalar_type() == s ? t : t.to(s);
+}
+
+struct SplitQK : public torch::autograd::Function<SplitQK> {
+  static at::Tensor forward(AutogradContext *ctx, at::Tensor q, at::Tensor k,
+                            at::IntArrayRef kernel, at::IntArrayRef stride,
+                            at::IntArrayRef dilation, at::IntArrayRef causal, double scale,
+                            int64_t flags, int64_t stream) {
+    check_device(q);
+    check_device(k);
+    const auto kd = k.scalar_type();
+    q = q.contiguous();
+    k = to_type(k, q.scalar_type()).contiguous();
+    const na_params p =
+        make_params(q, k, kernel, stride, dilation, causal, scale, 0, flags, at::Tensor());
+    at::Tensor logits = at::empty(split_sizes(q, stride, product(kernel)), q.options());
+    check_rc(na_qk_fwd(&p, q.data_ptr(), k.data_ptr(), logits.data_ptr(), as_stream(stream)),
+             "na_qk_fwd");
+    ctx->save_for_backward({q, k});
+    ctx->saved_data["p"] = pack(p, {stream, (int64_t)kd});
+    return logits;
+  }
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const at::Tensor &q = s[0], &k = s[1];
+    const std::vector<int64_t> packed = ctx->saved_data["p"].toIntVector();
+    const int64_t *more;
+    const na_params p = unpack<na_params>(packed, &more);
+    const at::Tensor g = to_type(grads[0], q.scalar_type()).contiguous();
+    at::Tensor dq = at::empty_like(q), dk = at::empty_like(k);
+    check_rc(na_qk_bwd(&p, q.data_ptr(), k.data_ptr(), g.data_ptr(), dq.data_ptr(),
+                       dk.data_ptr(), as_stream(more[0])),
+             "na_qk_bwd");
+    const at::Tensor none;
+    return {dq, to_type(dk, (at::ScalarType)more[1]), none, none, none, none, none, none, none};
+  }
+};
+
+struct SplitAV : public torch::autograd::Function<SplitAV> {
+  static at::Tensor forward(AutogradContext *ctx, at::Tensor attn, at::Tensor v,
+                            at::IntArrayRef kernel, at::IntArrayRef stride,
+                            at::IntArrayRef dilation, at::IntArrayRef causal, int64_t stream) {
+    check_device(attn);
+    check_device(v);
+    const auto ad = attn.scalar_type(), vd = v.scalar_type();
+    const auto dt = at::promote_types(ad, vd);
+    attn = to_type(attn, dt).contiguous();
+    v = to_type(v, dt).contiguous();
+    na_params p = make_params(v, v, kernel, stride, dilation, causal, 1.0, 0, 0, at::Tensor());
+    p.heads = (int32_t)attn.size(-2);
+    std::vector<int64_t> osz(attn.sizes().begin(), attn.sizes().end());
+    osz.back() = v.size(-1);
+    at::Tensor out = at::empty(osz, v.options());
+    check_rc(na_av_fwd(&p, attn.data_ptr(), v.data_ptr(), out.data_ptr(), as_stream(stream)),
+             "na_av_fwd");
+    ctx->save_for_backward({attn, v});
+    ctx->saved_data["p"] = pack(p, {stream, (int64_t)ad, (int64_t)vd});
+    return out;
+  }
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const at::Tensor &attn = s[0], &v = s[1];
+    const std::vector<int64_t> packed = ctx->saved_data["p"].toIntVector();
+    const int64_t *more;
+    const na_params p = unpack<na_params>(packed, &more);
+    const at::Tensor g = to_type(grads[0], v.scalar_type()).contiguous();
+    at::Tensor dattn = at::empty_like(attn), dv = at::empty_like(v);
+    check_rc(na_av_bwd(&p, attn.data_ptr(), v.data_ptr(), g.data_ptr(), dattn.data_ptr(),
+                       dv.data_ptr(), as_stream(more[0])),
+             "na_av_bwd");
+    const at::Tensor none;
+    return {to_type(dattn, (at::ScalarType)more[1]), to_type(dv, (at::ScalarType)more[2]),
+            none, none, none, none, none};
+  }
+};
+
+// ---- DiNAT ops (autograd/allin1.py) ----------------------------------------
+
+na_rpb_params make_rpb(const at::Tensor &x, at::IntArrayRef kernel, at::IntArrayRef dilation,
+                       double scale, bool has_scale, bool heads_first) {
+  const int64_t rank = x.dim() - 3;
+  TORCH_CHECK((rank == 1 || rank == 2) && (int64_t)kernel.size() == rank &&
+                  (int64_t)dilation.size() == rank,
+              "natten_amd: a rank-1 or rank-2 tensor with one kernel and dilation per axis");
+  na_rpb_params p{};
+  p.rank = (int32_t)rank;
+  p.batch = (int32_t)x.size(0);
+  p.heads = (int32_t)x.size(heads_first ? 1 : -2);
+  p.head_dim = (int32_t)x.size(-1);
+  for (int a = 0; a < 2; ++a) {
+    p.extent[a] = a < rank ? (int32_t)x.size((heads_first ? 2 : 1) + a) : 1;
+    p.kernel[a] = a < rank ? (int32_t)kernel[a] : 1;
+    p.dilation[a] = a < rank ? (int32_t)dilation[a] : 1;
+  }
+  p.heads_first = heads_first ? 1 : 0;
+  p.dtype = dtype_code(x.scalar_type());
+  p.scale = has_scale ? (float)scale : 1.f;
+  p.has_scale = has_scale ? 1 : 0;
+  return p;
+}
+
+at::Tensor f32(const at::Tensor &t) { return to_type(t, at::kFloat).contiguous(); }
+
+struct RpbQK : public torch::autograd::Function<RpbQK> {
+  // rpb: float [H, 2K-1] (rank 2: [H, 2K0-1, 2K1-1]) or absent, checked by
+  // the caller, as q's and k's equal shapes are
+  static at::Tensor forward(AutogradContext *ctx, at::Tensor q, at::Tensor k,
+                            std::optional<at::Tensor> rpb_opt, at::IntArrayRef kernel,
+                            at::IntArrayRef dilation, double scale, bool has_scale,
+                            bool heads_first, int64_t stream) {
+    const at::Tensor rpb = rpb_opt.value_or(at::Tensor());
+    for (const at::Tensor *t : std::initializer_list<const at::Tensor *>{&q, &k, &rpb})
+      check_device(*t);
+    const auto kd = k.scalar_type();
+    q = q.contiguous();
+    k = to_type(k, q.scalar_type()).contiguous();
+    const na_rpb_params p = make_rpb(q, kernel, dilation, scale, has_scale, heads_first);
+    const at::Tensor bias = rpb.defined() ? f32(rpb) : rpb;
+    std::vector<int64_t> osz(q.sizes().begin(), q.sizes().end());
+    osz.back() = product(kernel);
+    at::Tensor out = at::empty(osz, q.options().dtype(at::kFloat));
+    check_rc(na_rpb_qk_fwd(&p, q.data_ptr(), k.data_ptr(), static_cast<const float *>(cptr(bias)),
+                           static_cast<float *>(out.data_ptr()), as_stream(stream)),
+             "na_rpb_qk_fwd");
+    ctx->save_for_backward({q, k});
+    ctx->saved_data["p"] = pack(
+        p, {stream, (int64_t)kd, rpb.defined() ? (int64_t)rpb.scalar_type() : (int64_t)-1});
+    return out;
+  }
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const at::Tensor &q = s[0], &k = s[1];
+    const std::vector<int64_t> packed = ctx->saved_data["p"].toIntVector();
+    const int64_t *more;
+    const na_rpb_params p = unpack<na_rpb_params>(packed, &more);
+    const bool has_rpb = more[2] >= 0;
+    const at::Tensor g = f32(grads[0]);
+    at::Tensor dq, dk, drpb, ws;
+    if (ctx->needs_input_grad(0)) dq = at::empty_like(q);
+    if (ctx->needs_input_grad(1)) dk = at::empty_like(k);
+    size_t ws_bytes = 0;
+    if (has_rpb && ctx->needs_input_grad(2)) {
+      std::vector<int64_t> bsz{p.heads};
+      for (int a = 0; a < p.rank; ++a) bsz.push_back(2 * p.kernel[a] - 1);
+      drpb = at::empty(bsz, q.options().dtype(at::kFloat));
+      ws_bytes = na_rpb_bwd_workspace_bytes(&p);
+      ws = at::empty({(int64_t)std::max<size_t>(ws_bytes, 1)}, q.options().dtype(at::kByte));
+    }
+    check_rc(na_rpb_qk_bwd(&p, q.data_ptr(), k.data_ptr(), static_cast<const float *>(g.data_ptr()),
+                           mptr(dq), mptr(dk), static_cast<float *>(mptr(drpb)), mptr(ws),
+                           ws_bytes, as_stream(more[0])),
+             "na_rpb_qk_bwd");
+    if (dk.defined()) dk = to_type(dk, (at::ScalarType)more[1]);
+    if (drpb.defined()) drpb = to_type(drpb, (at::ScalarType)more[2]);
+    const at::Tensor none;
+    return {dq, dk, drpb, none, none, none, none, none, none};
+  }
+};
+
+struct RpbAV : public torch::autograd::Function<RpbAV> {
+  // out_f32: the output (and its gradient) is float32, else v's dtype
+  static at::Tensor forward(AutogradContext *ctx, at::Tensor attn, at::Tensor v,
+                            at::IntArrayRef kernel, at::IntArrayRef dilation, bool heads_first,
+                            bool out_f32, int64_t stream) {
+    check_device(attn);
+    check_device(v);
+    const auto ad = attn.scalar_type();
+    v = v.contiguous();
+    attn = f32(attn);
+    const na_rpb_params p = make_rpb(v, kernel, dilation, 1.0, false, heads_first);
+    at::Tensor out =
+        at::empty(v.sizes(), out_f32 ? v.options().dtype(at::kFloat) : v.options());
+    check_rc(na_rpb_av_fwd(&p, static_cast<const float *>(attn.data_ptr()), v.data_ptr(),
+                           out.data_ptr(), dtype_code(out.scalar_type()), as_stream(stream)),
+             "na_rpb_av_fwd");
+    ctx->save_for_backward({attn, v});
+    ctx->saved_data["p"] = pack(p, {stream, (int64_t)ad});
+    return out;
+  }
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const at::Tensor &attn = s[0], &v = s[1];
+    const std::vector<int64_t> packed = ctx->saved_data["p"].toIntVector();
+    const int64_t *more;
+    const na_rpb_params p = unpack<na_rpb_params>(packed, &more);
+    at::Tensor g = grads[0];
+    if (g.scalar_type() != at::kFloat && g.scalar_type() != v.scalar_type()) g = g.to(at::kFloat);
+    g = g.contiguous();
+    at::Tensor dattn, dv;
+    if (ctx->needs_input_grad(0)) dattn = at::empty_like(attn);
+    if (ctx->needs_input_grad(1)) dv = at::empty_like(v);
+    check_rc(na_rpb_av_bwd(&p, static_cast<const float *>(attn.data_ptr()), v.data_ptr(),
+                           g.data_ptr(), dtype_code(g.scalar_type()),
+                           static_cast<float *>(mptr(dattn)), mptr(dv), as_stream(more[0])),
+             "na_rpb_av_bwd");
+    if (dattn.defined()) dattn = to_type(dattn, (at::ScalarType)more[1]);
+    const at::Tensor none;
+    return {dattn, dv, none, none, none, none, none};
+  }
+};
+
+at::Tensor na_split_qk(const at::Tensor &q, const at::Tensor &k, at::IntArrayRef kernel,
+                       at::IntArrayRef stride, at::IntArrayRef dilation, at::IntArrayRef causal,
+                       double scale, int64_t flags, int64_t stream) {
+  return SplitQK::apply(q, k, kernel, stride, dilation, causal, scale, flags, stream);
+}
+at::Tensor na_split_av(const at::Tensor &attn, const at::Tensor &v, at::IntArrayRef kernel,
+                       at::IntArrayRef stride, at::IntArrayRef dilation, at::IntArrayRef causal,
+                       int64_t stream) {
+  return SplitAV::apply(attn, v, kernel, stride, dilation, causal, stream);
+}
+at::Tensor na_rpb_qk(const at::Tensor &q, const at::Tensor &k, const std::optional<at::Tensor> &rpb,
+                     at::IntArrayRef kernel, at::IntArrayRef dilation, double scale,
+                     bool has_scale, bool heads_first, int64_t stream) {
+  return RpbQK::apply(q, k, rpb, kernel, dilation, scale, has_scale, heads_first, stream);
+}
+at::Tensor na_rpb_av(const at::Tensor &attn, const at::Tensor &v, at::IntArrayRef kernel,
+                     at::IntArrayRef dilation, bool heads_first, bool out_f32, int64_t stream) {
+  return RpbAV::apply(attn, v, kernel, dilation, heads_first, out_f32, stream);
+}
+
 }  // namespace
 
 TORCH_LIBRARY(natten_amd, m) {
@@ -231,6 +487,24 @@ TORCH_LIBRARY(natten_amd, m) {
       "na_fused(Tensor q, Tensor k, Tensor v, Tensor? extra_k, Tensor? extra_v, "
       "Tensor? sample_extent, int[] kernel, int[] stride, int[] dilation, int[] causal, "
       "float scale, int flags, int stream) -> (Tensor, Tensor)");
+  m.def(
+      "na_split_qk(Tensor q, Tensor k, int[] kernel, int[] stride, int[] dilation, "
+      "int[] causal, float scale, int flags, int stream) -> Tensor");
+  m.def(
+      "na_split_av(Tensor attn, Tensor v, int[] kernel, int[] stride, int[] dilation, "
+      "int[] causal, int stream) -> Tensor");
+  m.def(
+      "na_rpb_qk(Tensor q, Tensor k, Tensor? rpb, int[] kernel, int[] dilation, float scale, "
+      "bool has_scale, bool heads_first, int stream) -> Tensor");
+  m.def(
+      "na_rpb_av(Tensor attn, Tensor v, int[] kernel, int[] dilation, bool heads_first, "
+      "bool out_f32, int stream) -> Tensor");
 }
 
-TORCH_LIBRARY_IMPL(natten_amd, CompositeImplicitAutograd, m) { m.impl("na_fused", na_fused); }
+TORCH_LIBRARY_IMPL(natten_amd, CompositeImplicitAutograd, m) {
+  m.impl("na_fused", na_fused);
+  m.impl("na_split_qk", na_split_qk);
+  m.impl("na_split_av", na_split_av);
+  m.impl("na_rpb_qk", na_rpb_qk);
+  m.impl("na_rpb_av", na_rpb_av);
+}

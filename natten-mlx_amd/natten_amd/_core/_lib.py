@@ -163,6 +163,7 @@ _lib = None
 _lock = threading.Lock()
 _load_error: str | None = None
 _fused_op = None
+_node_ops = None
 
 
 def load():
@@ -190,14 +191,17 @@ def load():
 
 
 def _load_fused_op() -> None:
-    """Register natten_amd::na_fused from libnatten_amd_torch.so (built
-    beside the library; it links this library, which the loader then shares
-    with the ctypes handle)."""
-    global _fused_op
+    """Register the operators of libnatten_amd_torch.so (built beside the
+    library; it links this library, which the loader then shares with the
+    ctypes handle)."""
+    global _fused_op, _node_ops
     if not os.path.exists(OP_LIB_PATH):
         return
     torch.ops.load_library(OP_LIB_PATH)
-    _fused_op = torch.ops.natten_amd.na_fused
+    ns = torch.ops.natten_amd
+    _fused_op = ns.na_fused.default
+    _node_ops = {"qk": ns.na_split_qk.default, "av": ns.na_split_av.default,
+                 "rpb_qk": ns.na_rpb_qk.default, "rpb_av": ns.na_rpb_av.default}
 
 
 def fused_op():
@@ -207,6 +211,24 @@ def fused_op():
     if _lib is None:
         load()
     return _fused_op
+
+
+_OP_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
+
+
+def node_op(name: str, a: torch.Tensor, b: torch.Tensor):
+    """The C++ operator of a split ("qk", "av") or DiNAT ("rpb_qk", "rpb_av")
+    op where it takes these tensors: built, and both of a supported dtype on
+    one HIP device.  None otherwise (the Python autograd Function then runs
+    the same kernels, or raises)."""
+    if _lib is None:
+        if not a.is_cuda:
+            return None
+        load()
+    if (_node_ops is None or not a.is_cuda or a.device != b.device
+            or a.dtype not in _OP_DTYPES or b.dtype not in _OP_DTYPES):
+        return None
+    return _node_ops[name]
 
 
 def available() -> bool:

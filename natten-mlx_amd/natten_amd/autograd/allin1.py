@@ -4,14 +4,18 @@ The reference's public ``na{1,2}d_qk_rpb`` / ``na{1,2}d_av_fused`` are
 forward-only; its Metal backward lives in separate functions
 (``extras/allin1/functional_metal.py:1206-1918``: dq, dk, drpb and dattn,
 dvalue).  Here both directions are joined in ``torch.autograd.Function`` s
-whose backward calls the library's deterministic gather kernels.
+whose backward calls the library's deterministic kernels: operators with
+their nodes in C++ (``csrc/na_torch.cpp``), or the same as Python Functions
+where the operator library is not built, for arguments it does not take and
+under ``python_autograd()``.
 """
 
 from __future__ import annotations
 
 import torch
 
-from .._core import hip
+from .._core import _lib, hip
+from . import fused as _fused
 
 
 class _QKRPB(torch.autograd.Function):
@@ -53,6 +57,17 @@ class _AVRPB(torch.autograd.Function):
         return da, dv, None, None, None, None
 
 
+def _op(name, a, b, kernel_size, dilation):
+    """(operator, kernel and dilation per axis), or None."""
+    rank = a.dim() - 3
+    if _fused._py_autograd or rank not in (1, 2):
+        return None
+    op = _lib.node_op(name, a, b)
+    if op is None:
+        return None
+    return (op, hip._per_axis(kernel_size, rank), hip._per_axis(dilation, rank))
+
+
 def _axes(v):
     """An int, or a per-axis tuple of ints (non-square windows)."""
     return tuple(int(x) for x in v) if isinstance(v, (tuple, list)) else int(v)
@@ -61,6 +76,13 @@ def _axes(v):
 def qk_rpb_with_grad(q, k, rpb, kernel_size, dilation, scale=None, heads_first=False):
     """float32 logits of the fused QK + RPB op, differentiable in q, k, rpb.
     kernel_size / dilation: an int or one value per axis."""
+    op = _op("rpb_qk", q, k, kernel_size, dilation)
+    if op is not None and q.shape == k.shape:
+        heads = q.shape[1 if heads_first else -2]
+        if rpb is None or (rpb.device == q.device and rpb.is_floating_point()
+                           and tuple(rpb.shape) == (heads, *(2 * x - 1 for x in op[1]))):
+            return op[0](q, k, rpb, op[1], op[2], 0.0 if scale is None else float(scale),
+                         scale is not None, bool(heads_first), _lib.stream_of(q))
     return _QKRPB.apply(q, k, rpb, _axes(kernel_size), _axes(dilation), scale,
                         bool(heads_first))
 
@@ -68,6 +90,11 @@ def qk_rpb_with_grad(q, k, rpb, kernel_size, dilation, scale=None, heads_first=F
 def av_rpb_with_grad(attn, v, kernel_size, dilation, heads_first=False,
                      out_dtype=torch.float32):
     """AV op output, differentiable in attn and v."""
+    op = _op("rpb_av", v, attn, kernel_size, dilation)
+    if (op is not None and out_dtype in (torch.float32, v.dtype)
+            and tuple(attn.shape) == hip._slots_shape(v, op[1], heads_first)):
+        return op[0](attn, v, op[1], op[2], bool(heads_first), out_dtype == torch.float32,
+                     _lib.stream_of(v))
     return _AVRPB.apply(attn, v, _axes(kernel_size), _axes(dilation), bool(heads_first),
                         out_dtype)
 

@@ -51,6 +51,7 @@ class FusedSpec(NamedTuple):
     # every per-sample extent satisfies dilation * kernel_size <= extent on
     # each non-causal axis (checked by the caller on the host)
     varlen_clamped: bool = False
+    causal_ints: tuple = ()  # is_causal as 0 / 1, for the operator
 
 
 class _FusedNA(torch.autograd.Function):
@@ -96,7 +97,7 @@ def na_fused_with_grad(q, k, v, spec: FusedSpec, extra_k=None, extra_v=None,
         if op is not None and ops.backend_module() is _hip:
             scale = q.shape[-1] ** -0.5 if spec.scale is None else float(spec.scale)
             return op(q, k, v, extra_k, extra_v, sample_extent, spec.kernel_size, spec.stride,
-                      spec.dilation, [int(c) for c in spec.is_causal], scale,
+                      spec.dilation, spec.causal_ints or [int(c) for c in spec.is_causal], scale,
                       _op_flags(spec, sample_extent), _lib.stream_of(q))
     return _FusedNA.apply(q, k, v, extra_k, extra_v, sample_extent, spec)
 

@@ -139,7 +139,7 @@ def _fused_spec(rank, query, key, value, kernel_size, stride, dilation, is_causa
     dense = (_is_full_attention(ks, spatial_shape) and all(s == 1 for s in st)
              and not any(caus))
     return FusedSpec(tuple(ks), tuple(st), tuple(dil), tuple(bool(c) for c in caus), scale_value,
-                     dense)
+                     dense, causal_ints=tuple(int(bool(c)) for c in caus))
 
 
 def _na(rank, query, key, value, kernel_size, stride, dilation, is_causal, scale, return_lse,
@@ -222,9 +222,7 @@ def na3d(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
 # ---------------------------------------------------------------------------
 # split ops (reference functional.py:476-634)
 
-def _qk(rank, query, key, kernel_size, dilation, stride, is_causal, scale, fn):
-    _validate_qkv(query, key, key, rank)
-    spatial = tuple(query.shape[1:-2])
+def _split_spec(spatial, rank, kernel_size, dilation, stride, is_causal):
     ks = normalize_kernel_size(kernel_size, rank)
     st = normalize_tuple_param(stride, rank, "stride")
     dil = normalize_tuple_param(dilation, rank, "dilation")
@@ -232,10 +230,42 @@ def _qk(rank, query, key, kernel_size, dilation, stride, is_causal, scale, fn):
     check_kernel_size_vs_input(ks, spatial)
     check_stride_vs_kernel(st, ks)
     check_dilation_kernel_vs_input(dil, ks, spatial)
+    return tuple(ks), tuple(st), tuple(dil), tuple(bool(c) for c in caus)
+
+
+def _cached_spec(key, make):
+    """``make()``, kept by call signature as the fused op's specs are."""
+    try:
+        spec = _spec_cache.get(key)
+    except TypeError:  # an unhashable argument
+        return make()
+    if spec is None:
+        spec = make()
+        if len(_spec_cache) >= _SPEC_MAX:
+            _spec_cache.clear()
+        _spec_cache[key] = spec
+    return spec
+
+
+def _qk(rank, query, key, kernel_size, dilation, stride, is_causal, scale, fn):
+    def make():
+        _validate_qkv(query, key, key, rank)
+        return _split_spec(tuple(query.shape[1:-2]), rank, kernel_size, dilation, stride,
+                           is_causal)
+
+    ks, st, dil, caus = _cached_spec(("qk", rank, query.shape, key.shape, kernel_size, dilation,
+                                      stride, is_causal), make)
     return fn(query, key, ks, st, dil, caus, scale)
 
 
 def _av(rank, attn, value, kernel_size, dilation, stride, is_causal, fn):
+    ks, st, dil, caus = _cached_spec(
+        ("av", rank, attn.shape, value.shape, kernel_size, dilation, stride, is_causal),
+        lambda: _av_spec(rank, attn, value, kernel_size, dilation, stride, is_causal))
+    return fn(attn, value, ks, st, dil, caus)
+
+
+def _av_spec(rank, attn, value, kernel_size, dilation, stride, is_causal):
     nd = rank + 3
     if attn.ndim != nd or value.ndim != nd:
         raise ValueError(f"attn and value must be {nd}D for na{rank}d_av")
@@ -243,15 +273,7 @@ def _av(rank, attn, value, kernel_size, dilation, stride, is_causal, fn):
         raise ValueError(
             "attn and value must match batch and heads dimensions; "
             f"got {tuple(attn.shape)} and {tuple(value.shape)}")
-    spatial = tuple(value.shape[1:-2])
-    ks = normalize_kernel_size(kernel_size, rank)
-    st = normalize_tuple_param(stride, rank, "stride")
-    dil = normalize_tuple_param(dilation, rank, "dilation")
-    caus = normalize_tuple_param(is_causal, rank, "is_causal")
-    check_kernel_size_vs_input(ks, spatial)
-    check_stride_vs_kernel(st, ks)
-    check_dilation_kernel_vs_input(dil, ks, spatial)
-    return fn(attn, value, ks, st, dil, caus)
+    return _split_spec(tuple(value.shape[1:-2]), rank, kernel_size, dilation, stride, is_causal)
 
 
 def na1d_qk(query, key, kernel_size, dilation=1, *, stride=1, is_causal=False, scale=None):
