@@ -79,6 +79,8 @@ struct LProb {
   float sl2;          // scale * log2(e)
   int32_t n_tiles, n_launch;
   int32_t sa;         // stack axis: the workgroup's waves tile this axis
+  int32_t wsh;        // rank 3: wave w is the (w >> wsh)-th along axis 0 too
+                      // (8: it is not, the waves tile one axis)
   int32_t ebox;       // staged rows: Em2 (rank 1) or Em0 * Em1 * 2^lgP2
   int32_t lgP2;       // rank >= 2: staged box rows are 2^lgP2 >= Em2 wide
   int32_t rep;        // query heads per key/value head
@@ -284,7 +286,9 @@ __device__ __forceinline__ WSub wave_sub(const LProb &P, const LTile &t,
       continue;
     }
     const LAx &x = P.ax[a];
-    const int off = a == P.sa ? w * x.T : 0;
+    int off = a == P.sa ? w * x.T : 0;
+    if (R == 3)
+      off = a == P.sa ? (w & ((1 << P.wsh) - 1)) * x.T : a == 0 ? (w >> P.wsh) * x.T : 0;
     s.i0[a] = t.i0[a] + off;
     s.nv[a] = min(t.nv[a] - off, x.T);
     s.nvt[a] = min(t.nvt[a] - off, x.T);
@@ -620,6 +624,7 @@ constexpr int kLeanCUs = 256;
 struct LChoice {
   int T[3];      // wave tile (product 16 over the active axes)
   int W, sa;     // waves per workgroup and the axis they are stacked along
+  int w0;        // rank 3: of them along axis 0 besides (1: all along sa)
   int Em[3];     // workgroup key box (largest over tiles)
   int sl;        // box layers (rank 3) or rows (rank 2) staged at a time
                  // (Em of that axis: all at once)
@@ -704,6 +709,7 @@ LChoice lean_choice_compute(const Prob &P, LMode mode) {
   const int R = P.rank, lead = 3 - R;
   LChoice best{};
   best.ok = false;
+  best.w0 = 1;
   double best_cost = 1e300;
   auto ext = [&](int a, int t) {
     if (a < lead) return 1;
@@ -848,6 +854,44 @@ LChoice lean_choice_compute(const Prob &P, LMode mode) {
         }
       }
   }
+  // Rank 3 boxes beyond LDS: eight waves on several layers of queries, each
+  // layer of keys staged once for all of them (K0 = 3 causal, two layers of four
+  // waves: 4 layers for 128 queries instead of 3 for 64).  Two such workgroups
+  // give a CU 16 waves, where the prefetching form of four waves has registers
+  // for 8 (bf16, forward / backward: [1, 16, 32, 32, 8, 64] K = (3, 7, 7) causal
+  // in depth 47 -> 38 / 119 -> 98 us, [1, 24, 40, 40, 8, 64] K = (3, 5, 5) 117 ->
+  // 66 / 312 -> 190, [1, 24, 40, 40, 8, 32] K = (3, 7, 7) 94 -> 65 / 213 -> 166).
+  if (best.ok && R == 3 && (mode == kLFwd || mode == kLBwd) && best.sl < best.Em[0] &&
+      P.sample_extent == nullptr && P.n_extra == 0 && !lean_waves_forced()) {
+    double least = best_per_wave;
+    const LChoice base = best;
+    for (int w0 = 2; w0 <= 8; w0 <<= 1)
+      for (int sa = 1; sa < 3; ++sa) {
+        const int W1 = 8 / w0;
+        const int TW[3] = {base.T[0] * w0, base.T[1] * (sa == 1 ? W1 : 1),
+                           base.T[2] * (sa == 2 ? W1 : 1)};
+        int Em[3];
+        int64_t wgs = (int64_t)P.B * (mode == kLBwd ? P.Hkv : P.H);
+        bool fits = true;  // every wave tile starts inside the phase
+        for (int a = 0; a < 3; ++a) {
+          const int Lr = (P.ax[a].L + P.ax[a].d - 1) / P.ax[a].d;
+          fits = fits && TW[a] - base.T[a] < Lr;
+          wgs *= (int64_t)P.ax[a].d * ((Lr + TW[a] - 1) / TW[a]);
+          Em[a] = ext(a, TW[a]);
+        }
+        // a layer's barrier and round trip, with 16 waves to hide them
+        const double rows = (double)lds_rows(R, Em) / 8 * (1.0 + 0.15 * (Em[0] - 1));
+        if (!fits || wgs < 2 * kLeanCUs || rows >= least ||
+            lean_lds_bytes(P, mode, lds_rows(R, Em) / Em[0], 8) > lds_budget())
+          continue;
+        least = rows;
+        best.W = 8;
+        best.w0 = w0;
+        best.sa = sa;
+        best.sl = 1;
+        for (int a = 0; a < 3; ++a) best.Em[a] = Em[a];
+      }
+  }
   return best;
 }
 
@@ -900,6 +944,7 @@ LProb make_lprob(const Prob &P, const LChoice &C) {
   L.Ltot = P.ax[0].L * P.ax[1].L * P.ax[2].L;
   L.sl2 = P.scale * kLog2e;
   L.sa = C.sa;
+  L.wsh = C.w0 > 1 ? ilog2c(C.W / C.w0) : 8;
   int tok = 1;
   int grid = 1;
   for (int a = 2; a >= 0; --a) {
@@ -914,7 +959,7 @@ LProb make_lprob(const Prob &P, const LChoice &C) {
     y.Lrem = x.L % x.d;
     y.T = C.T[a];
     y.lgT = ilog2c(C.T[a]);
-    y.TW = C.T[a] * (a == C.sa ? C.W : 1);
+    y.TW = C.T[a] * (a == C.sa ? C.W / C.w0 : a == 0 ? C.w0 : 1);
     y.lgTW = ilog2c(y.TW);
     y.Em = C.Em[a];
     const int Lr = (x.L + x.d - 1) / x.d;

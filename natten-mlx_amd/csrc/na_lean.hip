@@ -383,10 +383,10 @@ __global__ void __launch_bounds__(512)
 // lanes holding one row.  load() only reads memory into registers, so a
 // wave may issue it before the barrier that ends the other waves' reads of
 // the LDS it will overwrite; store() writes the LDS.  NU: units per lane
-// in flight, by default two for the wider rank-1 heads, whose backward
-// keeps four waves per SIMD (its dK / dV accumulators and the key's own
-// rows stay live across the staging), else four.
-template <typename T, int D, int R, int NU_ = (R == 1 && D >= 64 ? 2 : 4)>
+// in flight, two for the wider heads at rank 1 (and rank 3 without the slab
+// prefetch), whose backward keeps four waves per SIMD (its dK / dV accumulators
+// and the key's own rows stay live across the staging), else four.
+template <typename T, int D, int R, int NU_>
 struct QboxRound {
   typedef typename L16<T>::v8 v8;
   typedef typename L16<T>::e E;
@@ -442,7 +442,7 @@ struct QboxRound {
 
 // Stage the dK/dV role's query box from unit u_begin on (the rounds before
 // it staged by the caller), then clear the slack rows.
-template <typename T, int D, int R>
+template <typename T, int D, int R, int NU>
 __device__ __forceinline__ void stage_qbox(const LProb &P, const LTile &t,
                                            const T *__restrict__ q,
                                            const T *__restrict__ dout,
@@ -452,7 +452,7 @@ __device__ __forceinline__ void stage_qbox(const LProb &P, const LTile &t,
                                            typename L16<T>::e *qs,
                                            typename L16<T>::e *os, int tid,
                                            int nthr, int s0, int u_begin) {
-  typedef QboxRound<T, D, R> QR;
+  typedef QboxRound<T, D, R, NU> QR;
   const int nun = P.ebox * QR::OCT;
   for (int u0 = u_begin; u0 < nun; u0 += QR::NU * nthr) {
     QR r;
@@ -551,7 +551,7 @@ __device__ __forceinline__ void pair_rows(const WSub &ws, Cursor &cc, int c0,
 // issued while the previous slab is computed (SlabPrefetch).
 template <typename T, int D, int R, bool CPR1, bool VX, bool CA, bool PFS>
 __global__ void __launch_bounds__(512)
-    __attribute__((amdgpu_waves_per_eu(D == 64 && R == 1 ? 4 : 1)))
+    __attribute__((amdgpu_waves_per_eu(D == 64 && (R == 1 || (R == 3 && !PFS)) ? 4 : 1)))
     k_wbwd(LProb Pin, const T *__restrict__ q, const T *__restrict__ k,
            const T *__restrict__ v, const T *__restrict__ ek,
            const T *__restrict__ ev, const T *__restrict__ out,
@@ -745,7 +745,9 @@ __global__ void __launch_bounds__(512)
           }
         // K^T operands of dQ^T += K^T . dS^T: read now so their latency
         // overlaps the score MFMAs and exponentials, or after the scores
-        // for the wider rank-1 heads (as in the dK / dV half)
+        // for the wider heads where that leaves room for more waves (rank 1,
+        // rank 3 without and rank 2 with the slab prefetch, head_dim 128; as in
+        // the dK / dV half)
         v8 kt[NDB];
         auto read_kt = [&]() {
 #pragma unroll
@@ -755,7 +757,7 @@ __global__ void __launch_bounds__(512)
             kt[db] = __builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7);
           }
         };
-        constexpr bool EARLY_KT = D == 32 || (R != 1 && D < 128);
+        constexpr bool EARLY_KT = D == 32 || (D < 128 && (R == 2 ? !PFS : R == 3 && PFS));
         if (EARLY_KT) read_kt();
         __builtin_amdgcn_sched_barrier(0);  // keep every read of the pair ahead
         // S^T masked through its initial value, dP^T - delta through its
@@ -866,6 +868,7 @@ __global__ void __launch_bounds__(512)
   // with its chunks has those loads in flight while the others finish
   // (rank 3 keeps its registers for the slabs)
   constexpr bool PRE = R <= 2;
+  constexpr int QN = D >= 64 && (R == 1 || (R == 3 && !PFS)) ? 2 : 4;
   typedef QboxRound<T, D, R, (R == 1 && D >= 64 ? 2 : 3)> QP;
   for (int hr = 0; hr < P.rep; ++hr) {
     t.kbase = qbase0 + hr * D;  // query head hk * rep + hr
@@ -876,11 +879,11 @@ __global__ void __launch_bounds__(512)
       pre.load(P, t, q, dout, out, lse, dlse, 0, tid, nthr, s0);
       __syncthreads();
       pre.store(xs, ys, tid);
-      stage_qbox<T, D, R>(P, t, q, dout, out, lse, dlse, xs, ys, tid, nthr, s0,
+      stage_qbox<T, D, R, QN>(P, t, q, dout, out, lse, dlse, xs, ys, tid, nthr, s0,
                           QP::NU * nthr);
     } else {
       __syncthreads();  // the LDS reads of the previous box or slab are done
-      stage_qbox<T, D, R>(P, t, q, dout, out, lse, dlse, xs, ys, tid, nthr, s0, 0);
+      stage_qbox<T, D, R, QN>(P, t, q, dout, out, lse, dlse, xs, ys, tid, nthr, s0, 0);
     }
     __syncthreads();
     if (!ws.any) continue;
@@ -926,7 +929,7 @@ __global__ void __launch_bounds__(512)
           qt[db] = __builtin_shufflevector(q0, q1, 0, 1, 2, 3, 4, 5, 6, 7);
         }
       };
-      constexpr bool EARLY_T = D == 32 || (R != 1 && D < 128);
+      constexpr bool EARLY_T = D == 32 || (D < 128 && (R == 2 ? !PFS : R == 3 && PFS));
       if (EARLY_T) read_t();
       __builtin_amdgcn_sched_barrier(0);  // keep every read of the pair ahead
       // S masked through its initial value, dP - delta through its

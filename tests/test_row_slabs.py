@@ -71,3 +71,44 @@ def test_row_slabs_against_oracle(case):
     torch.autograd.backward((out, lse), (go.to(DEV), gl.to(DEV)))
     for t, r, n in zip(ts, O.grads(f, (q, k, v), (go, gl)), ("dq", "dk", "dv")):
         assert_close(t.grad, r, dtype, n)
+
+
+# Rank-3 boxes beyond LDS: eight waves on several layers.  (dtype, B, spatial, H,
+# Hkv, D, kernel, dilation, causal), large enough for two workgroups per CU.
+DEPTH = [
+    (BF16, 2, (9, 34, 33), 8, 4, 32, (3, 7, 7), (1, 1, 1), (False, False, False)),
+    (F16, 1, (11, 40, 40), 8, 8, 64, (3, 5, 5), (1, 1, 1), (True, False, False)),
+    (BF16, 1, (10, 33, 41), 16, 4, 64, (3, 7, 7), (1, 1, 2), (False, True, False)),
+]
+
+
+@pytest.mark.parametrize("case", DEPTH, ids=[f"{c[2]}-d{c[5]}" for c in DEPTH])
+def test_planned_on_several_layers(case):
+    from natten_amd._core import hip
+
+    dtype, B, sp, H, Hkv, D, ks, dil, caus = case
+    q = torch.empty((B, *sp, H, D), dtype=dtype, device="meta")
+    k = torch.empty((B, *sp, Hkv, D), dtype=dtype, device="meta")
+    p = hip.kernel_plan(q, k, ks, (1, 1, 1), dil, caus)
+    assert p["path"] == "lean" and p["waves"] == 8 and p["slabs"] == p["box"][0], p
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", DEPTH, ids=[f"{c[2]}-d{c[5]}" for c in DEPTH])
+def test_several_layers_against_the_32_query_kernels(case):
+    import natten_amd
+    from natten_amd._core import hip
+
+    dtype, B, sp, H, Hkv, D, ks, dil, caus = case
+    print(f"[case] several layers {case}", flush=True)
+    ts = [randn((B, *sp, h, D), dtype, i).to(DEV).requires_grad_(True)
+          for i, h in enumerate((H, Hkv, Hkv))]
+    res = []
+    for other in (False, True):
+        with hip.no_lean_kernels(other):
+            out, lse = natten_amd.na3d(*ts, ks, 1, dil, caus, return_lse=True)
+            go = randn(out.shape, dtype, 7).to(DEV)
+            gl = randn(lse.shape, dtype, 8).to(DEV)
+            res.append([out, lse, *torch.autograd.grad((out, lse), ts, (go, gl))])
+    for a, b, n in zip(*res, ("out", "lse", "dq", "dk", "dv")):
+        assert_close(a, b.double(), dtype, n)
