@@ -361,6 +361,21 @@ int na_merge_bwd(const na_merge_params *p, const void *const *outs,
                  const float *const *lses, const void *dout, const float *dlse,
                  void *const *d_outs, float *const *d_lses, void *stream);
 
+/* ---- layer projections ---------------------------------------------------- */
+/*
+ * Weight and bias gradient of y = x W^T + b over `rows` rows, for the
+ * attention layer's projections (nn/na2d.py:41-78): dw [n, k] = g^T x and,
+ * where db is non-NULL, db [n] = column sums of g; g [rows, n], x [rows, k],
+ * all bf16 or fp16 (enum na_dtype), sums in float32, rounded once.  n and k
+ * are multiples of 8, at most 16384.  The workspace size is 0 for what is not
+ * supported.
+ */
+size_t na_linear_wgrad_workspace_bytes(int32_t dtype, int64_t rows, int64_t n,
+                                       int64_t k);
+int na_linear_wgrad(int32_t dtype, int64_t rows, int64_t n, int64_t k,
+                    const void *g, const void *x, void *dw, void *db,
+                    void *workspace, size_t workspace_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

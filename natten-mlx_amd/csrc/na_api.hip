@@ -738,6 +738,26 @@ int na_rpb_av_bwd(const na_rpb_params *p, const float *attn, const void *value,
   return launch_status("na_rpb_av_bwd");
 }
 
+size_t na_linear_wgrad_workspace_bytes(int32_t dtype, int64_t rows, int64_t n, int64_t k) {
+  return na::linear_wgrad_ok(dtype, rows, n, k) ? na::linear_wgrad_workspace(rows, n, k) : 0;
+}
+
+int na_linear_wgrad(int32_t dtype, int64_t rows, int64_t n, int64_t k, const void *g,
+                    const void *x, void *dw, void *db, void *workspace,
+                    size_t workspace_bytes, void *stream) {
+  if (!na::linear_wgrad_ok(dtype, rows, n, k))
+    return fail(NA_ERR_UNSUPPORTED, "na_linear_wgrad: dtype %d, %lld x %lld over %lld rows", dtype,
+                (long long)n, (long long)k, (long long)rows);
+  if (g == nullptr || x == nullptr || dw == nullptr)
+    return fail(NA_ERR_INVALID, "g/x/dw must be non-NULL");
+  const size_t need = na::linear_wgrad_workspace(rows, n, k);
+  if (workspace == nullptr || workspace_bytes < need)
+    return fail(NA_ERR_WORKSPACE, "workspace needs %zu bytes, got %zu", need,
+                workspace == nullptr ? (size_t)0 : workspace_bytes);
+  na::linear_wgrad(dtype, rows, n, k, g, x, dw, db, workspace, as_stream(stream));
+  return launch_status("na_linear_wgrad");
+}
+
 int na_merge_fwd(const na_merge_params *p, const void *const *outs,
                  const float *const *lses, void *out, float *lse,
                  void *stream) {

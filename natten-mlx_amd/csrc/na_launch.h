@@ -201,6 +201,13 @@ void wsplit_rpb_qk_bwd(const RpbProb &A, const float *dl, const float *q, const 
 void wsplit_rpb_av_bwd(const RpbProb &A, const float *attn, const float *v,
                        const float *dout, float *dattn, float *dv, hipStream_t st);
 
+// Weight and bias gradient of a bf16 / fp16 linear map over M rows
+// (na_linear.hip): dw [N, K] = g^T x, db [N] = column sums of g (nullable).
+bool linear_wgrad_ok(int dtype, int64_t M, int64_t N, int64_t K);
+size_t linear_wgrad_workspace(int64_t M, int64_t N, int64_t K);
+void linear_wgrad(int dtype, int64_t M, int64_t N, int64_t K, const void *g, const void *x,
+                  void *dw, void *db, void *workspace, hipStream_t st);
+
 // Generic pieces reused around the MFMA backward.
 void valu_delta(const Prob &P, int dtype, const void *out, const void *dout,
                 const float *dlse, float *delta, hipStream_t st);

@@ -28,6 +28,8 @@ import torch
 from torch import nn as _nn
 
 from . import functional as F
+from ._core import _lib
+from .autograd import fused as _fused
 from .utils.params import normalize_tuple_param
 
 IntOrTuple = Union[int, Tuple[int, ...]]
@@ -38,6 +40,40 @@ _QK = {1: F.na1d_qk, 2: F.na2d_qk, 3: F.na3d_qk}
 _AV = {1: F.na1d_av, 2: F.na2d_av, 3: F.na3d_av}
 _VARLEN = {1: F.na1d_varlen, 2: F.na2d_varlen, 3: F.na3d_varlen}
 _INPUT = {1: "[B, L, C]", 2: "[B, H, W, C]", 3: "[B, D, H, W, C]"}
+
+
+_HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
+
+# Rows from which the projections' weight gradient takes the split kernels.
+_WGRAD_ROWS = 1024
+
+
+def _linear(m: _nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """``m(x)``.  A plain ``nn.Linear`` in training on 16-bit HIP tensors runs
+    as the operator whose backward forms the weight and bias gradient with
+    this library's kernels, bit for bit the same forward; anything else --
+    subclasses, parametrizations, hooks, autocast, transforms, compilation,
+    tensor subclasses, few rows -- is the module call itself."""
+    if type(m) is not _nn.Linear or not x.is_cuda or not torch.is_grad_enabled():
+        return m(x)
+    w, b = m.weight, m.bias
+    if (x.dtype not in (torch.bfloat16, torch.float16) or w.dtype != x.dtype
+            or not w.requires_grad or type(x) is not torch.Tensor
+            or type(w) is not _nn.Parameter or not w.is_contiguous()
+            or (b is not None and (type(b) is not _nn.Parameter or b.dtype != x.dtype
+                                   or b.device != x.device))
+            or x.numel() // max(x.shape[-1], 1) < _WGRAD_ROWS
+            or w.shape[0] % 8 or w.shape[1] % 8
+            or any(getattr(m, h) for h in _HOOKS) or "forward" in m.__dict__
+            or _fused._py_autograd
+            or torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling()
+            or torch.jit.is_tracing() or torch.overrides._is_torch_function_mode_enabled()
+            or torch._C._functorch.maybe_current_level() is not None
+            or torch.autograd.forward_ad._current_level >= 0
+            or torch.nn.modules.module._has_any_global_hook()):
+        return m(x)
+    op = _lib.node_op("linear", x, w)
+    return m(x) if op is None else op(x, w, b, _lib.stream_of(x))
 
 
 class _NeighborhoodAttention(_nn.Module):
@@ -107,11 +143,11 @@ class _NeighborhoodAttention(_nn.Module):
         into the projection output; the ops make them contiguous)."""
         lead = x.shape[:-1]
         if self._use_gqa:
-            q = self.q_proj(x).reshape(*lead, self.num_heads, self.head_dim)
-            kv = self.kv_proj(x).reshape(*lead, 2, self.num_kv_heads, self.head_dim)
+            q = _linear(self.q_proj, x).reshape(*lead, self.num_heads, self.head_dim)
+            kv = _linear(self.kv_proj, x).reshape(*lead, 2, self.num_kv_heads, self.head_dim)
             k, v = kv.unbind(dim=-3)
         else:
-            qkv = self.qkv(x).reshape(*lead, 3, self.num_heads, self.head_dim)
+            qkv = _linear(self.qkv, x).reshape(*lead, 3, self.num_heads, self.head_dim)
             q, k, v = qkv.unbind(dim=-3)
         return q, k, v
 
@@ -137,7 +173,7 @@ class _NeighborhoodAttention(_nn.Module):
         else:
             out = _FUSED[r](q, k, v, kernel_size=self.kernel_size, stride=self.stride,
                             dilation=self.dilation, is_causal=self.is_causal, scale=self.scale)
-        out = self.proj(out.reshape(*out.shape[:-2], self.embed_dim))
+        out = _linear(self.proj, out.reshape(*out.shape[:-2], self.embed_dim))
         if self.proj_drop is not None:
             out = self.proj_drop(out)
         return out
