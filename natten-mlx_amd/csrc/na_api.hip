@@ -738,6 +738,17 @@ int na_rpb_av_bwd(const na_rpb_params *p, const float *attn, const void *value,
   return launch_status("na_rpb_av_bwd");
 }
 
+int na_pack3(int32_t split, int64_t tokens, int64_t row_bytes, const void *src, void *dst,
+             void *stream) {
+  if (tokens == 0) return NA_OK;
+  if (!na::pack3_ok(tokens, row_bytes))
+    return fail(NA_ERR_UNSUPPORTED, "na_pack3: %lld rows of %lld bytes", (long long)tokens,
+                (long long)row_bytes);
+  if (src == nullptr || dst == nullptr) return fail(NA_ERR_INVALID, "src/dst must be non-NULL");
+  na::pack3(split != 0, tokens, row_bytes, src, dst, as_stream(stream));
+  return launch_status("na_pack3");
+}
+
 size_t na_linear_wgrad_workspace_bytes(int32_t dtype, int64_t rows, int64_t n, int64_t k) {
   return na::linear_wgrad_ok(dtype, rows, n, k) ? na::linear_wgrad_workspace(rows, n, k) : 0;
 }

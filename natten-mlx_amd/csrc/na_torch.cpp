@@ -241,6 +241,78 @@ std::tuple<at::Tensor, at::Tensor> na_fused(const at::Tensor &q, const at::Tenso
   return {r[0], r[1]};
 }
 
+// The fused op on a layer's packed projection qkv [B, X..., 3, H, D] (nn.py): the
+// three tensors come out of it in one pass and their gradients go back into one
+// packed gradient.
+struct FusedQKV : public torch::autograd::Function<FusedQKV> {
+  static variable_list forward(AutogradContext *ctx, at::Tensor qkv, at::IntArrayRef kernel,
+                               at::IntArrayRef stride, at::IntArrayRef dilation,
+                               at::IntArrayRef causal, double scale, int64_t flags,
+                               int64_t stream) {
+    check_device(qkv);
+    TORCH_CHECK(qkv.dim() >= 5 && qkv.size(-3) == 3,
+                "natten_amd na_fused_qkv: qkv is [B, *spatial, 3, H, D]");
+    qkv = qkv.contiguous();
+    std::vector<int64_t> sz(qkv.sizes().begin(), qkv.sizes().end());
+    const int64_t row = qkv.size(-1) * qkv.size(-2) * (int64_t)qkv.element_size();
+    sz.erase(sz.end() - 3);
+    std::vector<int64_t> all(sz);
+    all.insert(all.begin(), 3);
+    const int64_t tokens = row > 0 ? (int64_t)(qkv.numel() * qkv.element_size() / (3 * row)) : 0;
+    at::Tensor parts = at::empty(all, qkv.options());
+    check_rc(na_pack3(1, tokens, row, qkv.data_ptr(), parts.data_ptr(), reinterpret_cast<void *>(stream)),
+             "na_pack3");
+    const at::Tensor q = parts.select(0, 0), k = parts.select(0, 1), v = parts.select(0, 2);
+    const na_params p =
+        make_params(q, k, kernel, stride, dilation, causal, scale, 0, flags, at::Tensor());
+    for (size_t a = 0; a < kernel.size(); ++a) sz[1 + a] = (sz[1 + a] + stride[a] - 1) / stride[a];
+    at::Tensor out = at::empty(sz, qkv.options());
+    sz.pop_back();
+    at::Tensor lse = at::empty(sz, qkv.options().dtype(at::kFloat));
+    check_rc(na_fwd(&p, q.data_ptr(), k.data_ptr(), v.data_ptr(), nullptr, nullptr, out.data_ptr(),
+                    static_cast<float *>(lse.data_ptr()), as_stream(stream)),
+             "na_fwd");
+    ctx->save_for_backward({parts, out, lse});
+    ctx->saved_data["p"] = pack(p, {stream, tokens, row});
+    return {out};
+  }
+  static variable_list backward(AutogradContext *ctx, variable_list grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const at::Tensor &parts = s[0], &out = s[1], &lse = s[2];
+    const std::vector<int64_t> packed = ctx->saved_data["p"].toIntVector();
+    const int64_t *more;
+    const na_params p = unpack<na_params>(packed, &more);
+    void *stream = as_stream(more[0]);
+    const at::Tensor g = (grads[0].scalar_type() == parts.scalar_type()
+                              ? grads[0] : grads[0].to(parts.scalar_type())).contiguous();
+    const size_t ws_bytes = na_bwd_workspace_bytes(&p);
+    at::Tensor d = at::empty_like(parts);
+    at::Tensor ws = ws_bytes ? at::empty({(int64_t)ws_bytes}, parts.options().dtype(at::kByte))
+                             : at::Tensor();
+    auto part = [](const at::Tensor &t, int i) {
+      return static_cast<void *>(static_cast<char *>(t.data_ptr()) +
+                                 i * (t.numel() / 3) * (int64_t)t.element_size());
+    };
+    check_rc(na_bwd(&p, part(parts, 0), part(parts, 1), part(parts, 2), nullptr, nullptr,
+                    out.data_ptr(), static_cast<const float *>(lse.data_ptr()), g.data_ptr(),
+                    nullptr, part(d, 0), part(d, 1), part(d, 2), nullptr, nullptr, mptr(ws),
+                    ws_bytes, stream),
+             "na_bwd");
+    std::vector<int64_t> sz(parts.sizes().begin() + 1, parts.sizes().end());
+    sz.insert(sz.end() - 2, 3);
+    at::Tensor dqkv = at::empty(sz, parts.options());
+    check_rc(na_pack3(0, more[1], more[2], d.data_ptr(), dqkv.data_ptr(), stream), "na_pack3");
+    const at::Tensor none;
+    return {dqkv, none, none, none, none, none, none, none};
+  }
+};
+
+at::Tensor na_fused_qkv(const at::Tensor &qkv, at::IntArrayRef kernel, at::IntArrayRef stride,
+                        at::IntArrayRef dilation, at::IntArrayRef causal, double scale,
+                        int64_t flags, int64_t stream) {
+  return FusedQKV::apply(qkv, kernel, stride, dilation, causal, scale, flags, stream)[0];
+}
+
 // ---- split ops (autograd/split.py) ----------------------------------------
 // The caller has validated shapes (functional.py) and passes tensors of
 // supported dtypes on one device.
@@ -548,6 +620,9 @@ TORCH_LIBRARY(natten_amd, m) {
   m.def(
       "na_rpb_av(Tensor attn, Tensor v, int[] kernel, int[] dilation, bool heads_first, "
       "bool out_f32, int stream) -> Tensor");
+  m.def(
+      "na_fused_qkv(Tensor qkv, int[] kernel, int[] stride, int[] dilation, int[] causal, "
+      "float scale, int flags, int stream) -> Tensor");
   m.def("na_linear(Tensor x, Tensor weight, Tensor? bias, int stream) -> Tensor");
 }
 
@@ -558,4 +633,5 @@ TORCH_LIBRARY_IMPL(natten_amd, CompositeImplicitAutograd, m) {
   m.impl("na_rpb_qk", na_rpb_qk);
   m.impl("na_rpb_av", na_rpb_av);
   m.impl("na_linear", na_linear);
+  m.impl("na_fused_qkv", na_fused_qkv);
 }

@@ -155,6 +155,7 @@ SIGNATURES = {
     "na_rpb_qk_bwd": (ctypes.c_int, [_R, _V, _V, _V, _V, _V, _V, _V, ctypes.c_size_t, _V]),
     "na_rpb_av_bwd": (ctypes.c_int, [_R, _V, _V, _V, _I, _V, _V, _V]),
     "na_rpb_kernel_plan": (ctypes.c_int, [_R, ctypes.POINTER(NaRpbPlan)]),
+    "na_pack3": (ctypes.c_int, [_I, ctypes.c_int64, ctypes.c_int64, _V, _V, _V]),
     "na_linear_wgrad_workspace_bytes": (ctypes.c_size_t, [_I] + [ctypes.c_int64] * 3),
     "na_linear_wgrad": (ctypes.c_int, [_I] + [ctypes.c_int64] * 3 + [_V] * 5
                         + [ctypes.c_size_t, _V]),
@@ -205,7 +206,7 @@ def _load_fused_op() -> None:
     _fused_op = ns.na_fused.default
     _node_ops = {"qk": ns.na_split_qk.default, "av": ns.na_split_av.default,
                  "rpb_qk": ns.na_rpb_qk.default, "rpb_av": ns.na_rpb_av.default,
-                 "linear": ns.na_linear.default}
+                 "linear": ns.na_linear.default, "fused_qkv": ns.na_fused_qkv.default}
 
 
 def fused_op():
@@ -222,7 +223,8 @@ _OP_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
 
 def node_op(name: str, a: torch.Tensor, b: torch.Tensor):
     """The C++ operator of a split ("qk", "av") or DiNAT ("rpb_qk", "rpb_av")
-    op, or a layer's projection ("linear"), where it takes these tensors: built, and both of a supported dtype on
+    op, or a layer's projection ("linear") and packed attention
+    ("fused_qkv"), where it takes these tensors: built, and both of a supported dtype on
     one HIP device.  None otherwise (the Python autograd Function then runs
     the same kernels, or raises)."""
     if _lib is None:

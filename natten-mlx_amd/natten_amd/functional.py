@@ -142,6 +142,18 @@ def _fused_spec(rank, query, key, value, kernel_size, stride, dilation, is_causa
                      dense, causal_ints=tuple(int(bool(c)) for c in caus))
 
 
+def _packed_spec(rank, shape, qkv, kernel_size, stride, dilation, is_causal, scale) -> FusedSpec:
+    """The spec of the fused op on ``qkv`` [B, *spatial, 3 H D] holding q, k and
+    v of ``shape``."""
+    def make():
+        part = qkv.detach()[..., :shape[-1] * shape[-2]].reshape(shape)
+        return _fused_spec(rank, part, part, part, kernel_size, stride, dilation, is_causal,
+                           scale, None, None)
+
+    return _cached_spec(("qkv", rank, shape, kernel_size, stride, dilation, is_causal, scale),
+                        make)
+
+
 def _na(rank, query, key, value, kernel_size, stride, dilation, is_causal, scale, return_lse,
         additional_keys, additional_values):
     add = additional_keys is not None or additional_values is not None

@@ -28,7 +28,8 @@ import torch
 from torch import nn as _nn
 
 from . import functional as F
-from ._core import _lib
+from ._core import _lib, ops
+from ._core import hip as _hip
 from .autograd import fused as _fused
 from .utils.params import normalize_tuple_param
 
@@ -138,6 +139,48 @@ class _NeighborhoodAttention(_nn.Module):
                 f"num_kv_heads={self.num_kv_heads}, kernel_size={self.kernel_size}, "
                 f"stride={self.stride}, dilation={self.dilation}, is_causal={self.is_causal}")
 
+    def _attend_packed(self, x: torch.Tensor) -> Optional[torch.Tensor]:
+        """The fused op on the projection's packed output, where the operator
+        takes it: q, k and v leave it in one pass instead of three copies, and
+        their gradients return to it in one.  None otherwise."""
+        if (self._use_gqa or not x.is_cuda or type(x) is not torch.Tensor or _fused._py_autograd
+                or self.embed_dim * x.element_size() % 16
+                or 3 * x.numel() * x.element_size() >= 1 << 34
+                or torch.is_autocast_enabled("cuda") or ops.backend_module() is not _hip):
+            return None
+        op = _lib.node_op("fused_qkv", x, x)
+        if op is None:
+            return None
+        qkv = _linear(self.qkv, x)
+        shape = (*x.shape[:-1], self.num_heads, self.head_dim)
+        if (type(qkv) is not torch.Tensor or qkv.dtype != x.dtype or not qkv.is_contiguous()
+                or qkv.shape != (*x.shape[:-1], 3 * self.embed_dim)):
+            return self._attend_projected(*self._split_qkv(qkv))
+        spec = F._packed_spec(self.rank, torch.Size(shape), qkv, self.kernel_size, self.stride,
+                              self.dilation, self.is_causal, self.scale)
+        return op(qkv.view(*x.shape[:-1], 3, self.num_heads, self.head_dim), spec.kernel_size,
+                  spec.stride, spec.dilation, spec.causal_ints, spec.scale,
+                  _fused._op_flags(spec, None), _lib.stream_of(x))
+
+    def _split_qkv(self, qkv: torch.Tensor):
+        return qkv.reshape(*qkv.shape[:-1], 3, self.num_heads, self.head_dim).unbind(dim=-3)
+
+    def _attend_projected(self, q, k, v, sizes: Optional[torch.Tensor] = None) -> torch.Tensor:
+        r = self.rank
+        if sizes is not None:
+            return _VARLEN[r](q, k, v, sizes, kernel_size=self.kernel_size,
+                              dilation=self.dilation, scale=self.scale)
+        if self.attn_drop_rate > 0.0:
+            logits = _QK[r](q, k, kernel_size=self.kernel_size, dilation=self.dilation,
+                            stride=self.stride, is_causal=self.is_causal, scale=self.scale)
+            attn = torch.softmax(logits, dim=-1)
+            if self.attn_drop is not None:
+                attn = self.attn_drop(attn)
+            return _AV[r](attn, v, kernel_size=self.kernel_size, dilation=self.dilation,
+                          stride=self.stride, is_causal=self.is_causal)
+        return _FUSED[r](q, k, v, kernel_size=self.kernel_size, stride=self.stride,
+                         dilation=self.dilation, is_causal=self.is_causal, scale=self.scale)
+
     def _project(self, x: torch.Tensor):
         """``[B, *S, C]`` -> q ``[B, *S, H, D]``, k/v ``[B, *S, H_kv, D]`` (views
         into the projection output; the ops make them contiguous)."""
@@ -147,8 +190,7 @@ class _NeighborhoodAttention(_nn.Module):
             kv = _linear(self.kv_proj, x).reshape(*lead, 2, self.num_kv_heads, self.head_dim)
             k, v = kv.unbind(dim=-3)
         else:
-            qkv = _linear(self.qkv, x).reshape(*lead, 3, self.num_heads, self.head_dim)
-            q, k, v = qkv.unbind(dim=-3)
+            q, k, v = self._split_qkv(_linear(self.qkv, x))
         return q, k, v
 
     def _attend(self, x: torch.Tensor, sizes: Optional[torch.Tensor]) -> torch.Tensor:
@@ -158,21 +200,9 @@ class _NeighborhoodAttention(_nn.Module):
         if x.shape[-1] != self.embed_dim:
             raise ValueError(
                 f"Input channel dim ({x.shape[-1]}) must match embed_dim ({self.embed_dim})")
-        q, k, v = self._project(x)
-        if sizes is not None:
-            out = _VARLEN[r](q, k, v, sizes, kernel_size=self.kernel_size,
-                             dilation=self.dilation, scale=self.scale)
-        elif self.attn_drop_rate > 0.0:
-            logits = _QK[r](q, k, kernel_size=self.kernel_size, dilation=self.dilation,
-                            stride=self.stride, is_causal=self.is_causal, scale=self.scale)
-            attn = torch.softmax(logits, dim=-1)
-            if self.attn_drop is not None:
-                attn = self.attn_drop(attn)
-            out = _AV[r](attn, v, kernel_size=self.kernel_size, dilation=self.dilation,
-                         stride=self.stride, is_causal=self.is_causal)
-        else:
-            out = _FUSED[r](q, k, v, kernel_size=self.kernel_size, stride=self.stride,
-                            dilation=self.dilation, is_causal=self.is_causal, scale=self.scale)
+        out = self._attend_packed(x) if sizes is None and self.attn_drop_rate == 0.0 else None
+        if out is None:
+            out = self._attend_projected(*self._project(x), sizes)
         out = _linear(self.proj, out.reshape(*out.shape[:-2], self.embed_dim))
         if self.proj_drop is not None:
             out = self.proj_drop(out)

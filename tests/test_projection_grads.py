@@ -102,3 +102,29 @@ def test_what_is_not_plain_keeps_the_module_call():
         (gw,) = torch.autograd.grad(v, m.qkv.weight, create_graph=True)
         second.append(torch.autograd.grad(gw.float().square().sum(), m.qkv.weight)[0])
     assert _rel(second[1], second[0].double()) < 2.0 ** -6  # bf16 products in another order
+
+
+@pytest.mark.parametrize("dtype,rank,sp,dim,heads,kw", [
+    (torch.float32, 1, (70,), 48, 3, dict(kernel_size=7, stride=2)),
+    (torch.float32, 2, (9, 11), 4, 1, dict(kernel_size=3)),           # one 16-byte unit a row
+    (torch.float32, 2, (9, 11), 6, 2, dict(kernel_size=3)),           # not whole units: parts
+    (BF16, 2, (17, 15), 64, 2, dict(kernel_size=5, dilation=2)),
+    (F16, 3, (5, 8, 9), 32, 1, dict(kernel_size=3, is_causal=(True, False, False))),
+    (BF16, 1, (33,), 128, 2, dict(kernel_size=33)),                   # dense
+], ids=str)
+def test_packed_projection_matches_parts(dtype, rank, sp, dim, heads, kw):
+    import natten_amd
+    import natten_amd.autograd.fused as AF
+
+    torch.manual_seed(1)
+    m = getattr(natten_amd, f"NeighborhoodAttention{rank}D")(dim, heads, **kw).to(DEV, dtype)
+    for batch in (2, 0):
+        x = randn((batch, *sp, dim), dtype, 5).to(DEV).requires_grad_(True)
+        res = []
+        for py in (False, True):
+            with AF.python_autograd(py):
+                out = m(x)
+                g = randn(out.shape, dtype, 6).to(DEV)
+                res.append([out, *torch.autograd.grad(out, [x, *m.parameters()], g)])
+        for a, b in zip(*res):
+            assert a.shape == b.shape and torch.equal(a, b)
