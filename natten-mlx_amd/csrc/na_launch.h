@@ -197,7 +197,10 @@ void wsplit_rpb_gather(const RpbProb &A, const float *w, const float *y, float *
 void wsplit_rpb_inverse(const RpbProb &A, const float *w, const float *x, float *out,
                         float post, hipStream_t st);
 void wsplit_rpb_qk_bwd(const RpbProb &A, const float *dl, const float *q, const float *key,
-                       float *dq, float *dk, hipStream_t st);
+                       float *dq, float *dk, double *bias_part, hipStream_t st);
+// Partials per bias cell that wsplit_rpb_qk_bwd writes to bias_part (nullable;
+// [heads * cells][tiles] doubles); 0 where it does not apply.
+int32_t wsplit_rpb_bias_tiles(const RpbProb &A);
 void wsplit_rpb_av_bwd(const RpbProb &A, const float *attn, const float *v,
                        const float *dout, float *dattn, float *dv, hipStream_t st);
 

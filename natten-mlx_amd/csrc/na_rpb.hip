@@ -16,6 +16,8 @@
 // DiNAT head_dim of 12 in fp32).  Every kernel is a gather: dK/dV walk each
 // key's inverse neighborhood and the bias gradient is a fixed-order
 // two-pass reduction, so results are deterministic (no atomics).
+#include <algorithm>
+
 #include "na_common.h"
 #include "na_launch.h"
 #include "na_row.h"
@@ -2273,6 +2275,15 @@ void bias_chunking(const RpbProb &A, int32_t *chunk, int32_t *n_chunks) {
   *n_chunks = (int32_t)((nq + kBiasChunk - 1) / kBiasChunk);
 }
 
+// Bias partials per cell that the matrix-core dq pass writes, or 0 for a pass
+// of their own: ragged tiles may need more of them than chunks, which is taken
+// only while the partials stay below 32 MB.
+int32_t bias_tiles(const RpbProb &A, int32_t n_chunks) {
+  const int32_t n = wsplit_rpb_bias_tiles(A);
+  const int64_t bytes = (int64_t)n * A.H * A.R0 * A.R1 * (int64_t)sizeof(double);
+  return n <= n_chunks || bytes <= (32 << 20) ? n : 0;
+}
+
 }  // namespace
 
 void rpb_qk_fwd(const RpbProb &A, int dtype, const void *q, const void *key,
@@ -2298,7 +2309,7 @@ size_t rpb_bias_workspace_bytes(const RpbProb &A) {
   int32_t chunk, n_chunks;
   bias_chunking(A, &chunk, &n_chunks);
   const size_t nb = (size_t)A.H * A.R0 * A.R1;
-  return (size_t)n_chunks * nb * sizeof(double);
+  return (size_t)std::max(n_chunks, bias_tiles(A, n_chunks)) * nb * sizeof(double);
 }
 
 void rpb_qk_bwd(const RpbProb &A, int dtype, const void *q, const void *key,
@@ -2328,8 +2339,9 @@ void rpb_qk_bwd(const RpbProb &A, int dtype, const void *q, const void *key,
       if (pbias) n_fused = nph;
     }
     if (!pair && wsplit_rpb_eligible(A, kWsBwd)) {
+      if (drpb != nullptr) n_fused = bias_tiles(A, n_chunks);
       wsplit_rpb_qk_bwd(A, dlogits, (const float *)q, (const float *)key, (float *)dq,
-                        (float *)dk, st);
+                        (float *)dk, n_fused > 0 ? (double *)workspace : nullptr, st);
       pair = true;
     }
   }

@@ -24,8 +24,8 @@
 // LDS, product) rather than the matrix cores.  Against the vector-ALU kernels,
 // which read every neighbour row per query and divide per candidate in the
 // inverse pass: float32 [4, 56, 56, 2, 32] K = 7 with position bias, logits
-// 32.1 -> 13.5 us, AV 27.9 -> 10.4, QK backward 137 -> 31.7 (21 of it the bias
-// gradient's own passes), AV backward 117 -> 14.7; split ops on [4, 80, 80, 8,
+// 32.1 -> 13.5 us, AV 27.9 -> 10.4, QK backward 137 -> 21.6 (with the bias
+// gradient), AV backward 117 -> 14.7; split ops on [4, 80, 80, 8,
 // 32] K = 5: 75 -> 33, 56 -> 32, 188 -> 52, 196 -> 51.
 //
 // As in na_wave.hip a result with a NaN is computed again key by key, so a
@@ -61,6 +61,7 @@ struct WsQuery {
   bool valid = true;
   int row = 0;         // query-side row inside the sample
   int slot0 = 0, cell0 = 0;
+  uint32_t pb = 0;     // bias row of slot 0 per axis (axis 1 << 16 | axis 2)
   int64_t krow = 0;    // key-side row of box point 0 (head 0)
   template <int D>
   __device__ __forceinline__ void init(const WvProb &P, const WsLay &S, const WvTile &t, int n) {
@@ -78,6 +79,7 @@ struct WsQuery {
       win.axis(a, wv_start(x, i, t.Lr[a]) - box.lo[a], wv_end(x, i, t.Lr[a]) - 1 - box.lo[a]);
       slot0 += (box.lo[a] - raw) * S.st[a];
       cell0 += (box.lo[a] - i + x.K - 1) * S.rs[a];
+      if (a > 0) pb |= (uint32_t)((raw - i + x.K - 1) & 0xffff) << (a == 1 ? 16 : 0);
     }
     row += t.h * S.q_rh;
     box.finish();
@@ -167,16 +169,74 @@ __device__ __forceinline__ void ws_qk(const WvProb &P, const WsLay &S, uint32_t 
   ws_rows<false>(S, cr, out + t.b * P.Ltot * P.H * S.KK, nullptr, Q.row, Q.valid, lane);
 }
 
+// The tile's part of the bias gradient (rank 2), in float64: for each cell of
+// the table the sum over the tile's queries of the compact value whose slot has
+// that cell, to bpart[(head, cell)][tile of the head].  Where no window of the
+// tile is clamped slot 0's cell is K/2 on both axes: the K0 K1 cells from there
+// hold one sum each, the others are zero.  A tile past the end of a short phase
+// has no query and writes zeros (`any` false): every partial is written.
+// The rows are in LDS for dq already; read again by a pass of its own they
+// made QK backward 31.7 us at [4, 56, 56, 2, 32] K = 7 (21.6 so), 137 at
+// [6, 80, 80, 8, 32] K = 5 (89), 115 at [2, 56, 56, 4, 32] K = 13 (53).  At
+// rank 1 a table has too few cells for 64 lanes (82.0 -> 83.4 at [6, 6000, 12,
+// 32] K = 7 d = 2): it keeps the pass.
+__device__ __forceinline__ void ws_bias(const WvProb &P, const WsLay &S, const WvTile &t, uint32_t tile,
+                                        const WsQuery<2> &Q, const float *cr, int lane, bool any,
+                                        double *bpart) {
+  const WvAx &x1 = P.ax[1], &x2 = P.ax[2];
+  const int grid = (int)P.gq.fGrid.d, per_head = P.B * grid;
+  const int sp = (int)tile - (t.b * P.H + t.h) * grid;
+  double *dst = bpart + (int64_t)t.h * S.cells * per_head + t.b * grid + sp;
+  if (!any) {
+    for (int c = lane; c < S.cells; c += 64) dst[(int64_t)c * per_head] = 0.0;
+    return;
+  }
+  const uint32_t mid = (uint32_t)x1.nh << 16 | (uint32_t)x2.nh;
+  const uint32_t live = (uint32_t)__builtin_amdgcn_ballot_w64(Q.valid) & 0xffffu;
+  const bool inner = __builtin_amdgcn_ballot_w64(Q.pb != mid) == 0;
+  const int R2 = 2 * x2.K - 1;
+  const float rr = __builtin_amdgcn_rcpf((float)R2);
+  for (int c = lane; c < S.cells; c += 64) {
+    const int c1 = (int)(((float)c + 0.5f) * rr), c2 = c - c1 * R2;
+    double s = 0.0;
+    if (inner) {
+      const int k1 = c1 - x1.nh, k2 = c2 - x2.nh;
+      const bool ok = (unsigned)k1 < (unsigned)x1.K && (unsigned)k2 < (unsigned)x2.K;
+      const float *p = cr + (ok ? k1 * x2.K + k2 : 0);
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (live >> i & 1u) s += (double)p[i * S.KP];
+      s = ok ? s : 0.0;
+    } else {
+#pragma unroll 4
+      for (int i = 0; i < 16; ++i) {
+        const uint32_t pb = (uint32_t)__builtin_amdgcn_readlane((int)Q.pb, i);
+        const int k1 = c1 - (int)(pb >> 16), k2 = c2 - (int)(pb & 0xffffu);
+        const bool ok = (live >> i & 1u) && (unsigned)k1 < (unsigned)x1.K &&
+                        (unsigned)k2 < (unsigned)x2.K;
+        const float v = cr[i * S.KP + (ok ? k1 * x2.K + k2 : 0)];
+        s += ok ? (double)v : 0.0;
+      }
+    }
+    dst[(int64_t)c * per_head] = s;
+  }
+}
+
 template <int D, int R>
 __device__ __forceinline__ void ws_av(const WvProb &P, const WsLay &S, uint32_t tile, float *sm, int lane,
-                                      const float *a, const float *y, float *out, float mult) {
+                                      const float *a, const float *y, float *out, float mult,
+                                      double *bpart) {
   typedef Wv<float>::frag frag;
   constexpr int NF = D / 16, NDB = D / 16, RS = wv_rs<D>();
   const int n = lane & 15, gq = lane >> 4;
   WvTile t;
-  if (!wv_decode<R>(P, P.gq, P.fH, tile, false, t)) return;
-  const int hk = (int)fdiv((uint32_t)t.h, P.fRep);
   WsQuery<R> Q;
+  if (!wv_decode<R>(P, P.gq, P.fH, tile, false, t)) {
+    if constexpr (R == 2)
+      if (bpart != nullptr && t.b < P.B) ws_bias(P, S, t, tile, Q, sm, lane, false, bpart);
+    return;
+  }
+  const int hk = (int)fdiv((uint32_t)t.h, P.fRep);
   Q.template init<D>(P, S, t, n);
   const char *yb = reinterpret_cast<const char *>(y) +
                    (t.b * P.Ltot * P.Hkv + Q.krow + (int64_t)hk * S.k_rh) * (D * 4);
@@ -230,6 +290,8 @@ __device__ __forceinline__ void ws_av(const WvProb &P, const WsLay &S, uint32_t 
       for (int db = 0; db < NDB; ++db) acc[db] += w * ld4<float>(yr + 64 * db);
     }
   }
+  if constexpr (R == 2)
+    if (bpart != nullptr) ws_bias(P, S, t, tile, Q, cr, lane, true, bpart);
   if (!Q.valid) return;
   char *ob = reinterpret_cast<char *>(out + t.b * P.Ltot * P.H * D) + (uint64_t)(uint32_t)Q.row * (D * 4);
 #pragma unroll
@@ -350,7 +412,8 @@ __global__ void __launch_bounds__(256)
     k_wsplit(WvProb P, WsLay S, int n_inv, const float *__restrict__ x, const float *__restrict__ y,
              const float *__restrict__ bias, const float *__restrict__ a, float *__restrict__ out,
              float pre, float mult, float fill, const float *__restrict__ ia,
-             const float *__restrict__ ix, float *__restrict__ iz, float imult) {
+             const float *__restrict__ ix, float *__restrict__ iz, float imult,
+             double *__restrict__ bpart) {
   extern __shared__ __align__(16) float ws_smem[];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int nw = blockDim.x >> 6;
@@ -363,7 +426,7 @@ __global__ void __launch_bounds__(256)
   if constexpr (QK)
     ws_qk<D, R>(P, S, tile, sm, lane, x, y, bias, out, pre, mult, fill);
   else
-    ws_av<D, R>(P, S, tile, sm, lane, a, y, out, mult);
+    ws_av<D, R>(P, S, tile, sm, lane, a, y, out, mult, bpart);
 }
 
 // ---------------------------------------------------------------------------
@@ -410,7 +473,8 @@ struct WsInv {   // the key-side pass (z null: none)
   float *z, mult;
 };
 
-void ws_launch(const Prob &P, bool heads_first, const WsPass &p, const WsInv &v, hipStream_t st) {
+void ws_launch(const Prob &P, bool heads_first, const WsPass &p, const WsInv &v, hipStream_t st,
+               double *bpart = nullptr) {
   if (P.B == 0) return;
   WsLay S{};
   S.KK = P.kprod;
@@ -438,7 +502,7 @@ void ws_launch(const Prob &P, bool heads_first, const WsPass &p, const WsInv &v,
   if (grid.x == 0) return;
 #define WS_L(DD, RR, QQ)                                                                        \
   hipLaunchKernelGGL((k_wsplit<DD, RR, QQ>), grid, block, (size_t)S.lw * 4 * nw, st, W, S, n_inv, \
-                     p.x, p.y, p.bias, p.a, p.out, p.pre, p.mult, p.fill, v.a, v.x, v.z, v.mult)
+                     p.x, p.y, p.bias, p.a, p.out, p.pre, p.mult, p.fill, v.a, v.x, v.z, v.mult, bpart)
 #define WS_Q(DD, RR)                                     \
   do {                                                   \
     if (p.qk) WS_L(DD, RR, true); else WS_L(DD, RR, false); \
@@ -548,11 +612,18 @@ void wsplit_rpb_inverse(const RpbProb &A, const float *w, const float *x, float 
   ws_launch(rpb_prob(A), A.heads_first != 0, {}, {w, x, out, post}, st);
 }
 
+// One partial per tile of a head, for each cell of the bias table (rank 2).
+int32_t wsplit_rpb_bias_tiles(const RpbProb &A) {
+  if (A.rank != 2 || !wsplit_rpb_eligible(A, kWsBwd)) return 0;
+  const WvGrid G = wv_grid(rpb_prob(A), false, 4);
+  return (int32_t)(A.B * (int64_t)G.fGrid.d);
+}
+
 void wsplit_rpb_qk_bwd(const RpbProb &A, const float *dl, const float *q, const float *key, float *dq,
-                       float *dk, hipStream_t st) {
+                       float *dk, double *bias_part, hipStream_t st) {
   const float post = A.has_scale ? A.scale : 1.f;
   ws_launch(rpb_prob(A), A.heads_first != 0, {false, nullptr, key, nullptr, dl, dq, 1.f, post, 0.f},
-            {dl, q, dk, post}, st);
+            {dl, q, dk, post}, st, bias_part);
 }
 
 void wsplit_rpb_av_bwd(const RpbProb &A, const float *attn, const float *v, const float *dout,

@@ -176,3 +176,45 @@ def test_split_non_finite_values_stay_in_their_windows():
     want[0, :, :, 1, 3] = holds.to(DEV)
     assert torch.equal(bad, want)
     assert torch.allclose(out[~bad], clean[0][~bad], atol=1e-6)
+
+
+# (B, spatial, H, D, K, dilation) of the bias partials the dq pass writes;
+# empty tiles: short phases with no query in their last tile
+BIAS = [
+    (2, (97,), 3, 32, 7, 3),       # rank 1: a pass of its own
+    (1, (7, 9), 1, 16, 7, 1),      # every window but a few clamped, ragged tiles
+    (2, (17, 18), 2, 32, 3, 2),    # empty tiles, phases of two lengths
+    (1, (19, 33), 2, 64, 5, 3),
+    (3, (24, 40), 2, 32, 7, 1),    # inner tiles (no window clamped) and edges
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads_first", [False, True])
+@pytest.mark.parametrize("case", BIAS, ids=[f"{'x'.join(map(str, c[1]))}-k{c[4]}d{c[5]}" for c in BIAS])
+def test_bias_gradient_partials(case, heads_first):
+    """The workspace is NaN beforehand, so a partial that is not written shows.
+    Sums are float64 throughout: only the result's rounding to float32 (2^-24)
+    remains, and 2^-44 of the summed magnitudes for the order of the sum."""
+    from natten_amd._core import hip
+
+    B, sp, H, D, K, d = case
+    print(f"[case] bias partials {case} heads_first={heads_first}", flush=True)
+    r = len(sp)
+    q, k = (randn((B, *sp, H, D), F32, i) for i in range(2))
+    rpb = torch.zeros((H, *(2 * K - 1,) * r))
+    gl = randn((B, *sp, H, K**r), F32, 3)
+    ref = O.grads(lambda b: O.qk_rpb(q, k, b, K, d, 0.3), (rpb,), (gl,))[0]
+    mag = O.grads(lambda b: O.qk_rpb(q, k, b, K, d, 0.3), (rpb,), (gl.abs(),))[0]
+    put = (lambda t: t.movedim(-2, 1).contiguous().to(DEV)) if heads_first else (lambda t: t.to(DEV))
+    qd, kd, gd = put(q), put(k), put(gl)
+    lib = hip._lib.load()
+    p = hip._rpb_params(qd, K, d, heads_first, 0.3)
+    ws = torch.full((lib.na_rpb_bwd_workspace_bytes(p) // 8,), float("nan"), dtype=torch.float64,
+                    device=DEV)
+    dq, dk, drpb = torch.empty_like(qd), torch.empty_like(kd), torch.empty_like(rpb, device=DEV)
+    P = hip._lib.ptr
+    hip._lib.check(lib.na_rpb_qk_bwd(p, P(qd), P(kd), P(gd), P(dq), P(dk), P(drpb), P(ws),
+                                     ws.numel() * 8, hip._lib.stream_of(qd)), "na_rpb_qk_bwd")
+    err = (drpb.cpu().double() - ref).abs()
+    assert bool((err <= 2.0**-24 * ref.abs() + 2.0**-44 * mag).all()), err.max()
