@@ -226,7 +226,14 @@ def node_op(name: str, a: torch.Tensor, b: torch.Tensor):
     op, or a layer's projection ("linear") and packed attention
     ("fused_qkv"), where it takes these tensors: built, and both of a supported dtype on
     one HIP device.  None otherwise (the Python autograd Function then runs
-    the same kernels, or raises)."""
+    the same kernels, or raises): under compilation, which can leave a Python
+    Function to eager execution but not an operator without a fake kernel, while
+    tracing, and inside a torch.func transform or a forward-mode level, which a
+    Python Function refuses and vmap would pass by an operator."""
+    if (torch.compiler.is_compiling() or torch._C._functorch.maybe_current_level() is not None
+            or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._get_tracing_state() is not None):
+        return None
     if _lib is None:
         if not a.is_cuda:
             return None

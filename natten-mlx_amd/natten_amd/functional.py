@@ -247,6 +247,8 @@ def _split_spec(spatial, rank, kernel_size, dilation, stride, is_causal):
 
 def _cached_spec(key, make):
     """``make()``, kept by call signature as the fused op's specs are."""
+    if torch.compiler.is_compiling():
+        return make()
     try:
         spec = _spec_cache.get(key)
     except TypeError:  # an unhashable argument

@@ -154,3 +154,36 @@ def test_nodes_refuse_what_the_functions_refuse():
     out = F.na2d_av(torch.softmax(F.na2d_qk(empty, empty, 3), -1), empty, 3)
     assert out.shape == (0, 9, 9, 2, 32)
     assert torch.autograd.grad(out.sum(), empty)[0].shape == empty.shape
+
+
+@pytest.mark.gpu
+def test_compiled_split_ops_run_as_eager():
+    """The operators have no fake kernels: under compilation the split ops are
+    Python Functions left to eager execution."""
+    import natten_amd
+
+    torch.manual_seed(0)
+    layer = natten_amd.NeighborhoodAttention2D(64, 2, 3, attn_drop=0.1).to(DEV).eval()
+    x = _t((1, 12, 14, 64), F32, 1).requires_grad_()
+    ts = [_t((1, 12, 14, 2, 32), F32, i).requires_grad_() for i in range(3)]
+    for fn, leaves in ((lambda *a: _split(a, dict(kernel_size=3))[1], ts), (layer, [x])):
+        torch._dynamo.reset()
+        res = []
+        for f in (fn, torch.compile(fn, backend="eager")):
+            out = f(*leaves)
+            res.append([out, *torch.autograd.grad(out.square().sum(), leaves)])
+        for a, b in zip(*res):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ["split 2d bf16", "rpb 1d"])
+def test_transforms_stay_refused(case):
+    fn, shapes, arg = CASES[case]
+    ts = [_t(s, dt, i) for i, (s, dt) in enumerate(shapes)]
+    with pytest.raises(RuntimeError, match="functorch"):
+        torch.vmap(lambda *a: fn(a, arg)[1])(*[t[None].repeat(2, *[1] * t.dim()) for t in ts])
+    with pytest.raises(RuntimeError, match="functorch"):
+        torch.func.grad(lambda *a: fn(a, arg)[1].float().sum())(*ts)
+    with torch.autograd.forward_ad.dual_level(), pytest.raises(NotImplementedError):
+        fn([torch.autograd.forward_ad.make_dual(t, torch.ones_like(t)) for t in ts], arg)
