@@ -6,13 +6,14 @@
 // The reference's autograd layer (autograd/na1d.py:34-53, na2d.py:34-64,
 // na3d.py) wraps the fused forward / backward in an mx.custom_function; the
 // Python twins here are autograd/fused.py's _FusedNA, autograd/split.py's and
-// autograd/allin1.py's Functions.  These nodes do the same work without Python in the backward and without ctypes marshalling in
-// either direction: an eager training step is host-bound (the config-2
-// kernels take ~21 us per step, the host path several times that), so the
-// per-call host cost is what a caller who does not capture graphs sees.  A split
-// or DiNAT step has two nodes each way: eager, against the Python Functions over
-// ctypes, split [4, 56, 56, 4, 32] K = 7 186 -> 107 us, DiNAT [8, 2048, 12, 12]
-// K = 7 188 -> 116 us (66 and 57 us of them on the GPU).
+// autograd/allin1.py's Functions.  These nodes do the same work without
+// Python in the backward and without ctypes marshalling in either direction:
+// an eager training step is host-bound (the config-2 kernels take ~21 us per
+// step, the host path several times that), so the per-call host cost is what a
+// caller who does not capture graphs sees.  A split or DiNAT step has two nodes
+// each way: eager, against the Python Functions over ctypes, split
+// [4, 56, 56, 4, 32] K = 7 186 -> 107 us, DiNAT [8, 2048, 12, 12] K = 7
+// 188 -> 116 us (66 and 57 us of them on the GPU).
 //
 // Built with the host compiler against torch's headers only (no HIP
 // headers): the caller passes torch's current stream handle, and the
