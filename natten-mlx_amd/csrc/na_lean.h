@@ -1022,6 +1022,12 @@ bool lean_shape_ok(const Prob &P, int dtype) {
   return true;
 }
 
+// Rank 1 and 2 problems whose sample holds 2^24 elements or more.
+bool lean_large(const Prob &P) {
+  return P.rank < 3 && (int64_t)P.ax[1].L * P.ax[2].L * std::max(P.H, P.Hkv) * P.D >=
+                           (int64_t(1) << 24);
+}
+
 bool lean_disabled() {
   static const bool off = [] {
     const char *e = std::getenv("NATTEN_AMD_NO_LEAN");

@@ -44,13 +44,16 @@ namespace {
 // `ones` is an A operand whose row 0 is all ones, so lacc[0] of lane n
 // (lanes 0-15) accumulates the sum of query n's rounded probabilities (the
 // same values that weight V) and the other lanes' lacc stay zero.
-template <typename T, int D, int NB>
+// EX: the reference point m is the running maximum itself, so the largest
+// probability so far is exactly 1 in 16 bits, and the lane's ls sums its
+// float32 probabilities (the log-sum-exp's row sum).
+template <typename T, int D, int NB, bool EX>
 __device__ __forceinline__ void fwd_group(const typename L16<T>::e *ks,
                                           const typename L16<T>::e *vs,
                                           const int (&kb)[NB], f32x4 (&sv)[NB],
                                           const typename L16<T>::v8 (&qf)[D / 32],
                                           f32x4 (&o)[D / 16], float &m, f32x4 &lacc,
-                                          const typename L16<T>::v8 &ones,
+                                          float &ls, const typename L16<T>::v8 &ones,
                                           float sl2, int ka_off, int tr_off,
                                           bool fresh) {
   typedef L16<T> M;
@@ -78,15 +81,17 @@ __device__ __forceinline__ void fwd_group(const typename L16<T>::e *ks,
   // ---- online softmax ----
   mx = quad_max(mx) * sl2;
   // The reference point m may trail the running max by up to 8 (a factor
-  // 2^8 in P): exact after the final division by l, and it spares the O
-  // rescale on groups that do not raise any query's max by more.  The first
-  // group of a query head finds O and l zero: it only sets m.
+  // 2^8 in P; not with EX): exact after the final division by l but for the
+  // rounding of P, and it spares the O rescale on groups that do not raise any
+  // query's max by more.  The first group of a query head finds O and l zero:
+  // it only sets m.
   if (fresh) {
     m = mx;
-  } else if (__builtin_amdgcn_ballot_w64(mx > m + 8.f) != 0) {
+  } else if (__builtin_amdgcn_ballot_w64(mx > m + (EX ? 0.f : 8.f)) != 0) {
     const float mn = fmaxf(m, mx);
     const float alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
     lacc *= alpha;
+    if (EX) ls *= alpha;
 #pragma unroll
     for (int j = 0; j < NDB; ++j) o[j] *= alpha;
     m = mn;
@@ -101,6 +106,7 @@ __device__ __forceinline__ void fwd_group(const typename L16<T>::e *ks,
       for (int r = 0; r < 4; ++r) {
         const float p = __builtin_amdgcn_exp2f(fmaf(sv[2 * jj + h][r], sl2, -mu));
         bp[jj][4 * h + r] = (E)p;
+        if (EX) ls += p;
       }
   // ---- O^T += V^T . P^T, two chunks per MFMA ----
 #pragma unroll
@@ -130,11 +136,18 @@ __device__ __forceinline__ void fwd_group(const typename L16<T>::e *ks,
 // while the previous slab is computed (SlabPrefetch).  At rank 2 slabs are box
 // rows and only this form has them: a box that does not fit LDS whole (head_dim
 // 64 from K = 9 to 13, head_dim 128 from K = 5) ran as one-wave workgroups or on
-// 32-query tiles straight from L2 (fp16 [1, 384, 384, 8, 64] K = 13 forward 494
-// -> 292 us, backward 1358 -> 1102; [1, 256, 256, 16, 128] K = 7 454 -> 267 and
-// 1247 -> 907; [2, 96, 96, 8, 64] K = 9 backward 245 -> 92).  Loading a slab after
-// the one before it is done instead: 318 and 1152 us for the first of these.
-template <typename T, int D, int R, bool CPR1, bool VX, bool CA, bool PFS>
+// 32-query tiles straight from L2 (fp16 [1, 384, 384, 8, 64] K = 13 forward 490
+// -> 299 us, backward 1365 -> 1076; [1, 256, 256, 16, 128] K = 7 456 -> 284 and
+// 1258 -> 910; [2, 96, 96, 8, 64] K = 9 backward 250 -> 100).  Loading a slab after
+// the one before it is done instead: 318 and 1152 us for the first of these
+// (292 and 1102 with the loads ahead, then, without EX).
+// EX (fwd_group): row slabs, and problems of rank 1 and 2 whose sample holds
+// 2^24 elements or more.  Their other kernel (k_mfwd) sums float32 probabilities
+// against a maximum over more keys: fp16 [1, 384, 384, 8, 64] K = 13, LSE (rms
+// error) 2.9e-7 there, 2.5e-5 here without EX, 2.9e-7 with it; output 2.75e-4,
+// 2.82e-4, 2.65e-4; dq 3.009e-4, 3.025e-4, 3.005e-4.  It costs 1 to 5% of the
+// forward (288 -> 299 us; bf16 [1, 65536, 8, 64] K = 31 54.5 -> 55.4).
+template <typename T, int D, int R, bool CPR1, bool VX, bool CA, bool PFS, bool EX>
 __global__ void __launch_bounds__(512)
     k_wfwd(LProb Pin, const T *__restrict__ q, const T *__restrict__ k,
            const T *__restrict__ v, const T *__restrict__ ek,
@@ -266,6 +279,7 @@ __global__ void __launch_bounds__(512)
   float m = -INFINITY;
   bool fresh = true;  // no softmax group of this query head run yet
   f32x4 lacc = zero4();
+  float ls = 0.f;
   v8 ones;
 #pragma unroll
   for (int i = 0; i < 8; ++i) ones[i] = (E)(n == 0 ? 1.f : 0.f);
@@ -344,7 +358,8 @@ __global__ void __launch_bounds__(512)
         sv[j] = mask_init(ok, cb);
         if (R >= 2 && !CPR1) advance(cc, ws);
       }
-      fwd_group<T, D, G>(ks, vs, kb, sv, qf, o, m, lacc, ones, sl2, ka_off, tr_off, fresh);
+      fwd_group<T, D, G, EX>(ks, vs, kb, sv, qf, o, m, lacc, ls, ones, sl2, ka_off, tr_off,
+                             fresh);
       fresh = false;
     };
     if constexpr (NB >= 4) {
@@ -359,6 +374,7 @@ __global__ void __launch_bounds__(512)
 
   // ---- epilogue: sum l over the query's 4 lanes, normalise, store ----
   const float l = quad_sum(lacc[0]);
+  const float l32 = EX ? quad_sum(ls) : l;
   if (VX ? qt : qv) {
     const float inv = qv && l > 0.f ? 1.f / l : 0.f;
 #pragma unroll
@@ -369,7 +385,7 @@ __global__ void __launch_bounds__(512)
       *reinterpret_cast<v4 *>(out + qoff + 16 * db + 4 * gq) = wv;
     }
     if (lse != nullptr && gq == 0)
-      lse[(uint32_t)qoff / D] = !qv ? 0.f : l > 0.f ? (m + __log2f(l)) * kLn2 : -INFINITY;
+      lse[(uint32_t)qoff / D] = !qv ? 0.f : l32 > 0.f ? (m + __log2f(l32)) * kLn2 : -INFINITY;
   }
   }  // query heads
 }
@@ -1094,24 +1110,28 @@ void lean_fwd(const Prob &P, int dtype, const void *q, const void *k,
                    (int64_t)L.ebox * (P.D / 8) <= (int64_t)8 * 64 * C.W &&
                    3 * lds_f > (size_t)160 * 1024 && C.W <= 4 && !slab_prefetch_off();
   const bool slab2 = P.rank == 2 && C.sl < C.Em[1];
+  const bool ex = lean_large(P);
   const size_t lds = lean_lds_bytes(P, kLFwd, L.ebox, C.W);
   const dim3 grid(L.n_launch), block(64 * C.W);
-#define LF_LAUNCH2(TT, DD, RR, CC, VV, AA, PP)                                  \
-  hipLaunchKernelGGL((k_wfwd<TT, DD, RR, CC, VV, AA, PP>), grid, block, lds, st, L, \
+#define LF_LAUNCH2(TT, DD, RR, CC, VV, AA, PP, XX)                              \
+  hipLaunchKernelGGL((k_wfwd<TT, DD, RR, CC, VV, AA, PP, XX>), grid, block, lds, st, L, \
                      (const TT *)q, (const TT *)k, (const TT *)v,              \
                      (const TT *)ek, (const TT *)ev, (TT *)out, lse)
+#define LF_LAUNCH3(TT, DD, RR, CC, VV, PP, XX)                                  \
+  do {                                                                        \
+    if (ca) LF_LAUNCH2(TT, DD, RR, CC, VV, true, PP, XX);                     \
+    else LF_LAUNCH2(TT, DD, RR, CC, VV, false, PP, XX);                       \
+  } while (0)
 #define LF_LAUNCH1(TT, DD, RR, CC, VV)                                          \
   do {                                                                        \
-    if (RR == 3 && !VV && pfs) {                                              \
-      if (ca) LF_LAUNCH2(TT, DD, RR, CC, VV, true, (RR == 3 && !VV));         \
-      else LF_LAUNCH2(TT, DD, RR, CC, VV, false, (RR == 3 && !VV));           \
-    } else if (RR == 2 && CC && !VV && slab2) {                               \
-      if (ca) LF_LAUNCH2(TT, DD, RR, CC, VV, true, (RR == 2 && CC && !VV));   \
-      else LF_LAUNCH2(TT, DD, RR, CC, VV, false, (RR == 2 && CC && !VV));     \
-    } else {                                                                  \
-      if (ca) LF_LAUNCH2(TT, DD, RR, CC, VV, true, false);                    \
-      else LF_LAUNCH2(TT, DD, RR, CC, VV, false, false);                      \
-    }                                                                         \
+    if (RR == 3 && !VV && pfs)                                                \
+      LF_LAUNCH3(TT, DD, RR, CC, VV, (RR == 3 && !VV), false);                \
+    else if (RR == 2 && CC && !VV && slab2)                                   \
+      LF_LAUNCH3(TT, DD, RR, CC, VV, (RR == 2 && CC && !VV), (RR == 2));      \
+    else if (RR < 3 && ex)                                                    \
+      LF_LAUNCH3(TT, DD, RR, CC, VV, false, (RR < 3));                        \
+    else                                                                      \
+      LF_LAUNCH3(TT, DD, RR, CC, VV, false, false);                           \
   } while (0)
 #define LF_LAUNCH(TT, DD, RR, CC)                                              \
   do {                                                                        \
@@ -1137,6 +1157,7 @@ void lean_fwd(const Prob &P, int dtype, const void *q, const void *k,
 #undef LF_R
 #undef LF_LAUNCH
 #undef LF_LAUNCH1
+#undef LF_LAUNCH3
 #undef LF_LAUNCH2
 }
 
