@@ -903,7 +903,7 @@ LChoice lean_choice_compute(const Prob &P, LMode mode) {
 // lock, and keeps the last kPlanCache problems.
 constexpr int kPlanCache = 8;
 struct LChoiceKey {
-  int32_t v[20];
+  int32_t v[21];
 };
 LChoice lean_choice(const Prob &P, LMode mode) {
   LChoiceKey key{};
@@ -915,6 +915,7 @@ LChoice lean_choice(const Prob &P, LMode mode) {
   key.v[n++] = P.n_extra;
   key.v[n++] = P.sample_extent != nullptr ? 1 : 0;
   key.v[n++] = P.B;
+  key.v[n++] = P.H;
   key.v[n++] = P.Hkv;
   for (int a = 0; a < 3; ++a) {
     key.v[n++] = P.ax[a].L;
@@ -925,6 +926,7 @@ LChoice lean_choice(const Prob &P, LMode mode) {
   thread_local LChoiceKey keys[kPlanCache];
   thread_local LChoice vals[kPlanCache];
   thread_local int used = 0, next = 0;
+  static_assert(sizeof key.v / sizeof key.v[0] == 9 + 3 * 4, "one place per input");
   for (int i = 0; i < used; ++i)
     if (std::memcmp(&keys[i], &key, sizeof key) == 0) return vals[i];
   const LChoice c = lean_choice_compute(P, mode);

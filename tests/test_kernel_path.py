@@ -7,6 +7,9 @@ backward; unchecked varlen and over-budget rank-1/2 boxes stay on the
 32-query matrix-core kernels; fp32, even kernels and strides on the generic
 kernels."""
 
+from concurrent.futures import ThreadPoolExecutor
+
+import pytest
 import torch
 
 from natten_amd._core import hip
@@ -245,3 +248,31 @@ def test_plan_cache_returns_the_computed_plans():
     a = _plan((4, 56, 56, 4, 32), 4, (7, 7), (1, 1), (False, False), backward=True)
     b = _plan((1, 56, 56, 4, 32), 4, (7, 7), (1, 1), (False, False), backward=True)
     assert a["workgroups"] != b["workgroups"]
+
+
+# Problems that differ only in query heads: (shape_q at H, kernel, causal), with
+# the two H that the forward plans differently (key/value heads: 2).
+GROUPED = [
+    ((1, 10, 33, 41, 64), (3, 7, 7), (True, False, False), 16, 2),
+    ((1, 12, 32, 32, 64), (3, 7, 7), (False, False, False), 16, 2),
+    ((1, 112, 112, 32), (11, 11), (False, False), 16, 2),
+]
+
+
+@pytest.mark.parametrize("case", GROUPED, ids=[f"{c[0]}" for c in GROUPED])
+def test_plan_does_not_depend_on_other_query_heads(case):
+    """A plan is the same in a thread that has planned nothing and after the
+    problem with other query heads over the same key/value heads."""
+    shape, ks, caus, *heads = case
+    one = (1,) * len(ks)
+
+    def plans(order):
+        with ThreadPoolExecutor(1) as ex:  # a thread of its own: an empty cache
+            return ex.submit(lambda: {h: _plan((*shape[:-1], h, shape[-1]), 2, ks, one, caus)
+                                      for h in order}).result()
+
+    alone = {**plans(heads[:1]), **plans(heads[1:])}
+    assert plans(heads) == alone
+    assert plans(heads[::-1]) == alone
+    assert alone[heads[0]]["slabs"] != alone[heads[1]]["slabs"] or \
+        alone[heads[0]]["waves"] != alone[heads[1]]["waves"]  # else the case shows nothing
