@@ -60,7 +60,10 @@ enum na_flags {
    * Lets na_fwd and na_bwd run such problems on the lean kernels; a sample
    * that breaks the promise gets wrong values in its rows (every memory
    * access stays inside the tensors). */
-  NA_FLAG_VARLEN_CLAMPED = 8
+  NA_FLAG_VARLEN_CLAMPED = 8,
+  /* rank-2 lean kernels stage row slabs wherever they can run, whatever the
+     launch gains by it (tests of their edges on small problems) */
+  NA_FLAG_ROW_SLABS = 16
 };
 
 /*

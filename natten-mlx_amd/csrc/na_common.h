@@ -193,6 +193,7 @@ struct Prob {
   float scale;
   const int32_t *sample_extent;  // [B, rank] or nullptr
   int32_t varlen_clamped;  // caller: d * K <= sample extent, non-causal axes
+  int32_t row_slabs;       // caller: row slabs whatever the launch gains
 };
 
 // Division by a divisor fixed at launch (round-up multiply method of

@@ -579,14 +579,8 @@ int ilog2c(int x) {
 
 constexpr size_t kLdsBudget = 80 * 1024;  // per workgroup: >= 2 per CU
 
-// Rank-2 forward boxes beyond this are staged in row slabs although they would
-// fit the budget: three workgroups to a CU instead of two ([2, 96, 96, 8, 64]
-// K = 9, 78 KB: 27.4 -> 22.7 us; [2, 112, 112, 4, 64] K = 5, 60 KB: 19.5 ->
-// 16.4; [2, 72, 100, 8, 128] K = 5: 41 -> 28).  Head_dim 32, with half the
-// loads per row, gains from four workgroups per CU on ([4, 112, 112, 4, 32]
-// K = 11: 34.2 -> 31.9; [4, 56, 56, 4, 32] K = 13: 13.1 -> 14.0).  The backward, whose slabs restage
-// the query box too, keeps what fits ([4, 56, 56, 4, 64] K = 7, 69 KB: 26.4 us
-// whole, 30.9 in slabs).
+// A third of a CU's LDS: forward boxes beyond it may be staged in row slabs
+// although they fit the budget (row_slabs).
 constexpr size_t kRowSlabBox = 160 * 1024 / 3;
 
 // LDS budget per workgroup; NATTEN_AMD_LEAN_LDS_KB overrides it (tuning).
@@ -639,6 +633,8 @@ int lds_rows(int R, const int Em[3]) {
   while (p2 < Em[2]) p2 <<= 1;
   return Em[0] * Em[1] * p2;
 }
+
+bool lean_large(const Prob &P);
 
 // The axis a box is staged along in slabs: layers at rank 3, rows at rank 2.
 int slab_axis(int R) { return R == 2 ? 1 : 0; }
@@ -700,6 +696,97 @@ int box_max(const Axis &x, int t, bool inverse) {
   return best;
 }
 
+// The fused rank-2 kernels may stage their box a few rows at a time, as many as
+// one round of prefetched units covers, where a wave's part of a row is one
+// chunk (the backward: two, which an inverse box has beside an edge of the
+// image).  C is the choice among whole boxes (not ok: none fits), its cost
+// per_wave; a choice in slabs replaces it by rules on the launch:
+//
+// A box beyond the budget, where a smaller workgroup's box fits whole (one or
+// two waves): four waves over slabs stage fewer rows but leave a quarter of the
+// workgroups.  From one per CU on they gain (times in slabs over whole, [256,
+// 512) workgroups: forward 0.53 to 0.9 at head_dim 64, 0.51 to 1.07 at 128, all
+// but 1.07 above 256; backward 0.5 to 0.96, grouped heads up to 1.18), below they
+// lose (forward 1.02 to 1.35, backward 1.1 to 1.6).  Head_dim 32's smaller rows
+// need more (forward 1.19 at 256, 1.08 at 608, 0.59 to 0.8 from 1024).
+// A box beyond the budget and no whole one (the 32-query kernels otherwise, which
+// split a tile's chunks over four waves): the forward always gains (0.28 to 0.97);
+// the backward, whose dK / dV half walks the query heads of a group one after the
+// other, by the rows it stages for each product the windows need (`fill`): up to
+// 0.1 it takes 0.49 to 1.1 times as long from 512 workgroups on (384 at head_dim
+// 128; grouped heads of head_dim 32 only up to 0.07, or 1.13), above it up to 1.34;
+// with 256 to 512 workgroups 0.7 to 1.19, with fewer up to 3.6 times as long.
+// Head_dim 128 with full rows gains up to 0.13 (0.6 to 0.96 from 512 workgroups).
+// A whole box that fits the budget but not three times a CU (forward): three
+// workgroups to a CU instead of two pay when there are many (head_dim 64 / 128
+// from 5 per CU on 0.79 to 0.99, below 0.87 to 1.19; head_dim 32, with half the
+// loads per row, from 32 on 0.89 to 0.99, below up to 1.12).  The backward, whose
+// slabs restage the query box too, keeps what fits ([4, 56, 56, 4, 64] K = 7, 69
+// KB: 26.4 us whole, 30.9 in slabs).
+template <typename Ext, typename Wgs>
+void row_slabs(const Prob &P, LMode mode, const int *Ws, int nW, Ext ext, Wgs wgs_of, LChoice &C,
+               double &per_wave) {
+  const bool bwd = mode == kLBwd, any = P.row_slabs != 0;
+  auto slab = [&](const int (&Em)[3], int W) {  // rows of a slab
+    return std::min(Em[1], 4 * 64 * W / (P.D / 8) / (lds_rows(2, Em) / Em[1]));
+  };
+  auto cost = [&](const int (&Em)[3], int W, int sl) {  // staged rows per wave
+    return (double)lds_rows(2, Em) / W * (1.0 + 0.25 * ((Em[1] + sl - 1) / sl - 1));
+  };
+  // a large sample's whole box in two-wave workgroups of head_dim 64 is slower in
+  // the backward than the 32-query kernels (1.21 to 1.29, other widths 0.5 to 1.03)
+  const bool whole = C.ok && !(bwd && P.D == 64 && C.W < 4 && lean_large(P));
+  C.ok = whole;
+  if (!C.cpr1 && !(bwd && ext(2, C.T[2]) <= 32)) return;
+  bool thirds = false;  // the whole box in slabs after all
+  if (whole && !bwd && slab(C.Em, C.W) > 0 &&
+      lean_lds_bytes(P, mode, lds_rows(2, C.Em), C.W) > kRowSlabBox &&
+      (any || wgs_of(C.W, C.sa) >= (P.D == 32 ? 32 : 5) * kLeanCUs)) {
+    thirds = true;
+    C.sl = slab(C.Em, C.W);
+    per_wave = cost(C.Em, C.W, C.sl);
+  }
+  // padded rows staged by the whole launch
+  double total = whole ? per_wave * C.W * (double)wgs_of(C.W, C.sa) : 1e300;
+  const bool grouped = P.rep > 1;
+  bool found = whole;
+  for (int wi = 0; wi < nW; ++wi)
+    for (int sa = 1; sa < 3; ++sa) {
+      const int W = Ws[wi];
+      const Axis &x = P.ax[sa];
+      if (W > 1 && C.T[sa] * (W - 1) >= (x.L + x.d - 1) / x.d) continue;
+      int Em[3];
+      for (int a = 0; a < 3; ++a) Em[a] = ext(a, C.T[a] * (a == sa ? W : 1));
+      if (lean_lds_bytes(P, mode, lds_rows(2, Em), W) <= lds_budget()) continue;
+      const int sl = slab(Em, W), lrows = lds_rows(2, Em) / Em[1];
+      if (sl < 1 || lean_lds_bytes(P, mode, lrows * sl, W) > lds_budget()) continue;
+      const int64_t wgs = wgs_of(W, sa), n = wgs * W / 4;  // n: in workgroups of four waves
+      if (any) {
+        // no rule on the launch
+      } else if (whole) {
+        if (bwd ? n < (grouped ? 2 : 1) * kLeanCUs : P.D == 32 ? n < 3 * kLeanCUs : n <= kLeanCUs)
+          continue;
+      } else if (bwd) {
+        const double fill = (double)lds_rows(2, Em) * (double)wgs /
+                            ((double)P.B * P.Hkv * P.ax[1].L * P.ax[2].L * P.kprod);
+        const bool full = P.D == 128 && !grouped && n >= 2 * kLeanCUs && 3 * Em[2] > 2 * lrows;
+        if (2 * n < (grouped || P.D < 128 ? 4 : 3) * kLeanCUs ||
+            fill > (full ? 0.13 : grouped && P.D == 32 ? 0.07 : 0.1))
+          continue;
+      }
+      const double c = cost(Em, W, sl), t = c * W * (double)wgs;
+      if (whole && !any && t >= total) continue;
+      if (found && c >= per_wave * 0.999 && !(c < per_wave * 1.001 && sl > C.sl && !thirds)) continue;
+      found = true;
+      per_wave = c;
+      C.W = W;
+      C.sa = sa;
+      C.sl = sl;
+      for (int a = 0; a < 3; ++a) C.Em[a] = Em[a];
+    }
+  C.ok = found;
+}
+
 // Wave tile: the power-of-two shape with the fewest (waves x chunks);
 // workgroup: up to 8 waves stacked along the axis with the smallest staged
 // box per wave whose box fits the LDS budget.  For the backward the boxes
@@ -754,6 +841,17 @@ LChoice lean_choice_compute(const Prob &P, LMode mode) {
         best.cpr1 = R > 1 && e2 <= 16;
       }
     }
+  // workgroups of W waves stacked along sa
+  const int heads = mode == kLBwd ? P.Hkv : P.H;
+  auto wgs_of = [&](int W, int sa) {
+    int64_t n = (int64_t)P.B * heads;
+    for (int a = lead; a < 3; ++a) {
+      const Axis &x = P.ax[a];
+      const int tw = best.T[a] * (a == sa ? W : 1);
+      n *= (int64_t)x.d * (((x.L + x.d - 1) / x.d + tw - 1) / tw);
+    }
+    return n;
+  };
   double best_per_wave = 1e300;
   // the largest wave count, then the powers of two below it
   int Ws[5], nW = 0;
@@ -761,6 +859,7 @@ LChoice lean_choice_compute(const Prob &P, LMode mode) {
   Ws[nW++] = wmax;
   for (int W = 8; W >= 1; W >>= 1)
     if (W < wmax) Ws[nW++] = W;
+  const int sx = slab_axis(R);
   for (int wi = 0; wi < nW; ++wi)
     for (int sa = lead; sa < 3; ++sa) {
       const int W = Ws[wi];
@@ -769,34 +868,11 @@ LChoice lean_choice_compute(const Prob &P, LMode mode) {
       if (W > 1 && best.T[sa] * (W - 1) >= (x.L + x.d - 1) / x.d) continue;
       int Em[3];
       for (int a = 0; a < 3; ++a) Em[a] = ext(a, best.T[a] * (a == sa ? W : 1));
-      // rank 3 may stage the box a few layers (axis 0) at a time; the fused
-      // rank-2 kernels a few rows, as many as one round of prefetched units
-      // covers, where a wave's part of a row is one chunk (the backward: two,
-      // which an inverse box has beside an edge of the image)
-      const int sx = slab_axis(R);
+      // rank 3 may stage the box a few layers (axis 0) at a time
       int sl = Em[sx];
       const int lrows = lds_rows(R, Em) / Em[sx];  // LDS rows per layer or row
-      const bool rows2 = R == 2 && P.sample_extent == nullptr && P.n_extra == 0 &&
-                         ((best.cpr1 && (mode == kLFwd || mode == kLBwd)) ||
-                          (mode == kLBwd && ext(2, best.T[2]) <= 32));
-      bool early = rows2 && mode == kLFwd;  // slabs before the budget asks for them
-      if (early && P.D == 32) {
-        int64_t wgs = (int64_t)P.B * P.H;
-        for (int a = lead; a < 3; ++a) {
-          const int tw = best.T[a] * (a == sa ? W : 1), Lr = (P.ax[a].L + P.ax[a].d - 1) / P.ax[a].d;
-          wgs *= (int64_t)P.ax[a].d * ((Lr + tw - 1) / tw);
-        }
-        early = wgs >= 4 * kLeanCUs;
-      }
-      if (R == 2 &&
-          lean_lds_bytes(P, mode, lrows * sl, W) > (early ? kRowSlabBox : lds_budget())) {
-        if (!rows2) continue;
-        sl = std::min(sl, 4 * 64 * W / (P.D / 8) / lrows);
-        if (sl < 1) continue;
-      }
       while (R == 3 && sl > 1 && lean_lds_bytes(P, mode, lrows * sl, W) > lds_budget()) --sl;
-      const int ebox = lrows * sl;
-      if (lean_lds_bytes(P, mode, ebox, W) > lds_budget()) continue;
+      if (lean_lds_bytes(P, mode, lrows * sl, W) > lds_budget()) continue;
       // staged rows per wave over all slabs, each extra slab (a restaging
       // round trip and barrier) counted as a quarter more
       const int nsl = (Em[sx] + sl - 1) / sl;
@@ -811,6 +887,8 @@ LChoice lean_choice_compute(const Prob &P, LMode mode) {
         best.ok = true;
       }
     }
+  if (R == 2 && (mode == kLFwd || mode == kLBwd) && P.sample_extent == nullptr && P.n_extra == 0)
+    row_slabs(P, mode, Ws, nW, ext, wgs_of, best, best_per_wave);
   // The rank-2 backward: a workgroup of 5 to 7 waves where its tile divides
   // every dilation phase exactly and fewer waves land on the busiest CU.
   // Every workgroup of such a launch is resident at once and the backward
@@ -820,17 +898,8 @@ LChoice lean_choice_compute(const Prob &P, LMode mode) {
   // lighter per wave, is not faster with them).  NATTEN_AMD_LEAN_WAVES
   // turns this off.
   if (best.ok && mode == kLBwd && R == 2 && best.sl == best.Em[1] && !lean_waves_forced()) {
-    auto tiles_of = [&](int W, int sa) {
-      int64_t n = (int64_t)P.B * P.Hkv;
-      for (int a = lead; a < 3; ++a) {
-        const Axis &x = P.ax[a];
-        const int tw = best.T[a] * (a == sa ? W : 1);
-        n *= (int64_t)x.d * (((x.L + x.d - 1) / x.d + tw - 1) / tw);
-      }
-      return n;
-    };
     auto busiest = [&](int W, int sa) {
-      return (tiles_of(W, sa) + kLeanCUs - 1) / kLeanCUs * W;
+      return (wgs_of(W, sa) + kLeanCUs - 1) / kLeanCUs * W;
     };
     int64_t cur = busiest(best.W, best.sa);
     for (int W = 7; W >= 5; --W)
@@ -903,7 +972,7 @@ LChoice lean_choice_compute(const Prob &P, LMode mode) {
 // lock, and keeps the last kPlanCache problems.
 constexpr int kPlanCache = 8;
 struct LChoiceKey {
-  int32_t v[21];
+  int32_t v[22];
 };
 LChoice lean_choice(const Prob &P, LMode mode) {
   LChoiceKey key{};
@@ -914,6 +983,7 @@ LChoice lean_choice(const Prob &P, LMode mode) {
   key.v[n++] = P.kprod;
   key.v[n++] = P.n_extra;
   key.v[n++] = P.sample_extent != nullptr ? 1 : 0;
+  key.v[n++] = P.row_slabs;
   key.v[n++] = P.B;
   key.v[n++] = P.H;
   key.v[n++] = P.Hkv;
@@ -926,7 +996,7 @@ LChoice lean_choice(const Prob &P, LMode mode) {
   thread_local LChoiceKey keys[kPlanCache];
   thread_local LChoice vals[kPlanCache];
   thread_local int used = 0, next = 0;
-  static_assert(sizeof key.v / sizeof key.v[0] == 9 + 3 * 4, "one place per input");
+  static_assert(sizeof key.v / sizeof key.v[0] == 10 + 3 * 4, "one place per input");
   for (int i = 0; i < used; ++i)
     if (std::memcmp(&keys[i], &key, sizeof key) == 0) return vals[i];
   const LChoice c = lean_choice_compute(P, mode);

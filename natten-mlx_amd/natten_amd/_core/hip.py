@@ -25,6 +25,7 @@ from . import _lib
 # the generic vector-ALU kernels even where the matrix-core kernels apply.
 _force_generic = os.environ.get("NATTEN_AMD_GENERIC", "0") == "1"
 _no_lean = False
+_row_slabs = False
 
 
 @contextlib.contextmanager
@@ -50,6 +51,19 @@ def no_lean_kernels(enabled: bool = True):
         yield
     finally:
         _no_lean = prev
+
+
+@contextlib.contextmanager
+def row_slab_kernels(enabled: bool = True):
+    """Temporarily let rank-2 problems take the lean kernels' row slabs
+    wherever they can run, also where the launch is too small to gain."""
+    global _row_slabs
+    prev = _row_slabs
+    _row_slabs = enabled
+    try:
+        yield
+    finally:
+        _row_slabs = prev
 
 
 def is_available() -> bool:
@@ -93,6 +107,7 @@ def _params_entry(q: torch.Tensor, k: torch.Tensor, kernel_size, stride, dilatio
                   sample_extent: Optional[torch.Tensor] = None, varlen_clamped: bool = False):
     flags = ((_lib.NA_FLAG_DENSE if dense else 0) | (_lib.NA_FLAG_GENERIC if _force_generic else 0)
              | (_lib.NA_FLAG_NO_LEAN if _no_lean else 0)
+             | (_lib.NA_FLAG_ROW_SLABS if _row_slabs else 0)
              | (_lib.NA_FLAG_VARLEN_CLAMPED if varlen_clamped and sample_extent is not None
                 else 0))
     se_ptr = None if sample_extent is None else sample_extent.data_ptr()

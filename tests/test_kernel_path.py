@@ -255,7 +255,7 @@ def test_plan_cache_returns_the_computed_plans():
 GROUPED = [
     ((1, 10, 33, 41, 64), (3, 7, 7), (True, False, False), 16, 2),
     ((1, 12, 32, 32, 64), (3, 7, 7), (False, False, False), 16, 2),
-    ((1, 112, 112, 32), (11, 11), (False, False), 16, 2),
+    ((1, 112, 112, 32), (11, 11), (False, False), 64, 2),
 ]
 
 

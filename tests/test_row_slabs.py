@@ -46,13 +46,54 @@ CASES = [
 
 @pytest.mark.parametrize("case", CASES, ids=[f"{c[2]}-d{c[5]}-k{c[6]}" for c in CASES])
 def test_planned_in_row_slabs(case):
-    p = _plan(*case[1:], case[0], True)
+    from natten_amd._core import hip
+
+    with hip.row_slab_kernels():  # small launches: see the rules below
+        p = _plan(*case[1:], case[0], True)
     assert p["path"] == "lean" and p["slabs"] > 1, p
+
+
+# What a launch's size and shape decide: (B, spatial, H, Hkv, D, kernel, backward)
+# and the plan: path, boxes in slabs, waves.
+LAUNCHES = [
+    # too few workgroups, or many query heads to one: not in slabs
+    ((1, (27, 36), 16, 1, 64, (15, 15), True), ("mfma", False)),
+    ((4, (56, 56), 16, 2, 32, (13, 13), True), ("mfma", False)),
+    ((1, (43, 27), 4, 1, 128, (5, 5), True), ("lean", False)),
+    ((1, (74, 52), 2, 2, 64, (7, 7), False), ("lean", False)),
+    ((2, (23, 26), 1, 1, 64, (11, 7), False), ("lean", False)),
+    ((4, (56, 56), 4, 4, 32, (13, 13), False), ("lean", False)),
+    # a row of 17 padded to 32; a large image's two-wave boxes
+    ((1, (290, 420), 1, 1, 64, (11, 11), True), ("mfma", False)),
+    ((2, (306, 351), 4, 4, 64, (5, 9), True), ("mfma", False)),
+    # enough of them
+    ((2, (96, 96), 8, 8, 64, (9, 9), True), ("lean", True)),
+    ((1, (256, 256), 16, 16, 128, (7, 7), True), ("lean", True)),
+    ((2, (112, 112), 4, 4, 64, (5, 5), False), ("lean", True)),
+    ((8, (91, 79), 16, 16, 32, (13, 13), False), ("lean", True)),  # 32 per CU and more
+    ((2, (72, 100), 8, 8, 128, (5, 5), False), ("lean", True)),
+    # no whole box: the forward in slabs at any size
+    ((1, (21, 20), 1, 1, 128, (13, 13), False), ("lean", True)),
+]
+
+
+@pytest.mark.parametrize("problem,want", LAUNCHES, ids=[f"{c[0]}" for c in LAUNCHES])
+def test_slabs_where_the_launch_gains(problem, want):
+    B, sp, H, Hkv, D, ks, backward = problem
+    p = _plan(B, sp, H, Hkv, D, ks, (1, 1), (False, False), F16, backward)
+    assert (p["path"], p["slabs"] > 1) == want, p
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", CASES, ids=[f"{c[2]}-d{c[5]}-k{c[6]}" for c in CASES])
 def test_row_slabs_against_oracle(case):
+    from natten_amd._core import hip
+
+    with hip.row_slab_kernels():
+        _row_slabs_against_oracle(case)
+
+
+def _row_slabs_against_oracle(case):
     import natten_amd
 
     dtype, B, sp, H, Hkv, D, ks, dil, caus = case
