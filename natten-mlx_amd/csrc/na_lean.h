@@ -930,17 +930,28 @@ LChoice lean_choice_compute(const Prob &P, LMode mode) {
   // for 8 (bf16, forward / backward: [1, 16, 32, 32, 8, 64] K = (3, 7, 7) causal
   // in depth 47 -> 38 / 119 -> 98 us, [1, 24, 40, 40, 8, 64] K = (3, 5, 5) 117 ->
   // 66 / 312 -> 190, [1, 24, 40, 40, 8, 32] K = (3, 7, 7) 94 -> 65 / 213 -> 166).
+  // Over 661 problems that the rules below admit they take 0.75 of the time
+  // (geometric mean, at most 1.04); what the rules turn down took up to 1.6 times as
+  // long: ragged tiles that add a third of waves or more (0.49 to 1.62), a second
+  // round of a few workgroups (0.75 to 1.61 below 1024 workgroups), and the backward
+  // and head_dim 32 where the four-wave form already runs three workgroups to a CU
+  // (0.65 to 1.17).
   if (best.ok && R == 3 && (mode == kLFwd || mode == kLBwd) && best.sl < best.Em[0] &&
       P.sample_extent == nullptr && P.n_extra == 0 && !lean_waves_forced()) {
-    double least = best_per_wave;
     const LChoice base = best;
+    // three of the four-wave workgroups to a CU
+    const bool thirds =
+        3 * lean_lds_bytes(P, mode, lds_rows(R, base.Em) / base.Em[0] * base.sl, base.W) <=
+        (size_t)160 * 1024;
+    double least = best_per_wave;
+    const double waves = (double)wgs_of(base.W, base.sa) * base.W;
     for (int w0 = 2; w0 <= 8; w0 <<= 1)
       for (int sa = 1; sa < 3; ++sa) {
         const int W1 = 8 / w0;
         const int TW[3] = {base.T[0] * w0, base.T[1] * (sa == 1 ? W1 : 1),
                            base.T[2] * (sa == 2 ? W1 : 1)};
         int Em[3];
-        int64_t wgs = (int64_t)P.B * (mode == kLBwd ? P.Hkv : P.H);
+        int64_t wgs = (int64_t)P.B * heads;
         bool fits = true;  // every wave tile starts inside the phase
         for (int a = 0; a < 3; ++a) {
           const int Lr = (P.ax[a].L + P.ax[a].d - 1) / P.ax[a].d;
@@ -948,9 +959,16 @@ LChoice lean_choice_compute(const Prob &P, LMode mode) {
           wgs *= (int64_t)P.ax[a].d * ((Lr + TW[a] - 1) / TW[a]);
           Em[a] = ext(a, TW[a]);
         }
-        // a layer's barrier and round trip, with 16 waves to hide them
-        const double rows = (double)lds_rows(R, Em) / 8 * (1.0 + 0.15 * (Em[0] - 1));
-        if (!fits || wgs < 2 * kLeanCUs || rows >= least ||
+        // a layer's barrier and round trip, with 16 waves to hide them, for the
+        // waves of ragged tiles too; `last`: the round of two workgroups per CU
+        // that is not full
+        const double pad = 8.0 * (double)wgs / waves;
+        const double rows = (double)lds_rows(R, Em) / 8 * (1.0 + 0.15 * (Em[0] - 1)) * pad;
+        const double round = 2.0 * kLeanCUs;
+        const double last = wgs < 4 * kLeanCUs ? std::ceil(wgs / round) * round / wgs : 1.0;
+        if (!fits || wgs < 2 * kLeanCUs || rows >= least || pad > 1.3 ||
+            rows * last >= best_per_wave * (P.D == 128 ? 0.9 : 1.15) ||
+            (thirds && (mode == kLBwd || P.D == 32)) ||
             lean_lds_bytes(P, mode, lds_rows(R, Em) / Em[0], 8) > lds_budget())
           continue;
         least = rows;

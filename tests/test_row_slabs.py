@@ -134,6 +134,32 @@ def test_planned_on_several_layers(case):
     assert p["path"] == "lean" and p["waves"] == 8 and p["slabs"] == p["box"][0], p
 
 
+# (B, spatial, H, Hkv, D, kernel, dilation, causal, backward) and waves per workgroup.
+LAYERS = [
+    # ragged tiles that add a third of waves, a second round of a few workgroups
+    ((1, (9, 30, 38), 2, 2, 128, (3, 3, 3), 1, (True, False, False), False), 4),
+    ((1, (9, 30, 38), 2, 2, 128, (3, 3, 3), 1, (True, False, False), True), 2),
+    ((8, (20, 32, 19), 1, 1, 64, (7, 3, 3), 2, (True, False, False), False), 4),
+    ((1, (10, 38, 28), 4, 4, 128, (7, 7, 7), (1, 2, 2), (False,) * 3, False), 4),
+    # three four-wave workgroups to a CU
+    ((2, (3, 21, 44), 16, 16, 32, (3, 7, 7), 1, (False,) * 3, True), 4),
+    ((1, (16, 32, 32), 8, 8, 64, (3, 7, 7), 1, (True, False, False), False), 8),
+    ((1, (16, 32, 32), 8, 8, 64, (3, 7, 7), 1, (True, False, False), True), 8),
+]
+
+
+@pytest.mark.parametrize("problem,waves", LAYERS, ids=[f"{c[0][1]}-{c[0][8]}" for c in LAYERS])
+def test_layers_where_the_launch_gains(problem, waves):
+    from natten_amd._core import hip
+
+    B, sp, H, Hkv, D, ks, dil, caus, backward = problem
+    q = torch.empty((B, *sp, H, D), dtype=BF16, device="meta")
+    k = torch.empty((B, *sp, Hkv, D), dtype=BF16, device="meta")
+    dil = (dil,) * 3 if isinstance(dil, int) else dil
+    p = hip.kernel_plan(q, k, ks, (1, 1, 1), dil, caus, backward=backward)
+    assert p["path"] == "lean" and p["waves"] == waves, p
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", DEPTH, ids=[f"{c[2]}-d{c[5]}" for c in DEPTH])
 def test_several_layers_against_the_32_query_kernels(case):
