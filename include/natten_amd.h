@@ -149,6 +149,23 @@ enum na_kernel_path_t {
 int na_kernel_path(const na_params *p, int32_t backward);
 
 /*
+ * Diagnostic with no counterpart in the reference: whether a pass that runs on
+ * the generic family (NA_PATH_GENERIC) takes its matrix-core form in 32-bit
+ * arithmetic (1) or the vector-ALU kernels (0; also where the pass runs on
+ * another family), or the negated na_status of invalid parameters.  Launches
+ * nothing and reads no device memory.
+ */
+enum na_pass_t {
+  NA_PASS_FWD = 0,    /* na_fwd */
+  NA_PASS_BWD = 1,    /* na_bwd */
+  NA_PASS_QK = 2,     /* na_qk_fwd */
+  NA_PASS_AV = 3,     /* na_av_fwd */
+  NA_PASS_QK_BWD = 4, /* na_qk_bwd */
+  NA_PASS_AV_BWD = 5  /* na_av_bwd */
+};
+int na_matrix_form(const na_params *p, int32_t pass);
+
+/*
  * Diagnostic with no counterpart in the reference: how na_fwd (backward =
  * 0) or na_bwd (backward = 1) launches for these parameters.  Fields past
  * `path` describe the lean kernels and are 0 on the other paths.  Launches
@@ -306,17 +323,20 @@ int na_rpb_av_bwd(const na_rpb_params *p, const float *attn, const void *value,
 /*
  * Host-only diagnostic: the kernel family each allin1 pass of these
  * parameters runs on, as the launchers choose it (no device work).  Rank-1
- * float32 problems take the staged kernels (a block's windows in LDS) or,
- * for large dilations, the phase-major ones; everything else the generic
- * kernels.  qk assumes a bias table, dq a requested drpb (fused_bias: the dq
- * pass also forms the bias gradient's partials).  The kernels' choice has
+ * float32 problems of head_dim up to 16 take the staged kernels (a block's
+ * windows in LDS) or, for large dilations, the phase-major ones; other float32
+ * problems the matrix-core tiles where they gain; everything else the generic
+ * kernels.  qk assumes a bias table; the backward passes assume that every
+ * gradient is requested (fused_bias: the dq pass also forms the bias gradient's
+ * partials).  The kernels' choice has
  * no counterpart in the reference (its Metal kernels are chosen by K and
  * head_dim, functional_metal.py:1921-2033).
  */
 enum na_rpb_kernel_t {
   NA_RPB_GENERIC = 0, /* k_rpb_dot / k_rpb_gather / k_rpb_inverse */
   NA_RPB_STAGED = 1,  /* k_r1_dot / k_r1_gather / k_r1_inverse */
-  NA_RPB_PHASE = 2    /* k_r1p_dot / k_r1p_gather */
+  NA_RPB_PHASE = 2,   /* k_r1p_dot / k_r1p_gather */
+  NA_RPB_TILE = 3     /* k_wsplit: float32 matrix-core tiles */
 };
 typedef struct na_rpb_plan {
   int32_t qk;         /* na_rpb_qk_fwd */

@@ -396,6 +396,23 @@ int na_kernel_path(const na_params *p, int32_t backward) {
   return NA_PATH_GENERIC;
 }
 
+int na_matrix_form(const na_params *p, int32_t pass) {
+  if (pass < NA_PASS_FWD || pass > NA_PASS_AV_BWD)
+    return -fail(NA_ERR_INVALID, "unknown pass %d", pass);
+  const int path = na_kernel_path(p, pass <= NA_PASS_BWD ? pass : 2);
+  if (path != NA_PATH_GENERIC) return path < 0 ? path : 0;
+  na::Prob P;
+  const int rc = make_prob(p, &P, pass <= NA_PASS_BWD);
+  if (rc != NA_OK) return -rc;
+  switch (pass) {
+    case NA_PASS_FWD: return use_wave_fwd(p, P);
+    case NA_PASS_BWD: return use_wave_bwd(p, P);
+    case NA_PASS_QK: return use_wsplit(p, P, na::kWsQk);
+    case NA_PASS_AV: return use_wsplit(p, P, na::kWsAv);
+    default: return use_wsplit(p, P, na::kWsBwd);
+  }
+}
+
 int na_kernel_plan(const na_params *p, int32_t backward, na_plan *plan) {
   if (plan == nullptr) return fail(NA_ERR_INVALID, "plan is NULL");
   if (backward != 0 && backward != 1)

@@ -1775,6 +1775,7 @@ size_t ph_inverse_lds(const RpbProb &A, int *cap) {
 // Which rank-1 fp32 kernels apply (the launchers below and rpb_plan share
 // these): the staged contiguous ones, the phase-major ones, or neither.
 enum R1Kind { kR1None = 0, kR1Staged = 1, kR1Phase = 2 };
+constexpr int kRpbTile = 3;  // NA_RPB_TILE: the matrix-core tiles (na_wsplit.hip)
 R1Kind r1_kind(const RpbProb &A, bool bias) {
   if (r1_lds(A, rpb_block(A), bias) != 0) return kR1Staged;
   if (ph_lds(A, bias) != 0) return kR1Phase;
@@ -2416,6 +2417,18 @@ void rpb_plan(const RpbProb &A, int dtype, RpbPlanInfo *o) {
                   ((staged_bias && nblk <= n_chunks) || (phase_bias && nph <= n_chunks));
   o->dq = o->fused_bias ? (staged_bias ? (int)kR1Staged : (int)kR1Phase) : kind(false);
   o->block = o->qk == kR1Phase ? kPhBlock : rb;
+  if (!f32) return;
+  // what is left runs on the matrix-core tiles where they apply; dq with dk and
+  // dattn with dv in one launch (the rank-1 kernels above take head_dims below theirs)
+  if (o->qk == 0 && wsplit_rpb_eligible(A, kWsQk)) o->qk = kRpbTile;
+  if (o->av == 0 && wsplit_rpb_eligible(A, kWsAv)) o->av = kRpbTile;
+  if (wsplit_rpb_eligible(A, kWsBwd)) {
+    if (o->dq == 0 && o->dk == 0) {
+      o->dq = o->dk = kRpbTile;
+      o->fused_bias = bias_tiles(A, n_chunks) > 0;
+    }
+    if (o->dattn == 0 && o->dv == 0) o->dattn = o->dv = kRpbTile;
+  }
 }
 
 void rpb_av_bwd(const RpbProb &A, int dtype, int out_dtype, const float *attn,

@@ -106,7 +106,8 @@ class NaRpbPlan(ctypes.Structure):
     ]
 
 
-RPB_GENERIC, RPB_STAGED, RPB_PHASE = 0, 1, 2
+RPB_GENERIC, RPB_STAGED, RPB_PHASE, RPB_TILE = 0, 1, 2, 3
+PASSES = {"fwd": 0, "bwd": 1, "qk": 2, "av": 3, "qk_bwd": 4, "av_bwd": 5}  # na_pass_t
 
 
 class NaMergeParams(ctypes.Structure):
@@ -140,6 +141,7 @@ SIGNATURES = {
     "na_neighbor_table": (ctypes.c_int, [_P, _V, _V, _V]),
     "na_mfma_selftest": (ctypes.c_int, [_I, _V, _V]),
     "na_kernel_path": (ctypes.c_int, [_P, _I]),
+    "na_matrix_form": (ctypes.c_int, [_P, _I]),
     "na_kernel_plan": (ctypes.c_int, [_P, _I, ctypes.POINTER(NaPlan)]),
     "na_fwd": (ctypes.c_int, [_P, _V, _V, _V, _V, _V, _V, _V, _V]),
     "na_bwd_workspace_bytes": (ctypes.c_size_t, [_P]),

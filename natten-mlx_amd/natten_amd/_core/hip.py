@@ -184,6 +184,20 @@ def kernel_path(q, k, kernel_size, stride, dilation, is_causal, scale=None, n_ex
     return KERNEL_PATHS[r]
 
 
+def matrix_form(which, q, k, kernel_size, stride, dilation, is_causal, scale=None, n_extra=0,
+                sample_extent=None):
+    """Whether pass ``which`` ("fwd", "bwd", "qk", "av", "qk_bwd", "av_bwd") of
+    this problem runs on the generic family's matrix-core form (a diagnostic;
+    launches nothing); False on the vector ALU and on the other families."""
+    lib = _lib.load()
+    p = _params(q, k, kernel_size, stride, dilation, is_causal, scale, n_extra, False,
+                sample_extent)
+    r = int(lib.na_matrix_form(p, _lib.PASSES[which]))
+    if r < 0:
+        _lib.check(-r, "na_matrix_form")
+    return bool(r)
+
+
 def kernel_plan(q, k, kernel_size, stride, dilation, is_causal, scale=None, n_extra=0,
                 dense=False, sample_extent=None, backward=False, varlen_clamped=False):
     """How na_fwd (or na_bwd) launches for this problem (a diagnostic;

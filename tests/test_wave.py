@@ -59,6 +59,44 @@ CASES = [
 ]
 
 
+def _form(which, case):
+    from natten_amd._core import hip
+
+    dtype, B, sp, H, Hkv, D, ks, dil, st, caus = case
+    q = torch.empty((B, *sp, H, D), dtype=dtype, device="meta")
+    k = torch.empty((B, *sp, Hkv, D), dtype=dtype, device="meta")
+    return hip.matrix_form(which, q, k, ks, st, dil, caus, 0.3)
+
+
+@pytest.mark.parametrize("case", CASES, ids=_ids(CASES))
+def test_backward_runs_on_matrix_cores(case):
+    from natten_amd._core import hip
+
+    assert _form("bwd", case)
+    with hip.generic_kernels():
+        assert not _form("bwd", case) and not _form("fwd", case)
+
+
+# Just outside a limit of the float32 matrix-core kernels.
+OUTSIDE = [
+    (F32, 1, (150,), 1, 1, 48, (7,), (1,), (1,), (False,)),            # head_dim
+    (F32, 1, (150,), 1, 1, 32, (8,), (1,), (1,), (False,)),            # even window
+    (F32, 1, (150,), 1, 1, 32, (7,), (2,), (3,), (False,)),            # stride and dilation
+    (F32, 1, (13, 20), 1, 1, 32, (7, 7), (2, 2), (1, 1), (False, False)),  # d K > L
+    (BF16, 1, (31,), 2, 2, 16, (5,), (1,), (2,), (False,)),            # 16 bits, head_dim 16
+    (F32, 1, (1 << 20,), 8, 8, 64, (7,), (1,), (1,), (False,)),        # 2^31 bytes a sample
+]
+
+
+@pytest.mark.parametrize("case", OUTSIDE, ids=_ids(OUTSIDE))
+def test_outside_the_limits(case):
+    for which in ("fwd", "bwd"):
+        assert not _form(which, case)
+    if case[8] == (1,) * len(case[8]):
+        for which in ("qk", "av", "qk_bwd", "av_bwd"):
+            assert not _form(which, case)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", CASES, ids=_ids(CASES))
 def test_against_oracle(case):
@@ -121,6 +159,14 @@ SPLIT = [
     (1, (5, 6, 9), 3, 1, 32, (3, 3, 5), (1, 2, 1), (False, True, False)),
     (1, (24, 24), 1, 1, 32, (21, 23), (1, 1), (False, False)),  # most slots: one wave per group
 ]
+
+
+@pytest.mark.parametrize("case", SPLIT, ids=[f"{'x'.join(map(str, c[1]))}-d{c[4]}" for c in SPLIT])
+def test_split_backward_runs_on_matrix_cores(case):
+    B, sp, H, Hkv, D, ks, dil, caus = case
+    for which in ("qk_bwd", "av_bwd"):
+        assert _form(which, (F32, B, sp, H, Hkv, D, ks, dil, (1,) * len(sp), caus))
+        assert not _form(which, (BF16, B, sp, H, Hkv, D, ks, dil, (1,) * len(sp), caus))
 
 
 @pytest.mark.gpu
@@ -187,6 +233,29 @@ BIAS = [
     (1, (19, 33), 2, 64, 5, 3),
     (3, (24, 40), 2, 32, 7, 1),    # inner tiles (no window clamped) and edges
 ]
+
+
+def _rpb_plan(B, sp, H, D, K, d, dtype):
+    import ctypes
+
+    from natten_amd._core import _lib
+
+    p = _lib.make_rpb_params(len(sp), B, H, D, sp, (K,) * len(sp), (d,) * len(sp), False, dtype, 0.3)
+    plan = _lib.NaRpbPlan()
+    assert _lib.load().na_rpb_kernel_plan(ctypes.byref(p), ctypes.byref(plan)) == 0
+    return {f: getattr(plan, f) for f, _ in plan._fields_}
+
+
+@pytest.mark.parametrize("case", BIAS, ids=[f"{'x'.join(map(str, c[1]))}-k{c[4]}d{c[5]}" for c in BIAS])
+def test_bias_plans_name_the_kernels(case):
+    from natten_amd._core import _lib
+
+    p = _rpb_plan(*case, _lib.NA_F32)
+    assert [p[f] for f in ("dq", "dk", "dattn", "dv")] == [_lib.RPB_TILE] * 4
+    assert p["fused_bias"] == (len(case[1]) == 2)  # rank 1: a pass of its own
+    assert not any(_rpb_plan(*case, _lib.NA_BF16)[f] for f in ("qk", "av", "dq", "dk", "fused_bias"))
+    B, sp, H, D, K, d = case
+    assert not any(_rpb_plan(B, sp, H, 24, K, d, _lib.NA_F32)[f] for f in ("qk", "av", "dq", "dv"))
 
 
 @pytest.mark.gpu
