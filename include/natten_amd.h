@@ -61,9 +61,10 @@ enum na_flags {
    * that breaks the promise gets wrong values in its rows (every memory
    * access stays inside the tensors). */
   NA_FLAG_VARLEN_CLAMPED = 8,
-  /* rank-2 lean kernels stage row slabs wherever they can run, whatever the
-     launch gains by it (tests of their edges on small problems) */
-  NA_FLAG_ROW_SLABS = 16
+  /* kernels chosen by a launch's size run wherever they can: row slabs of
+   * the rank-2 lean kernels, the matrix-core form of a generic forward (for
+   * tests of their edges on small problems) */
+  NA_FLAG_ANY_SIZE = 16
 };
 
 /*

@@ -70,7 +70,7 @@ int make_prob(const na_params *p, na::Prob *P, bool allow_varlen) {
   P->dense = dense ? 1 : 0;
   P->sample_extent = p->sample_extent;
   P->varlen_clamped = (p->flags & NA_FLAG_VARLEN_CLAMPED) != 0 ? 1 : 0;
-  P->row_slabs = (p->flags & NA_FLAG_ROW_SLABS) != 0 ? 1 : 0;
+  P->any_size = (p->flags & NA_FLAG_ANY_SIZE) != 0 ? 1 : 0;
   P->kprod = 1;
   const int lead = 3 - p->rank;
   for (int a = 0; a < 3; ++a) {

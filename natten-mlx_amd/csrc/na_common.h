@@ -193,7 +193,7 @@ struct Prob {
   float scale;
   const int32_t *sample_extent;  // [B, rank] or nullptr
   int32_t varlen_clamped;  // caller: d * K <= sample extent, non-causal axes
-  int32_t row_slabs;       // caller: row slabs whatever the launch gains
+  int32_t any_size;        // caller: kernels chosen by size wherever they can run
 };
 
 // Division by a divisor fixed at launch (round-up multiply method of

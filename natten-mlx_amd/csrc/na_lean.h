@@ -726,7 +726,7 @@ int box_max(const Axis &x, int t, bool inverse) {
 template <typename Ext, typename Wgs>
 void row_slabs(const Prob &P, LMode mode, const int *Ws, int nW, Ext ext, Wgs wgs_of, LChoice &C,
                double &per_wave) {
-  const bool bwd = mode == kLBwd, any = P.row_slabs != 0;
+  const bool bwd = mode == kLBwd, any = P.any_size != 0;
   auto slab = [&](const int (&Em)[3], int W) {  // rows of a slab
     return std::min(Em[1], 4 * 64 * W / (P.D / 8) / (lds_rows(2, Em) / Em[1]));
   };
@@ -1001,7 +1001,7 @@ LChoice lean_choice(const Prob &P, LMode mode) {
   key.v[n++] = P.kprod;
   key.v[n++] = P.n_extra;
   key.v[n++] = P.sample_extent != nullptr ? 1 : 0;
-  key.v[n++] = P.row_slabs;
+  key.v[n++] = P.any_size;
   key.v[n++] = P.B;
   key.v[n++] = P.H;
   key.v[n++] = P.Hkv;

@@ -463,23 +463,34 @@ bool wave_eligible(const Prob &P, int dtype) {
   return wv_geometry_ok(P, dtype == NA_F32 ? 4 : 2);
 }
 
-// The forward at head_dim 128 with strided queries: where a tile's box holds
-// many times a window's keys, the product over the box costs more than the
-// window alone on the vector ALU (K = 3 stride 3 on 4096 positions, 16 times:
-// bf16 7.5 us there, 9.8 here; float32 3 x 3 stride 2, 9 times: 16.6 and 20.4;
-// bf16 3 x 3 stride 2: 17.5 and 17.0).  Narrower heads gain at every ratio
-// (bf16 K = 3 stride 3: 5.9 -> 5.2 at head_dim 64), and so does the backward.
+// The forward where a tile's box holds many times a window's keys (few slots,
+// strided queries): the product over the box costs more than the window alone on
+// the vector ALU, the sooner the wider the head and the smaller the launch (one
+// chain of chunks per wave).  Times here over there by box over window (K = 3
+// stride 1 on one axis 6, stride 2 11, stride 3 16, 3 x 3 stride 2 9, 5 x 5 stride 3
+// 7.8) and output rows (positions times heads):
+//   float32  D 128: 5 to 8 1.03 to 1.2 up to 4e3 rows, 0.58 to 0.83 from 2.4e4 (1.01 at
+//            7e3); 9 1.0 to 1.12.  D 64: 7 to 8 at most 1.0; 9 to 11 0.96 to 1.16, 0.83 to
+//            0.87 from 8e4; 16 1.03 to 1.34.  D 16 / 32: up to 11 at most 1.0, 16 0.7 to
+//            1.15
+//   16 bits  D 128: 8 to 11 0.78 to 1.12 up to 7e3, 0.72 to 0.92 from 1.7e4; 16 1.0 to
+//            1.25.  D 32 / 64: up to 11 at most 1.0, 16 0.68 to 1.18
+// The backward gains at every ratio.
 bool wave_fwd_eligible(const Prob &P, int dtype) {
   if (!wave_eligible(P, dtype)) return false;
-  if (P.D != 128 || !strided(P)) return true;
+  if (P.any_size != 0) return true;
   int T[3] = {1, 1, 16};
   wv_tile(P, false, T);
-  int64_t pts = 1;
+  int64_t pts = 1, rows = (int64_t)P.B * P.H;
   for (int a = 3 - P.rank; a < 3; ++a) {
     const Axis &x = P.ax[a];
     pts *= std::min(phase_max(x), (T[a] - 1) * x.s + x.K);
+    rows *= x.O;
   }
-  return pts <= (int64_t)P.kprod * (dtype == NA_F32 ? 8 : 12);
+  int most = 12;
+  if (P.D == 128) most = rows < 1 << 14 ? (dtype == NA_F32 ? 5 : 7) : (dtype == NA_F32 ? 8 : 12);
+  if (P.D == 64 && dtype == NA_F32) most = rows < 1 << 16 ? 8 : 12;
+  return pts <= (int64_t)P.kprod * most;
 }
 
 #define WV_R(KERNEL, TT, DD)                       \

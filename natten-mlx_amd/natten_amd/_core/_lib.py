@@ -26,7 +26,7 @@ NA_FLAG_DENSE = 1
 NA_FLAG_GENERIC = 2
 NA_FLAG_NO_LEAN = 4
 NA_FLAG_VARLEN_CLAMPED = 8
-NA_FLAG_ROW_SLABS = 16
+NA_FLAG_ANY_SIZE = 16
 ABI_VERSION = 2
 
 _STATUS = {0: "ok", 1: "invalid argument", 2: "unsupported", 3: "launch failure",

@@ -25,7 +25,7 @@ from . import _lib
 # the generic vector-ALU kernels even where the matrix-core kernels apply.
 _force_generic = os.environ.get("NATTEN_AMD_GENERIC", "0") == "1"
 _no_lean = False
-_row_slabs = False
+_any_size = False
 
 
 @contextlib.contextmanager
@@ -54,16 +54,17 @@ def no_lean_kernels(enabled: bool = True):
 
 
 @contextlib.contextmanager
-def row_slab_kernels(enabled: bool = True):
-    """Temporarily let rank-2 problems take the lean kernels' row slabs
-    wherever they can run, also where the launch is too small to gain."""
-    global _row_slabs
-    prev = _row_slabs
-    _row_slabs = enabled
+def any_size_kernels(enabled: bool = True):
+    """Temporarily run the kernels that a launch's size decides on (row slabs,
+    the matrix-core form of a generic forward) wherever they can, also where
+    the launch is too small to gain."""
+    global _any_size
+    prev = _any_size
+    _any_size = enabled
     try:
         yield
     finally:
-        _row_slabs = prev
+        _any_size = prev
 
 
 def is_available() -> bool:
@@ -107,7 +108,7 @@ def _params_entry(q: torch.Tensor, k: torch.Tensor, kernel_size, stride, dilatio
                   sample_extent: Optional[torch.Tensor] = None, varlen_clamped: bool = False):
     flags = ((_lib.NA_FLAG_DENSE if dense else 0) | (_lib.NA_FLAG_GENERIC if _force_generic else 0)
              | (_lib.NA_FLAG_NO_LEAN if _no_lean else 0)
-             | (_lib.NA_FLAG_ROW_SLABS if _row_slabs else 0)
+             | (_lib.NA_FLAG_ANY_SIZE if _any_size else 0)
              | (_lib.NA_FLAG_VARLEN_CLAMPED if varlen_clamped and sample_extent is not None
                 else 0))
     se_ptr = None if sample_extent is None else sample_extent.data_ptr()

@@ -85,7 +85,7 @@ def _op_flags(spec: FusedSpec, sample_extent) -> int:
     return ((_lib.NA_FLAG_DENSE if spec.dense else 0)
             | (_lib.NA_FLAG_GENERIC if _hip._force_generic else 0)
             | (_lib.NA_FLAG_NO_LEAN if _hip._no_lean else 0)
-            | (_lib.NA_FLAG_ROW_SLABS if _hip._row_slabs else 0)
+            | (_lib.NA_FLAG_ANY_SIZE if _hip._any_size else 0)
             | (_lib.NA_FLAG_VARLEN_CLAMPED if spec.varlen_clamped and sample_extent is not None
                else 0))
 

@@ -48,7 +48,7 @@ CASES = [
 def test_planned_in_row_slabs(case):
     from natten_amd._core import hip
 
-    with hip.row_slab_kernels():  # small launches: see the rules below
+    with hip.any_size_kernels():  # small launches: see the rules below
         p = _plan(*case[1:], case[0], True)
     assert p["path"] == "lean" and p["slabs"] > 1, p
 
@@ -89,7 +89,7 @@ def test_slabs_where_the_launch_gains(problem, want):
 def test_row_slabs_against_oracle(case):
     from natten_amd._core import hip
 
-    with hip.row_slab_kernels():
+    with hip.any_size_kernels():
         _row_slabs_against_oracle(case)
 
 

@@ -121,6 +121,48 @@ def test_against_oracle(case):
         assert_close(t.grad, r, dtype, n)
 
 
+# Forwards that the size decides: (case, runs on matrix cores).
+SIZES = [
+    ((F32, 2, (500,), 4, 4, 128, (3,), (1,), (1,), (False,)), False),   # one chain per wave
+    ((F32, 4, (6000,), 12, 12, 128, (3,), (1,), (1,), (False,)), True),
+    ((F32, 2, (500,), 4, 4, 64, (3,), (1,), (1,), (False,)), True),
+    ((F32, 1, (67, 42), 4, 4, 64, (3, 3), (1, 1), (3, 3), (False, False)), False),  # 16 boxes
+    ((F32, 1, (100, 100), 4, 4, 64, (3, 3), (1, 1), (2, 2), (False, False)), False),
+    ((F32, 8, (200, 200), 8, 8, 64, (3, 3), (1, 1), (2, 2), (False, False)), True),
+    ((BF16, 1, (59, 90), 4, 4, 128, (3, 3), (1, 1), (2, 2), (False, False)), False),
+    ((BF16, 4, (57, 75), 4, 4, 64, (7, 7), (1, 1), (2, 2), (False, False)), True),
+    ((F32, 2, (61, 45), 8, 8, 32, (7, 7), (1, 1), (1, 1), (False, False)), True),
+]
+
+
+@pytest.mark.parametrize("case,runs", SIZES, ids=_ids([c for c, _ in SIZES]))
+def test_forward_by_size(case, runs):
+    from natten_amd._core import hip
+
+    assert _form("fwd", case) == runs
+    with hip.any_size_kernels():
+        assert _form("fwd", case)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES, ids=_ids(CASES))
+def test_forward_at_any_size(case):
+    """The forward of every case on matrix cores, also where its size would
+    choose the vector ALU."""
+    import natten_amd
+    from natten_amd._core import hip
+
+    dtype, B, sp, H, Hkv, D, ks, dil, st, caus = case
+    print(f"[case] wave forward {case}", flush=True)
+    q, k, v = (randn((B, *sp, h, D), dtype, i) for i, h in enumerate((H, Hkv, Hkv)))
+    with hip.any_size_kernels():
+        assert _form("fwd", case)
+        out, lse = hip.fused_forward(q.to(DEV), k.to(DEV), v.to(DEV), ks, st, dil, caus, 0.3)
+    ro, rl = O.na_functional(q, k, v, ks, st, dil, caus, 0.3, return_lse=True)
+    assert_close(out, ro, dtype, "out")
+    assert_close(lse, rl, F32, "lse", scale_tol=1.0 if dtype == F32 else 4.0)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("where", ["q", "k", "v", "grad"])
 @pytest.mark.parametrize("bad", [float("nan"), float("inf")], ids=str)
