@@ -541,21 +541,30 @@ Prob rpb_prob(const RpbProb &A) {
 }  // namespace
 
 // Where a window has few slots, a tile's 16-point chunks are mostly points of
-// no window and the vector ALU's one pass over the window is shorter.  The
-// forward passes, float32, microseconds there -> here (sizes [2, 4096, 4, D],
-// [4, 80, 80, 8, D] and [1, 14, 14, 2, D]):
-//   QK   3 slots, D 32 / 64: 5.1 -> 6.6, 7.4 -> 7.8; 9 slots, D 16 / 32: 18.0
-//        -> 22.5, 30.9 -> 27.4; 7 slots, D 32 / 64: 7.2 -> 7.0, 11.8 -> 8.3;
-//        13 slots, D 16: 7.9 -> 6.6; 25 slots, D 16: 62.5 -> 25.7
-//   AV   9 slots, D 32 / 64: 26.2 -> 29.1, 42.5 -> 42.3 (4.6 -> 7.5 on the
-//        small one); 13 slots, D 32 / 64: 7.2 -> 7.5, 12.2 -> 9.4; 25 slots,
-//        D 16 / 32: 39.2 -> 27.8, 7.8 -> 7.1
-// A backward call's two passes gain from 3 slots on (15.0 -> 9.4, 10.8 -> 7.6).
+// no window and the vector ALU's one pass over the window is shorter; and a
+// small launch is one chain of chunks (load, LDS, product), the longer the wider
+// the head.  Times here over there, float32, by slots, head_dim and rows (queries
+// times heads):
+//   QK   3 slots, D 128: 1.34 to 1.50 up to 4.4e3 rows, 0.7 to 0.8 from 3e4; 5 slots,
+//        D 64 / 128: 1.07 to 1.25, 0.5 to 0.8; 7 and 9 slots: D 32 0.81 to 1.01, D 64
+//        0.42 to 0.97, D 128 up to 1.08 below 1e3 rows, 0.35 to 0.98 above; D 16 up to
+//        9 slots 1.2; from 13 slots on 0.12 to 0.91
+//   AV   13 to 27 slots, D 64 / 128: 1.04 to 1.54 up to 5e3 rows, 0.25 to 0.79 from
+//        1.6e4; 31 to 49 slots, D 128: 0.95 to 1.07, 0.2 to 0.5; 25 slots, D 16 / 32: 0.58
+//        to 1.02; otherwise 0.15 to 0.99.  9 slots lose (D 32 / 64: 26.2 -> 29.1 us, 4.6
+//        -> 7.5 on a small one)
+// A backward call's two passes gain from 3 slots on at every size (0.1 to 0.7).
+constexpr int64_t kFilled = 1 << 14;  // rows that fill the chip: four waves per CU
+
 bool wsplit_eligible(const Prob &P, int dtype, WsplitPass pass) {
   const int kk = P.kprod;
-  const bool gains = pass == kWsQk   ? kk >= 13 || kk * P.D >= 224
-                     : pass == kWsAv ? kk >= 25 || (kk >= 13 && P.D >= 64)
-                                     : kk >= 3;
+  const int64_t rows = (int64_t)P.B * P.H * P.ax[0].L * P.ax[1].L * P.ax[2].L;
+  bool gains = kk >= 3;
+  if (pass == kWsQk)
+    gains = kk >= 13 || (kk >= 7 ? P.D >= 32 && (P.D < 128 || rows >= kFilled / 4)
+                                 : kk * P.D >= 224 && rows >= kFilled);
+  if (pass == kWsAv)
+    gains = P.D < 64 ? kk >= 25 : kk >= (rows >= kFilled ? 13 : P.D == 64 ? 31 : 49);
   return dtype == NA_F32 && gains && ws_ok(P);
 }
 
@@ -587,12 +596,27 @@ void wsplit_av_bwd(const Prob &P, const void *attn, const void *v, const void *d
 }
 
 // Rank 1 up to head_dim 16 has kernels of its own (na_rpb.hip) that stage
-// whole blocks of rows.  The logits as the split QK above (9 slots, D 16 / 32:
-// 22.9 -> 27.2, 39.4 -> 33.9); the generic AV and backward kernels lose from 7
-// slots on (AV, 9 slots, D 16 / 32: 24.7 -> 25.2, 40.3 -> 29.0; rank 1, 7
-// slots, [6, 6000, 12, 32]: 65.5 -> 43.7), not at 3 (26.2 -> 42.5).
+// whole blocks of rows.  Times here over there (the generic kernels), by slots,
+// head_dim and rows:
+//   logits, dattn alone   rank 1: 3 and 5 slots, D 64 / 128 0.95 to 1.5; 7 slots 0.65 to
+//        1.4; 9 slots, D 32 / 128 0.57 to 1.0, D 64 0.6 to 1.11; rank 2, 9 slots, D 32
+//        0.80 to 0.86, but 1.08 at 4e4 rows, D 64 / 128 0.79 to 0.98
+//   AV, dq alone          7 slots 0.7 to 1.54; 9 slots 0.89 to 1.26 up to 5e4 rows (D 16
+//        1.18 at 3e5), 0.57 to 0.81 from 2.4e5 with D 32 and more
+// and from 13 slots on 0.08 to 0.92 for every pass, but at rank 1 with up to four
+// heads, whose rows lie closer together for the generic kernels, 1.04 to 1.4 at 9 to
+// 25 slots from 3e4 rows on (AV of head_dim 128 at any), 0.3 to 0.6 at 31.  A
+// backward call's two passes together gain from 7 slots on at every size (0.1 to
+// 0.84).
 bool wsplit_rpb_eligible(const RpbProb &A, WsplitPass pass) {
-  const bool gains = pass == kWsQk ? A.KK >= 13 || A.KK * A.D >= 224 : A.KK >= 7;
+  const int64_t rows = (int64_t)A.n_rows;
+  bool gains = A.KK >= 7;
+  if (pass == kWsQk)
+    gains = A.KK >= 13 || (A.KK >= 9 && (A.rank == 1 ? A.D != 64
+                                                     : A.D >= 64 || (A.D == 32 && (rows < kFilled ||
+                                                                                   rows >= 8 * kFilled))));
+  if (pass == kWsAv) gains = A.KK >= 13 || (A.KK >= 9 && A.D >= 32 && rows >= 8 * kFilled);
+  if (pass != kWsBwd && A.rank == 1 && A.H <= 4) gains = A.KK >= 31;
   return gains && (A.rank == 2 || A.D > 16) && A.n_rows > 0 && ws_ok(rpb_prob(A));
 }
 

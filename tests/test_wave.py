@@ -200,7 +200,40 @@ SPLIT = [
     (2, (8, 13), 4, 2, 16, (3, 7), (2, 1), (True, False)),
     (1, (5, 6, 9), 3, 1, 32, (3, 3, 5), (1, 2, 1), (False, True, False)),
     (1, (24, 24), 1, 1, 32, (21, 23), (1, 1), (False, False)),  # most slots: one wave per group
+    (1, (60,), 2, 1, 128, (51,), (1,), (True,)),               # AV of a wide head
 ]
+
+# Split and position-bias forwards by size: (spatial, B, H, D, kernel) and what runs
+# on matrix cores of QK, AV, and of the logits and AV with position bias.
+FWD = [
+    (((500,), 2, 4, 128, 3), (False, False, False, False)),
+    (((6000,), 4, 10, 128, 3), (True, False, False, False)),
+    (((500,), 2, 4, 64, 5), (False, False, False, False)),
+    (((6000,), 4, 10, 32, 7), (True, False, False, False)),
+    (((600,), 2, 5, 128, 9), (True, False, True, False)),
+    (((6000,), 6, 12, 32, 9), (True, False, True, True)),
+    (((500,), 2, 5, 64, 13), (True, False, True, True)),
+    (((500,), 2, 4, 64, 13), (True, False, False, False)),  # few heads, one axis
+    (((500,), 2, 4, 64, 31), (True, True, True, True)),
+    (((6000,), 4, 10, 64, 13), (True, True, True, True)),
+    (((40, 40), 4, 5, 32, 3), (True, False, False, False)),
+    (((24, 24), 2, 4, 32, 3), (True, False, True, False)),
+    (((40, 40), 4, 5, 16, 5), (True, True, True, True)),
+    (((14, 14), 1, 2, 128, 5), (True, False, True, True)),
+    (((56, 56), 4, 2, 32, 7), (True, True, True, True)),
+]
+
+
+@pytest.mark.parametrize("problem,want", FWD, ids=[f"{c}" for c, _ in FWD])
+def test_split_forwards_by_size(problem, want):
+    from natten_amd._core import _lib
+
+    sp, B, H, D, K = problem
+    one = (1,) * len(sp)
+    case = (F32, B, sp, H, H, D, (K,) * len(sp), one, one, (False,) * len(sp))
+    p = _rpb_plan(B, sp, H, D, K, 1, _lib.NA_F32)
+    assert (_form("qk", case), _form("av", case), p["qk"] == _lib.RPB_TILE,
+            p["av"] == _lib.RPB_TILE) == want
 
 
 @pytest.mark.parametrize("case", SPLIT, ids=[f"{'x'.join(map(str, c[1]))}-d{c[4]}" for c in SPLIT])
