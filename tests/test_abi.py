@@ -125,6 +125,29 @@ def test_validation_messages_match_reference():
         natten_amd.na1d_varlen(q, q, q, torch.tensor([2], dtype=torch.int32), kernel_size=3)
 
 
+@pytest.mark.parametrize("bad", [7.0, np.int64(7), (7, 7.0), (np.int32(7), 7)], ids=repr)
+@pytest.mark.parametrize("what", ["kernel_size", "stride", "dilation"])
+def test_refused_arguments_stay_refused_after_equal_ones(what, bad):
+    """7, 7.0 and numpy's 7 are equal and hash alike: a call that validation
+    refuses does not pass once the same call with ints has run."""
+    import natten_amd
+    from natten_amd import functional as F
+
+    q = torch.randn(1, 49, 49, 2, 4)
+    attn = torch.randn(1, 49, 49, 2, 49)
+    small = torch.randn(1, 7, 7, 2, 49)
+    calls = [lambda **k: natten_amd.na2d(q, q, q, **k), lambda **k: F.na2d_qk(q, q, **k),
+             lambda **k: F.na2d_av(small if what == "stride" else attn, q, **k)]
+    for call in calls:
+        for value in (7, (7, 7)):
+            with pytest.raises(RuntimeError, match="HIP"):  # valid: no CPU implementation
+                call(**{"kernel_size": 7, what: value})
+        with pytest.raises(ValueError, match="must be int"):
+            call(**{"kernel_size": 7, what: bad})
+        with pytest.raises(RuntimeError, match="HIP"):
+            call(**{"kernel_size": 7, what: [7, 7]})
+
+
 def test_backend_registry():
     import natten_amd
 
