@@ -343,7 +343,7 @@ constexpr int wv_rs() {
 // ---------------------------------------------------------------------------
 // Host side.
 
-int phase_max(const Axis &x) { return (x.L + x.d - 1) / x.d; }
+int phase_max(const Axis &x) { return (int)(((int64_t)x.L + x.d - 1) / x.d); }
 
 // Tile extents (product 16) with the fewest chunks over the grid.
 void wv_tile(const Prob &P, bool keys, int T[3]) {
@@ -428,6 +428,31 @@ WvProb make_wvprob(const Prob &P, bool backward, int waves) {
   return W;
 }
 
+// The launch of both grids (a backward's two passes) holds fewer than 2^32
+// threads: ragged phases (three points of 16 rows each, or d > L on a causal axis)
+// take up to a wave per point.
+bool wv_launch_ok(const Prob &P) {
+  constexpr int64_t most = ((int64_t)1 << 32) / 64 - 64;  // waves, the last workgroups' apart
+  auto points = [&](int a) { return (int64_t)P.ax[a].d * phase_max(P.ax[a]); };
+  if (points(0) >= most || points(1) >= most || points(2) >= most) return false;
+  // every tile holds a point: far below the limit without the tiles
+  const double all = (double)P.B * P.H * points(0) * points(1) * points(2);
+  if (2.0 * all < (double)most) return true;
+  double waves = 0.0;
+  for (int keys = 0; keys < 2; ++keys) {
+    int T[3] = {1, 1, 16};
+    wv_tile(P, keys != 0, T);
+    double n = (double)P.B * (keys ? P.Hkv : P.H);
+    for (int a = 0; a < 3; ++a) {
+      const Axis &x = P.ax[a];
+      const int len = keys || x.s == 1 ? phase_max(x) : x.O;
+      n *= (double)x.d * ((len + T[a] - 1) / T[a]);
+    }
+    waves += n;
+  }
+  return waves < (double)most;
+}
+
 // Window rules, box sizes and index arithmetic of the wave kernels, for rows
 // of `es`-byte elements.
 bool wv_geometry_ok(const Prob &P, int64_t es) {
@@ -448,7 +473,7 @@ bool wv_geometry_ok(const Prob &P, int64_t es) {
   // 32-bit byte offsets inside a sample, 32-bit tile numbers
   const int64_t tokens = (int64_t)P.ax[0].L * P.ax[1].L * P.ax[2].L;
   if (tokens * std::max(P.H, P.Hkv) * P.D * es >= ((int64_t)1 << 31)) return false;
-  return (int64_t)P.B * P.H * tokens < ((int64_t)1 << 30);
+  return (int64_t)P.B * P.H * tokens < ((int64_t)1 << 30) && wv_launch_ok(P);
 }
 
 }  // namespace

@@ -88,6 +88,26 @@ OUTSIDE = [
 ]
 
 
+# Ragged phases: three points of a tile's 16 rows each.  Both grids of a backward
+# hold 64 threads per tile; below and above 2^32 of them.
+@pytest.mark.parametrize("B,runs", [(4, True), (5, False)])
+def test_launches_stay_below_2_32_threads(B, runs):
+    L, d = 24_000_000, 8_000_000
+    assert (2 * B * d * 64 < 1 << 32) == runs
+    case = (F32, B, (L,), 1, 1, 16, (3,), (d,), (1,), (False,))
+    for which in ("bwd", "qk_bwd", "av_bwd"):
+        assert _form(which, case) == runs
+
+
+def test_causal_dilation_past_the_extent():
+    """A causal axis of d > L has d phases, most of them empty (the C interface
+    takes it): run while the launch holds them, and no overflow past that."""
+    for d, runs in ((1000, True), (1 << 20, True), (1 << 25, False), ((1 << 31) - 1, False)):
+        case = (F32, 1, (50,), 1, 1, 32, (7,), (d,), (1,), (True,))
+        for which in ("fwd", "bwd", "qk", "qk_bwd"):
+            assert _form(which, case) == runs, (d, which)
+
+
 @pytest.mark.parametrize("case", OUTSIDE, ids=_ids(OUTSIDE))
 def test_outside_the_limits(case):
     for which in ("fwd", "bwd"):
