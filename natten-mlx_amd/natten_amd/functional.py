@@ -21,7 +21,6 @@ additional-token merge on the neighborhood path, where it is float32
 
 from __future__ import annotations
 
-import marshal
 from typing import Optional, Tuple, Union
 
 import torch
@@ -114,17 +113,34 @@ def _is_full_attention(kernel_size: tuple, spatial_shape: tuple) -> bool:
 # Validated specs by call signature (shapes, dtypes and the arguments as
 # passed): a training loop calls with the same few signatures every step,
 # and the checks and tuple normalisation cost more host time than the rest
-# of the call.  Only successful validations are stored.
+# of the call.  Only successful validations are stored; unhashable arguments
+# (lists) are validated on every call.  An entry keeps the validated kernel size,
+# stride and dilation: 7, 7.0 and numpy's 7 are equal and hash alike, but only the
+# first is valid, so a call finds its spec if it passes these objects again, or
+# ints.
 _spec_cache: dict = {}
 _SPEC_MAX = 512
 
 
-def _args_key(*args) -> bytes:
-    """The arguments' values with their types: 7, 7.0 and numpy's 7 are equal and
-    hash alike, but validation takes only the first (marshal in version 2: no
-    references, so equal arguments give equal bytes; 0.2 us, against 0.5 for the
-    types of each value).  ValueError for types it does not know."""
-    return marshal.dumps(args, 2)
+def _ints(*args) -> bool:
+    for a in args:
+        for v in a if isinstance(a, tuple) else (a,):
+            if not isinstance(v, int):
+                return False
+    return True
+
+
+def _kept_spec(key, ks, st, dil):
+    e = _spec_cache.get(key)
+    if e is not None and (e[1] is ks and e[2] is st and e[3] is dil or _ints(ks, st, dil)):
+        return e[0]
+    return None
+
+
+def _keep_spec(key, spec, ks, st, dil) -> None:
+    if len(_spec_cache) >= _SPEC_MAX:
+        _spec_cache.clear()
+    _spec_cache[key] = (spec, ks, st, dil)
 
 
 def _fused_spec(rank, query, key, value, kernel_size, stride, dilation, is_causal, scale,
@@ -158,22 +174,27 @@ def _packed_spec(rank, shape, qkv, kernel_size, stride, dilation, is_causal, sca
         return _fused_spec(rank, part, part, part, kernel_size, stride, dilation, is_causal,
                            scale, None, None)
 
-    return _cached_spec(("qkv", rank, shape), (kernel_size, stride, dilation, is_causal, scale),
+    return _cached_spec(("qkv", rank, shape, scale), kernel_size, stride, dilation, is_causal,
                         make)
 
 
 def _na(rank, query, key, value, kernel_size, stride, dilation, is_causal, scale, return_lse,
         additional_keys, additional_values):
     add = additional_keys is not None or additional_values is not None
-    extra = None
-    if add:
-        extra = tuple(None if t is None else (t.shape, t.dtype)
-                      for t in (additional_keys, additional_values))
-    spec = _cached_spec(
-        ("na", rank, query.shape, key.shape, value.shape, query.dtype, key.dtype, value.dtype,
-         extra), (kernel_size, stride, dilation, is_causal, scale),
-        lambda: _fused_spec(rank, query, key, value, kernel_size, stride, dilation, is_causal,
-                            scale, additional_keys, additional_values))
+    try:
+        ck = (rank, query.shape, key.shape, value.shape, query.dtype, key.dtype, value.dtype,
+              kernel_size, stride, dilation, is_causal, scale,
+              (None if additional_keys is None else (additional_keys.shape, additional_keys.dtype),
+               None if additional_values is None
+               else (additional_values.shape, additional_values.dtype)) if add else None)
+        spec = _kept_spec(ck, kernel_size, stride, dilation)
+    except TypeError:  # an unhashable argument
+        ck = spec = None
+    if spec is None:
+        spec = _fused_spec(rank, query, key, value, kernel_size, stride, dilation, is_causal,
+                           scale, additional_keys, additional_values)
+        if ck is not None:
+            _keep_spec(ck, spec, kernel_size, stride, dilation)
     add_k, add_v = additional_keys, additional_values
     if add:
         if add_k.dtype != query.dtype:
@@ -246,21 +267,18 @@ def _split_spec(spatial, rank, kernel_size, dilation, stride, is_causal):
     return tuple(ks), tuple(st), tuple(dil), tuple(bool(c) for c in caus)
 
 
-def _cached_spec(key, args, make):
-    """``make()``, kept by call signature (``key`` and the arguments as passed)
-    as the fused op's specs are."""
+def _cached_spec(key, ks, st, dil, caus, make):
+    """``make()``, kept by call signature as the fused op's specs are."""
     if torch.compiler.is_compiling():
         return make()
+    key = (*key, ks, st, dil, caus)
     try:
-        key = (*key, _args_key(*args))
-    except ValueError:  # an argument without a key
+        spec = _kept_spec(key, ks, st, dil)
+    except TypeError:  # an unhashable argument
         return make()
-    spec = _spec_cache.get(key)
     if spec is None:
         spec = make()
-        if len(_spec_cache) >= _SPEC_MAX:
-            _spec_cache.clear()
-        _spec_cache[key] = spec
+        _keep_spec(key, spec, ks, st, dil)
     return spec
 
 
@@ -270,14 +288,14 @@ def _qk(rank, query, key, kernel_size, dilation, stride, is_causal, scale, fn):
         return _split_spec(tuple(query.shape[1:-2]), rank, kernel_size, dilation, stride,
                            is_causal)
 
-    ks, st, dil, caus = _cached_spec(("qk", rank, query.shape, key.shape),
-                                     (kernel_size, dilation, stride, is_causal), make)
+    ks, st, dil, caus = _cached_spec(("qk", rank, query.shape, key.shape), kernel_size, stride,
+                                     dilation, is_causal, make)
     return fn(query, key, ks, st, dil, caus, scale)
 
 
 def _av(rank, attn, value, kernel_size, dilation, stride, is_causal, fn):
     ks, st, dil, caus = _cached_spec(
-        ("av", rank, attn.shape, value.shape), (kernel_size, dilation, stride, is_causal),
+        ("av", rank, attn.shape, value.shape), kernel_size, stride, dilation, is_causal,
         lambda: _av_spec(rank, attn, value, kernel_size, dilation, stride, is_causal))
     return fn(attn, value, ks, st, dil, caus)
 
