@@ -46,6 +46,16 @@ void check_device(const at::Tensor &t) {
               t.device(), ". There is no CPU implementation.");
 }
 
+// `t` is on `q`'s device (checked after the shapes: a mismatched call raises
+// the same wherever its tensors are).
+void check_devices(const at::Tensor &q, std::initializer_list<const at::Tensor *> others) {
+  check_device(q);
+  for (const at::Tensor *t : others)
+    if (t->defined())
+      TORCH_CHECK(t->device() == q.device(), "tensors are on different devices: ", q.device(),
+                  " and ", t->device());
+}
+
 int32_t dtype_code(at::ScalarType s) {
   switch (s) {
     case at::kFloat:
@@ -74,6 +84,9 @@ na_params make_params(const at::Tensor &q, const at::Tensor &k, at::IntArrayRef 
   TORCH_CHECK((int64_t)kernel.size() == rank && (int64_t)stride.size() == rank &&
                   (int64_t)dilation.size() == rank && (int64_t)causal.size() == rank,
               "natten_amd: per-axis parameters must have one entry per spatial axis");
+  for (int64_t a = 0; a < rank; ++a)
+    TORCH_CHECK(kernel[a] > 0 && stride[a] > 0 && dilation[a] > 0,
+                "natten_amd: kernel, stride and dilation must be positive");
   na_params p{};
   p.rank = (int32_t)rank;
   p.batch = (int32_t)q.size(0);
@@ -250,9 +263,8 @@ struct FusedQKV : public torch::autograd::Function<FusedQKV> {
                                at::IntArrayRef stride, at::IntArrayRef dilation,
                                at::IntArrayRef causal, double scale, int64_t flags,
                                int64_t stream) {
-    check_device(qkv);
-    TORCH_CHECK(qkv.dim() >= 5 && qkv.size(-3) == 3,
-                "natten_amd na_fused_qkv: qkv is [B, *spatial, 3, H, D]");
+    TORCH_CHECK(qkv.dim() >= 5 && qkv.dim() <= 7 && qkv.size(-3) == 3,
+                "natten_amd na_fused_qkv: qkv is [B, *spatial, 3, H, D], got ", qkv.sizes());
     qkv = qkv.contiguous();
     std::vector<int64_t> sz(qkv.sizes().begin(), qkv.sizes().end());
     const int64_t row = qkv.size(-1) * qkv.size(-2) * (int64_t)qkv.element_size();
@@ -261,11 +273,12 @@ struct FusedQKV : public torch::autograd::Function<FusedQKV> {
     all.insert(all.begin(), 3);
     const int64_t tokens = row > 0 ? (int64_t)(qkv.numel() * qkv.element_size() / (3 * row)) : 0;
     at::Tensor parts = at::empty(all, qkv.options());
-    check_rc(na_pack3(1, tokens, row, qkv.data_ptr(), parts.data_ptr(), reinterpret_cast<void *>(stream)),
-             "na_pack3");
     const at::Tensor q = parts.select(0, 0), k = parts.select(0, 1), v = parts.select(0, 2);
     const na_params p =
         make_params(q, k, kernel, stride, dilation, causal, scale, 0, flags, at::Tensor());
+    check_device(qkv);
+    check_rc(na_pack3(1, tokens, row, qkv.data_ptr(), parts.data_ptr(), as_stream(stream)),
+             "na_pack3");
     for (size_t a = 0; a < kernel.size(); ++a) sz[1 + a] = (sz[1 + a] + stride[a] - 1) / stride[a];
     at::Tensor out = at::empty(sz, qkv.options());
     sz.pop_back();
@@ -315,8 +328,8 @@ at::Tensor na_fused_qkv(const at::Tensor &qkv, at::IntArrayRef kernel, at::IntAr
 }
 
 // ---- split ops (autograd/split.py) ----------------------------------------
-// The caller has validated shapes (functional.py) and passes tensors of
-// supported dtypes on one device.
+// The functional layer has validated the call; its shape rules are restated for
+// direct callers of the operators, whose kernels index by these sizes.
 
 std::vector<int64_t> split_sizes(const at::Tensor &x, at::IntArrayRef stride, int64_t last) {
   std::vector<int64_t> sz(x.sizes().begin(), x.sizes().end());
@@ -340,13 +353,17 @@ struct SplitQK : public torch::autograd::Function<SplitQK> {
                             at::IntArrayRef kernel, at::IntArrayRef stride,
                             at::IntArrayRef dilation, at::IntArrayRef causal, double scale,
                             int64_t flags, int64_t stream) {
-    check_device(q);
-    check_device(k);
+    TORCH_CHECK(q.dim() == k.dim() && q.dim() >= 4 && q.dim() <= 6 &&
+                    q.sizes().slice(0, q.dim() - 2) == k.sizes().slice(0, q.dim() - 2) &&
+                    q.size(-1) == k.size(-1) && k.size(-2) > 0 && q.size(-2) % k.size(-2) == 0,
+                "natten_amd na_split_qk: q [B, *spatial, H, D], k [B, *spatial, H_kv, D], got ",
+                q.sizes(), " and ", k.sizes());
+    const na_params p =
+        make_params(q, k, kernel, stride, dilation, causal, scale, 0, flags, at::Tensor());
+    check_devices(q, {&k});
     const auto kd = k.scalar_type();
     q = q.contiguous();
     k = to_type(k, q.scalar_type()).contiguous();
-    const na_params p =
-        make_params(q, k, kernel, stride, dilation, causal, scale, 0, flags, at::Tensor());
     at::Tensor logits = at::empty(split_sizes(q, stride, product(kernel)), q.options());
     check_rc(na_qk_fwd(&p, q.data_ptr(), k.data_ptr(), logits.data_ptr(), as_stream(stream)),
              "na_qk_fwd");
@@ -374,13 +391,19 @@ struct SplitAV : public torch::autograd::Function<SplitAV> {
   static at::Tensor forward(AutogradContext *ctx, at::Tensor attn, at::Tensor v,
                             at::IntArrayRef kernel, at::IntArrayRef stride,
                             at::IntArrayRef dilation, at::IntArrayRef causal, int64_t stream) {
-    check_device(attn);
-    check_device(v);
     const auto ad = attn.scalar_type(), vd = v.scalar_type();
     const auto dt = at::promote_types(ad, vd);
+    na_params p = make_params(v, v, kernel, stride, dilation, causal, 1.0, 0, 0, at::Tensor());
+    p.dtype = dtype_code(dt);
+    std::vector<int64_t> want = split_sizes(v, stride, product(kernel));
+    if (attn.dim() == v.dim()) want[want.size() - 2] = attn.size(-2);
+    TORCH_CHECK(attn.sizes() == at::IntArrayRef(want) && v.size(-2) > 0 &&
+                    attn.size(-2) % v.size(-2) == 0,
+                "natten_amd na_split_av: attn is [B, *ceil(spatial / stride), H, slots] for v "
+                "[B, *spatial, H_kv, D], got ", attn.sizes(), " and ", v.sizes());
+    check_devices(attn, {&v});
     attn = to_type(attn, dt).contiguous();
     v = to_type(v, dt).contiguous();
-    na_params p = make_params(v, v, kernel, stride, dilation, causal, 1.0, 0, 0, at::Tensor());
     p.heads = (int32_t)attn.size(-2);
     std::vector<int64_t> osz(attn.sizes().begin(), attn.sizes().end());
     osz.back() = v.size(-1);
@@ -416,6 +439,8 @@ na_rpb_params make_rpb(const at::Tensor &x, at::IntArrayRef kernel, at::IntArray
   TORCH_CHECK((rank == 1 || rank == 2) && (int64_t)kernel.size() == rank &&
                   (int64_t)dilation.size() == rank,
               "natten_amd: a rank-1 or rank-2 tensor with one kernel and dilation per axis");
+  for (int64_t a = 0; a < rank; ++a)
+    TORCH_CHECK(kernel[a] > 0 && dilation[a] > 0, "natten_amd: kernel and dilation must be positive");
   na_rpb_params p{};
   p.rank = (int32_t)rank;
   p.batch = (int32_t)x.size(0);
@@ -436,19 +461,26 @@ na_rpb_params make_rpb(const at::Tensor &x, at::IntArrayRef kernel, at::IntArray
 at::Tensor f32(const at::Tensor &t) { return to_type(t, at::kFloat).contiguous(); }
 
 struct RpbQK : public torch::autograd::Function<RpbQK> {
-  // rpb: float [H, 2K-1] (rank 2: [H, 2K0-1, 2K1-1]) or absent, checked by
-  // the caller, as q's and k's equal shapes are
+  // rpb: float [H, 2K-1] (rank 2: [H, 2K0-1, 2K1-1]) or absent
   static at::Tensor forward(AutogradContext *ctx, at::Tensor q, at::Tensor k,
                             std::optional<at::Tensor> rpb_opt, at::IntArrayRef kernel,
                             at::IntArrayRef dilation, double scale, bool has_scale,
                             bool heads_first, int64_t stream) {
     const at::Tensor rpb = rpb_opt.value_or(at::Tensor());
-    for (const at::Tensor *t : std::initializer_list<const at::Tensor *>{&q, &k, &rpb})
-      check_device(*t);
+    const na_rpb_params p = make_rpb(q, kernel, dilation, scale, has_scale, heads_first);
+    TORCH_CHECK(q.sizes() == k.sizes(), "natten_amd na_rpb_qk: q and k must have identical shapes, "
+                "got ", q.sizes(), " and ", k.sizes());
+    if (rpb.defined()) {
+      std::vector<int64_t> want{p.heads};
+      for (const int64_t x : kernel) want.push_back(2 * x - 1);
+      TORCH_CHECK(rpb.is_floating_point() && rpb.sizes() == at::IntArrayRef(want),
+                  "natten_amd na_rpb_qk: rpb must have shape ", at::IntArrayRef(want), ", got ",
+                  rpb.sizes());
+    }
+    check_devices(q, {&k, &rpb});
     const auto kd = k.scalar_type();
     q = q.contiguous();
     k = to_type(k, q.scalar_type()).contiguous();
-    const na_rpb_params p = make_rpb(q, kernel, dilation, scale, has_scale, heads_first);
     const at::Tensor bias = rpb.defined() ? f32(rpb) : rpb;
     std::vector<int64_t> osz(q.sizes().begin(), q.sizes().end());
     osz.back() = product(kernel);
@@ -496,12 +528,15 @@ struct RpbAV : public torch::autograd::Function<RpbAV> {
   static at::Tensor forward(AutogradContext *ctx, at::Tensor attn, at::Tensor v,
                             at::IntArrayRef kernel, at::IntArrayRef dilation, bool heads_first,
                             bool out_f32, int64_t stream) {
-    check_device(attn);
-    check_device(v);
+    const na_rpb_params p = make_rpb(v, kernel, dilation, 1.0, false, heads_first);
+    std::vector<int64_t> want(v.sizes().begin(), v.sizes().end());
+    want.back() = product(kernel);
+    TORCH_CHECK(attn.sizes() == at::IntArrayRef(want), "natten_amd na_rpb_av: attn must have shape ",
+                at::IntArrayRef(want), ", got ", attn.sizes());
+    check_devices(v, {&attn});
     const auto ad = attn.scalar_type();
     v = v.contiguous();
     attn = f32(attn);
-    const na_rpb_params p = make_rpb(v, kernel, dilation, 1.0, false, heads_first);
     at::Tensor out =
         at::empty(v.sizes(), out_f32 ? v.options().dtype(at::kFloat) : v.options());
     check_rc(na_rpb_av_fwd(&p, static_cast<const float *>(attn.data_ptr()), v.data_ptr(),
@@ -540,8 +575,13 @@ struct RpbAV : public torch::autograd::Function<RpbAV> {
 struct Linear : public torch::autograd::Function<Linear> {
   static at::Tensor forward(AutogradContext *ctx, at::Tensor x, at::Tensor w,
                             std::optional<at::Tensor> b, int64_t stream) {
-    check_device(x);
-    check_device(w);
+    TORCH_CHECK(x.dim() >= 1 && w.dim() == 2 && x.size(-1) == w.size(1) &&
+                    (!b.has_value() || (b->dim() == 1 && b->size(0) == w.size(0))),
+                "natten_amd na_linear: x [..., k], weight [n, k], bias [n], got ", x.sizes(),
+                " and ", w.sizes());
+    dtype_code(x.scalar_type());  // one the backward knows
+    const at::Tensor bias = b.value_or(at::Tensor());
+    check_devices(x, {&w, &bias});
     ctx->save_for_backward({x, w});
     ctx->saved_data["p"] = std::vector<int64_t>{stream, b.has_value() ? 1 : 0};
     return at::linear(x, w, b);

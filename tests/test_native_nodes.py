@@ -127,6 +127,59 @@ def test_nodes_hooks_streams_and_capture(case):
         step()
 
 
+def _ops():
+    from natten_amd._core import _lib
+
+    _lib.load()
+    return torch.ops.natten_amd
+
+
+# Direct calls of the operators on CPU tensors: (operator, arguments, message).  The
+# shapes are checked on the host before the device is.
+_z = torch.zeros
+_HIP = "HIP"
+DIRECT = [
+    ("na_split_qk", (_z(1, 9, 9, 4, 32), _z(1, 9, 9, 2, 32), [3, 3], [1, 1], [1, 1], [0, 0], 1.0, 0), _HIP),
+    ("na_split_qk", (_z(1, 9, 9, 4, 32), _z(1, 9, 8, 2, 32), [3, 3], [1, 1], [1, 1], [0, 0], 1.0, 0), "q .B"),
+    ("na_split_qk", (_z(2, 9, 9, 4, 32), _z(1, 9, 9, 4, 32), [3, 3], [1, 1], [1, 1], [0, 0], 1.0, 0), "q .B"),
+    ("na_split_qk", (_z(1, 9, 9, 4, 32), _z(1, 9, 9, 3, 32), [3, 3], [1, 1], [1, 1], [0, 0], 1.0, 0), "q .B"),
+    ("na_split_qk", (_z(1, 9, 9, 4, 32), _z(1, 9, 9, 4, 16), [3, 3], [1, 1], [1, 1], [0, 0], 1.0, 0), "q .B"),
+    ("na_split_qk", (_z(1, 9, 9, 4, 32), _z(1, 9, 4, 32), [3, 3], [1, 1], [1, 1], [0, 0], 1.0, 0), "q .B"),
+    ("na_split_qk", (_z(1, 9, 9, 4, 32), _z(1, 9, 9, 4, 32), [3], [1], [1], [0], 1.0, 0), "per spatial axis"),
+    ("na_split_qk", (_z(1, 9, 9, 4, 32), _z(1, 9, 9, 4, 32), [3, 3], [1, 0], [1, 1], [0, 0], 1.0, 0), "positive"),
+    ("na_split_av", (_z(1, 5, 9, 4, 9), _z(1, 9, 9, 2, 32), [3, 3], [2, 1], [1, 1], [0, 0]), _HIP),
+    ("na_split_av", (_z(1, 4, 9, 4, 9), _z(1, 9, 9, 2, 32), [3, 3], [2, 1], [1, 1], [0, 0]), "attn is"),
+    ("na_split_av", (_z(1, 9, 9, 4, 8), _z(1, 9, 9, 2, 32), [3, 3], [1, 1], [1, 1], [0, 0]), "attn is"),
+    ("na_split_av", (_z(2, 9, 9, 4, 9), _z(1, 9, 9, 2, 32), [3, 3], [1, 1], [1, 1], [0, 0]), "attn is"),
+    ("na_split_av", (_z(1, 9, 9, 3, 9), _z(1, 9, 9, 2, 32), [3, 3], [1, 1], [1, 1], [0, 0]), "attn is"),
+    ("na_split_av", (_z(1, 9, 4, 9), _z(1, 9, 9, 2, 32), [3, 3], [1, 1], [1, 1], [0, 0]), "attn is"),
+    ("na_rpb_qk", (_z(1, 9, 8, 2, 32), _z(1, 9, 8, 2, 32), _z(2, 5, 5), [3, 3], [1, 1], 1.0, True, False), _HIP),
+    ("na_rpb_qk", (_z(1, 9, 8, 2, 32), _z(1, 9, 8, 2, 32), _z(2, 5, 3), [3, 3], [1, 1], 1.0, True, False), "rpb must"),
+    ("na_rpb_qk", (_z(1, 9, 8, 2, 32), _z(1, 9, 8, 2, 32), _z(2, 5, 5), [3, 3], [1, 1], 1.0, True, True), "rpb must"),
+    ("na_rpb_qk", (_z(1, 9, 8, 2, 32), _z(1, 8, 8, 2, 32), None, [3, 3], [1, 1], 1.0, True, False), "identical"),
+    ("na_rpb_qk", (_z(1, 9, 2, 32), _z(1, 9, 2, 32), None, [3, 3], [1, 1], 1.0, True, False), "rank-1 or rank-2"),
+    ("na_rpb_av", (_z(1, 9, 8, 2, 9), _z(1, 9, 8, 2, 32), [3, 3], [1, 1], False, True), _HIP),
+    ("na_rpb_av", (_z(1, 9, 8, 2, 8), _z(1, 9, 8, 2, 32), [3, 3], [1, 1], False, True), "attn must"),
+    ("na_rpb_av", (_z(1, 8, 9, 2, 9), _z(1, 9, 8, 2, 32), [3, 3], [1, 1], False, True), "attn must"),
+    ("na_rpb_av", (_z(1, 9, 8, 2, 9), _z(1, 9, 8, 2, 32), [3, -3], [1, 1], False, True), "positive"),
+    ("na_fused_qkv", (_z(1, 9, 3, 2, 32), [3], [1], [1], [0], 1.0, 0), _HIP),
+    ("na_fused_qkv", (_z(1, 9, 2, 2, 32), [3], [1], [1], [0], 1.0, 0), "qkv is"),
+    ("na_fused_qkv", (_z(1, 9, 3, 2, 32), [3, 3], [1], [1], [0], 1.0, 0), "per spatial axis"),
+    ("na_fused_qkv", (_z(1, 9, 3, 2, 32), [3], [0], [1], [0], 1.0, 0), "positive"),
+    ("na_linear", (_z(5, 32), _z(16, 32), _z(16)), _HIP),
+    ("na_linear", (_z(5, 32), _z(16, 24), None), "na_linear: x"),
+    ("na_linear", (_z(5, 32), _z(16, 32), _z(1)), "na_linear: x"),
+]
+
+
+@pytest.mark.parametrize("name,args,message", DIRECT, ids=[f"{i}-{c[0]}" for i, c in enumerate(DIRECT)])
+def test_direct_calls_check_shapes(name, args, message):
+    """A kernel indexes by the sizes of one tensor of a call: a mismatched call
+    raises before any launch."""
+    with pytest.raises(RuntimeError, match=message):
+        getattr(_ops(), name)(*args, 0)
+
+
 @pytest.mark.gpu
 def test_nodes_refuse_what_the_functions_refuse():
     from natten_amd import functional as F
