@@ -193,6 +193,7 @@ BwdPlan bwd_plan(const na_params *p, const na::Prob &P) {
     b.path = kBwdMfma;
     b.need_delta = extra || na::mfma_bwd_reads_delta(P);
   } else {
+    // one size for the whole family, of which only the vector-ALU kernels read it
     b.path = kBwdGeneric;
     b.need_delta = true;
   }

@@ -299,7 +299,7 @@ def test_split_against_oracle(case):
 
 @pytest.mark.gpu
 def test_split_non_finite_values_stay_in_their_windows():
-    """As above for AV and the inverse pass, whose products run over a box."""
+    """As above for the AV forward, whose product runs over a box."""
     from natten_amd import functional as F
 
     q, v, k = (randn((1, 21, 19, 2, 32), F32, i).to(DEV) for i in range(3))
@@ -317,6 +317,80 @@ def test_split_non_finite_values_stay_in_their_windows():
     want[0, :, :, 1, 3] = holds.to(DEV)
     assert torch.equal(bad, want)
     assert torch.allclose(out[~bad], clean[0][~bad], atol=1e-6)
+
+
+def _slots(sp, ks, dil, caus):
+    """Per query and slot (row-major): the key's token, and whether it counts."""
+    tok = torch.zeros((1, 1), dtype=torch.int64)
+    good = torch.ones((1, 1), dtype=torch.bool)
+    for n, K, d, c in zip(sp, ks, dil, caus):
+        idx, ok = (torch.as_tensor(x) for x in W.axis_indices(range(n), n, K, d, c))
+        tok = (tok[:, None, :, None] * n + idx[None, :, None, :]).reshape(tok.shape[0] * n, -1)
+        good = (good[:, None, :, None] & ok[None, :, None, :]).reshape(tok.shape)
+    return tok, good
+
+
+# (spatial, H, Hkv, D, kernel, dilation, causal, token that holds the bad value)
+NONFINITE = [
+    ((21, 19), 4, 2, 32, (7, 5), (1, 1), (False, False), 6 * 19 + 4),
+    ((17, 22), 2, 1, 64, (5, 3), (2, 3), (True, False), 9 * 22 + 1),
+    ((70,), 3, 3, 16, (13,), (3,), (True,), 40),
+    ((6, 7, 8), 2, 2, 32, (3, 3, 5), (1, 2, 1), (False, True, False), 150),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")], ids=str)
+@pytest.mark.parametrize("where", ["q", "k", "v", "attn", "grad"])
+@pytest.mark.parametrize("case", NONFINITE, ids=[f"{'x'.join(map(str, c[0]))}" for c in NONFINITE])
+def test_split_gradients_keep_non_finite_values_in_their_windows(case, where, bad):
+    """Both passes of both backward calls (and so the blocks that compute a
+    wave's rows again one by one): non-finite exactly where the window of the bad
+    row's query, or the windows that hold the bad row's key, put it."""
+    from natten_amd._core import hip
+
+    sp, H, Hkv, D, ks, dil, caus, t = case
+    print(f"[case] non-finite split gradients {case} {where} {bad}", flush=True)
+    tok, good = _slots(sp, ks, dil, caus)
+    n, kk, rep, one = tok.shape[0], tok.shape[1], H // Hkv, (1,) * len(sp)
+    h, e, slot = 1, 3, int(good[t].nonzero()[-1])
+    q, g = (randn((1, *sp, H, D), F32, i).to(DEV) for i in (0, 1))
+    k, v = (randn((1, *sp, Hkv, D), F32, i).to(DEV) for i in (2, 3))
+    a, dl = (randn((1, *sp, H, kk), F32, i).to(DEV) for i in (4, 5))
+
+    def run():
+        return (*hip.qk_backward(q, k, dl, ks, one, dil, caus, 0.3),
+                *hip.av_backward(a, v, g, ks, one, dil, caus))
+
+    clean = run()
+    hk = h // rep if where not in ("k", "v") else h % Hkv
+    x, head, last = {"q": (q, h, e), "k": (k, hk, e), "v": (v, hk, e), "grad": (g, h, e),
+                     "attn": (a, h, slot)}[where]
+    x.reshape(n, x.shape[-2], -1)[t, head, last] = bad
+    if where == "attn":  # the same slot of the logits' gradient
+        dl.reshape(n, H, kk)[t, h, slot] = bad
+    want = [torch.zeros((n, *y.shape[-2:]), dtype=torch.bool) for y in clean]
+    dq, dk, da, dv = want
+    if where == "q":
+        dk[tok[t, good[t]], hk, e] = True
+    if where == "grad":
+        dv[tok[t, good[t]], hk, e] = True
+        da[t, h, good[t]] = True
+    if where == "attn":
+        dq[t, h, :] = True
+        dk[tok[t, slot], hk, :] = True
+        dv[tok[t, slot], hk, :] = True
+    if where in ("k", "v"):
+        holds = (tok == t) & good
+        for r in range(hk * rep, (hk + 1) * rep):
+            if where == "k":
+                dq[holds.any(1), r, e] = True
+            else:
+                da[:, r] |= holds
+    for y, c, w, name in zip(run(), clean, want, ("dq", "dk", "dattn", "dv")):
+        y, c = (z.reshape(n, *z.shape[-2:]).cpu() for z in (y, c))
+        assert torch.equal(~torch.isfinite(y), w), name
+        assert_close(y[~w], c[~w].double(), F32, name, scale_tol=4.0)
 
 
 # (B, spatial, H, D, K, dilation) of the bias partials the dq pass writes;
