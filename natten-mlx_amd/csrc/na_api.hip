@@ -138,6 +138,12 @@ bool use_lsplit(const na_params *p, const na::Prob &P) {
          na::lsplit_eligible(P, p->dtype);
 }
 
+// The logits and the AV backward (dattn is the same product) of problems whose
+// other passes take the lean split kernels.
+bool use_lsplit_qk(const na_params *p, const na::Prob &P) {
+  return use_lsplit(p, P) && (na::lsplit_qk_gains(P) || !na::msplit_eligible(P, p->dtype));
+}
+
 bool use_msplit(const na_params *p, const na::Prob &P) {
   return (p->flags & NA_FLAG_GENERIC) == 0 && na::msplit_eligible(P, p->dtype);
 }
@@ -384,10 +390,11 @@ int na_mfma_selftest(int32_t dtype, float *out, void *stream) {
 
 int na_kernel_path(const na_params *p, int32_t backward) {
   na::Prob P;
-  const int rc = make_prob(p, &P, backward != 2);
+  const bool split = backward == 2 || backward == 3;
+  const int rc = make_prob(p, &P, !split);
   if (rc != NA_OK) return -rc;
-  if (backward == 2) {
-    if (use_lsplit(p, P)) return NA_PATH_LEAN;
+  if (split) {
+    if (backward == 2 ? use_lsplit(p, P) : use_lsplit_qk(p, P)) return NA_PATH_LEAN;
     if (use_msplit(p, P)) return NA_PATH_MFMA;
     return NA_PATH_GENERIC;
   }
@@ -586,7 +593,7 @@ int na_qk_fwd(const na_params *p, const void *q, const void *k, void *logits,
   if (use_lsplit(p, P) && na::vsplit_on() &&
       na::vsplit_qk(P, p->dtype, q, k, logits, P.scale, as_stream(stream)))
     ;
-  else if (use_lsplit(p, P))
+  else if (use_lsplit_qk(p, P))
     na::lsplit_qk(P, p->dtype, q, k, logits, P.scale, -INFINITY,
                   as_stream(stream));
   else if (use_msplit(p, P))
@@ -652,7 +659,7 @@ int na_av_bwd(const na_params *p, const void *attn, const void *v,
   if (attn == nullptr || v == nullptr || dout == nullptr || dattn == nullptr ||
       dv == nullptr)
     return fail(NA_ERR_INVALID, "attn/v/dout/dattn/dv must be non-NULL");
-  if (use_lsplit(p, P)) {
+  if (use_lsplit_qk(p, P)) {
     na::lsplit_av_bwd(P, p->dtype, attn, v, dout, dattn, dv, as_stream(stream));
   } else if (use_msplit(p, P)) {
     na::msplit_qk(P, p->dtype, dout, v, dattn, 1.f, 0.f, as_stream(stream));

@@ -868,6 +868,13 @@ bool lsplit_eligible(const Prob &P, int dtype) {
   return lean_choice(P, kLQK).ok && lean_choice(P, kLInv).ok;
 }
 
+// Logits of large rank-2 samples, lean against the 32-query kernels that ran them:
+// head_dim 128 from 25 slots on 1.02 to 1.17 times (0.92 once), with dv in the AV
+// backward 0.90 to 1.13; fewer slots 0.75 to 0.95, head_dim 32 / 64 0.53 to 1.06.
+bool lsplit_qk_gains(const Prob &P) {
+  return !(P.rank == 2 && P.D == 128 && P.kprod >= 25 && lean_large(P));
+}
+
 #define LS_D(D_, BODY) \
   do {                 \
     if ((D_) == 32) {  \

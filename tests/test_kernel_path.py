@@ -95,6 +95,17 @@ def _plan(shape_q, hkv, ks, dil, caus, dtype=torch.bfloat16, backward=False, **k
     return hip.kernel_plan(q, k, ks, (1,) * len(ks), dil, caus, backward=backward, **kw)
 
 
+def test_split_logits_of_large_samples():
+    """Large samples run the split ops lean, but the logits (and the AV backward,
+    whose dattn is the same product) of wide heads and many slots."""
+    no = (False, False)
+    for shape, ks, want in (((1, 301, 315, 4, 128), 5, "mfma"), ((1, 348, 363, 4, 128), 7, "mfma"),
+                            ((1, 275, 295, 4, 128), 3, "lean"), ((1, 282, 369, 4, 64), 7, "lean"),
+                            ((2, 120, 130, 4, 128), 5, "lean")):  # below 2^24 elements
+        got = [_path(shape, shape[-2], (ks, ks), (1, 1), no, split=s) for s in (True, "qk")]
+        assert got == ["lean", want], (shape, ks, got)
+
+
 def test_plans_of_the_benchmarked_configs():
     """The launch shapes the benchmark lines time: config 3 stages its key
     box in several depth slabs both ways; config 4 at its full size groups
