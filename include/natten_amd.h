@@ -387,6 +387,13 @@ int na_merge_bwd(const na_merge_params *p, const void *const *outs,
 
 /* ---- layer projections ---------------------------------------------------- */
 /*
+ * A packed projection's rows [tokens, 3, row_bytes] to three tensors
+ * [3, tokens, row_bytes] (split != 0), or back; row_bytes a multiple of 16,
+ * fewer than 2^31 16-byte units (nn/na2d.py:80-100).
+ */
+int na_pack3(int32_t split, int64_t tokens, int64_t row_bytes, const void *src,
+             void *dst, void *stream);
+/*
  * Weight and bias gradient of y = x W^T + b over `rows` rows, for the
  * attention layer's projections (nn/na2d.py:41-78): dw [n, k] = g^T x and,
  * where db is non-NULL, db [n] = column sums of g; g [rows, n], x [rows, k],
@@ -394,11 +401,6 @@ int na_merge_bwd(const na_merge_params *p, const void *const *outs,
  * are multiples of 8, at most 16384.  The workspace size is 0 for what is not
  * supported.
  */
-/* A packed projection's rows [tokens, 3, row_bytes] to three tensors
- * [3, tokens, row_bytes] (split != 0), or back; row_bytes a multiple of 16,
- * fewer than 2^31 16-byte units (nn/na2d.py:80-100). */
-int na_pack3(int32_t split, int64_t tokens, int64_t row_bytes, const void *src,
-             void *dst, void *stream);
 size_t na_linear_wgrad_workspace_bytes(int32_t dtype, int64_t rows, int64_t n,
                                        int64_t k);
 int na_linear_wgrad(int32_t dtype, int64_t rows, int64_t n, int64_t k,

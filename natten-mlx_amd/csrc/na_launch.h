@@ -205,13 +205,13 @@ int32_t wsplit_rpb_bias_tiles(const RpbProb &A);
 void wsplit_rpb_av_bwd(const RpbProb &A, const float *attn, const float *v,
                        const float *dout, float *dattn, float *dv, hipStream_t st);
 
-// Weight and bias gradient of a bf16 / fp16 linear map over M rows
-// (na_linear.hip): dw [N, K] = g^T x, db [N] = column sums of g (nullable).
 // Packed rows [tokens, 3, row_bytes] to three tensors one after the other
 // (split) or back; rows of whole 16-byte units.
 bool pack3_ok(int64_t tokens, int64_t row_bytes);
 void pack3(bool split, int64_t tokens, int64_t row_bytes, const void *src, void *dst,
            hipStream_t st);
+// Weight and bias gradient of a bf16 / fp16 linear map over M rows
+// (na_linear.hip): dw [N, K] = g^T x, db [N] = column sums of g (nullable).
 bool linear_wgrad_ok(int dtype, int64_t M, int64_t N, int64_t K);
 size_t linear_wgrad_workspace(int64_t M, int64_t N, int64_t K);
 void linear_wgrad(int dtype, int64_t M, int64_t N, int64_t K, const void *g, const void *x,

@@ -140,7 +140,12 @@ __device__ __forceinline__ void fwd_group(const typename L16<T>::e *ks,
 // -> 299 us, backward 1365 -> 1076; [1, 256, 256, 16, 128] K = 7 456 -> 284 and
 // 1258 -> 910; [2, 96, 96, 8, 64] K = 9 backward 250 -> 100).  Loading a slab after
 // the one before it is done instead: 318 and 1152 us for the first of these
-// (292 and 1102 with the loads ahead, then, without EX).
+// (292 and 1102 with the loads ahead, then, without EX).  By counters the first
+// forward reads its inputs from memory once (454 MB; rows that boxes share come
+// from the caches) and writes 189 MB (151 of output; a workgroup's LSE is one head's
+// 4 bytes in 32, so those 4.7 MB cost eight times that), 2.3 TB/s; its waves, nine to a
+// CU, spend 41% of their time waiting for loads, LDS and barriers and 26% for an issue
+// slot, matrix cores 12% busy: latency and issue bound it, not the traffic.
 // EX (fwd_group): row slabs, and problems of rank 1 and 2 whose sample holds
 // 2^24 elements or more.  Their other kernel (k_mfwd) sums float32 probabilities
 // against a maximum over more keys: fp16 [1, 384, 384, 8, 64] K = 13, LSE (rms
